@@ -545,14 +545,24 @@ static int launch_dtl(const GemmArgs& a, int c_dtype, bool kedge, dim3 grid, hip
   return check_launch("pd_gemm bf16 (buffer-fed)");
 }
 
-// Any operand layout through the buffer-fed kernel (a_kmaj / b_kmaj: K-contiguous).
-template <class CFG, int MODE>
-static int launch_dtl_any(const GemmArgs& a, bool a_kmaj, bool b_kmaj, int c_dtype, bool kedge, dim3 grid,
-                          hipStream_t s) {
-  if (a_kmaj && b_kmaj) return launch_dtl<CFG, MODE, false, false>(a, c_dtype, kedge, grid, s);
-  if (a_kmaj) return launch_dtl<CFG, MODE, false, true>(a, c_dtype, kedge, grid, s);
-  if (b_kmaj) return launch_dtl<CFG, MODE, true, false>(a, c_dtype, kedge, grid, s);
-  return launch_dtl<CFG, MODE, true, true>(a, c_dtype, kedge, grid, s);
+// Any operand layout through the buffer-fed kernel (a_kmaj / b_kmaj: K-contiguous), in 256x256
+// or 128x128 tiles.
+template <int MODE, bool BIG_OK>
+static int launch_dtl_any(const GemmArgs& a, bool a_kmaj, bool b_kmaj, int c_dtype, bool kedge, bool big,
+                          unsigned batch, hipStream_t s) {
+  const int64_t t = BIG_OK && big ? 256 : 128;
+  const dim3 grid((unsigned)cdiv(a.N, t), (unsigned)cdiv(a.M, t), batch);
+#define PD_L(AMN, BMN)                                                                              \
+  {                                                                                                 \
+    if constexpr (BIG_OK)                                                                           \
+      if (big) return launch_dtl<CfgDtlBig, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);            \
+    return launch_dtl<CfgDtlSmall<AMN, BMN>, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);           \
+  }
+  if (a_kmaj && b_kmaj) PD_L(false, false)
+  if (a_kmaj) PD_L(false, true)
+  if (b_kmaj) PD_L(true, false)
+  PD_L(true, true)
+#undef PD_L
 }
 
 // Every operand of the buffer-fed kernel within its 31-bit addressing range.
@@ -584,18 +594,8 @@ int pd_gemm(int dtype, int64_t M, int64_t N, int64_t K, const void* A, int64_t l
   if (!bf16_operand_ok(A, lda, a_kmaj ? K : M) || !bf16_operand_ok(B, ldb, b_kmaj ? K : N))
     return fail(PD_EUNSUPPORTED, "pd_gemm: bf16 operands need 16B alignment and contiguous dims / ld % 8 == 0");
   GemmArgs a{M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, C, ldc, alpha, beta, nullptr, 0, 0, 0};
-  if (dtl_fits_any(M, N, K, lda, a_kmaj, ldb, b_kmaj)) {
-    // 256x256 tiles once they fill every CU at least once: they read each operand panel
-    // half as often. Measured in the LM step (21.8 -> 21.1 ms) and the dense step (0.83 ->
-    // 0.81 ms); only whole rounds of big tiles (no 1.5-round shapes) was 21.5 ms.
-    if (cdiv(M, CfgDtlBig::BM) * cdiv(N, CfgDtlBig::BN) >= 256)
-      return launch_dtl_any<CfgDtlBig, MODE_DENSE>(
-          a, a_kmaj, b_kmaj, c_dtype, K % CfgDtlBig::BK != 0,
-          dim3((unsigned)cdiv(N, CfgDtlBig::BN), (unsigned)cdiv(M, CfgDtlBig::BM)), s);
-    return launch_dtl_any<CfgDtlRA, MODE_DENSE>(a, a_kmaj, b_kmaj, c_dtype, K % CfgDtlRA::BK != 0,
-                                                dim3((unsigned)cdiv(N, CfgDtlRA::BN), (unsigned)cdiv(M, CfgDtlRA::BM)),
-                                                s);
-  }
+  if (dtl_fits_any(M, N, K, lda, a_kmaj, ldb, b_kmaj))
+    return launch_dtl_any<MODE_DENSE, true>(a, a_kmaj, b_kmaj, c_dtype, K % 64 != 0, big_tiles(M, N), 1, s);
   if (use_big_tile(M, N))
     return launch_bf16<CfgBig, MODE_DENSE>(a, a_kmaj, b_kmaj, c_dtype,
                                            dim3((unsigned)cdiv(N, 256), (unsigned)cdiv(M, 256)), s);
@@ -628,9 +628,7 @@ int pd_gemm_strided_batched(int dtype, int64_t batch, int64_t M, int64_t N, int6
   GemmArgs a{M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, C, ldc, alpha, beta, nullptr, 0, stride_b,
              stride_c, stride_a};
   if (dtl_fits_any(M, N, K, lda, a_kmaj, ldb, b_kmaj))
-    return launch_dtl_any<CfgDtlRA, MODE_BATCHED>(
-        a, a_kmaj, b_kmaj, c_dtype, K % CfgDtlRA::BK != 0,
-        dim3((unsigned)cdiv(N, CfgDtlRA::BN), (unsigned)cdiv(M, CfgDtlRA::BM), (unsigned)batch), s);
+    return launch_dtl_any<MODE_BATCHED, false>(a, a_kmaj, b_kmaj, c_dtype, K % 64 != 0, false, (unsigned)batch, s);
   return launch_bf16<CfgSmall, MODE_BATCHED>(
       a, a_kmaj, b_kmaj, c_dtype, dim3((unsigned)cdiv(N, 128), (unsigned)cdiv(M, 128), (unsigned)batch), s);
 }
@@ -659,15 +657,19 @@ int grouped_gemm(const void* lhs, const void* rhs, const int32_t* offsets, int64
                        out_dtype == PD_DTYPE_F32 ? 4 : 2, out);
   GemmArgs a{J, N, K, (const bf16_t*)lhs, K, (const bf16_t*)rhs, b_kmaj ? K : N, out, N, 1.f, 0.f, offsets, E,
              K * N, 0};
-  static_assert(CfgDtl::BM == CfgSmall::BM && CfgDtl::BN == CfgSmall::BN, "one grid shape for both kernels");
   int64_t max_tiles = cdiv(J, CfgSmall::BM) + E;
   if (max_tiles > 65535) return fail(PD_EUNSUPPORTED, "pd_grouped_gemm: too many rows");
   dim3 grid((unsigned)cdiv(N, CfgSmall::BN), (unsigned)max_tiles);
   static_assert(CfgDtlRA::BM == CfgSmall::BM && CfgDtlRA::BN == CfgSmall::BN, "one grid shape for both kernels");
-  if (b_kmaj && dtl_fits(J, K, N, K))
-    return launch_dtl<CfgDtlRA, MODE_GROUPED>(a, out_dtype, K % CfgDtlRA::BK != 0, grid, s);
+  const bool kedge = K % 64 != 0;
+  if (b_kmaj && dtl_fits(J, K, N, K)) {
+    if (big_tiles_grouped(J, E, N))
+      return launch_dtl<CfgDtlBig, MODE_GROUPED>(a, out_dtype, kedge,
+                                                 dim3((unsigned)cdiv(N, 256), (unsigned)(cdiv(J, 256) + E)), s);
+    return launch_dtl<CfgDtlRA, MODE_GROUPED>(a, out_dtype, kedge, grid, s);
+  }
   if (!b_kmaj && dtl_fits(J, K, 0, 0) && dtl_fits_mn(K, N))  // each expert's rhs stored [K][N]
-    return launch_dtl<CfgDtlRA, MODE_GROUPED, false, true>(a, out_dtype, K % CfgDtlRA::BK != 0, grid, s);
+    return launch_dtl<CfgDtl, MODE_GROUPED, false, true>(a, out_dtype, kedge, grid, s);
   return launch_bf16<CfgSmall, MODE_GROUPED>(a, true, b_kmaj, out_dtype, grid, s);
 }
 
@@ -723,8 +725,7 @@ int gemm_splitk(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int
   if (!ws || ws_bytes < (size_t)splits * M * N * sizeof(float)) return fail(PD_EWORKSPACE, "gemm_splitk: scratch");
   hipStream_t s = (hipStream_t)stream;
   GemmArgs a{M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, ws, N, 1.f, 0.f, nullptr, 0, 0, M * N, kc};
-  const dim3 grid((unsigned)cdiv(N, CfgDtlRA::BN), (unsigned)cdiv(M, CfgDtlRA::BM), (unsigned)splits);
-  int rc = launch_dtl_any<CfgDtlRA, MODE_SPLITK>(a, a_kmaj, b_kmaj, PD_DTYPE_F32, K % CfgDtlRA::BK != 0, grid, s);
+  int rc = launch_dtl_any<MODE_SPLITK, false>(a, a_kmaj, b_kmaj, PD_DTYPE_F32, K % 64 != 0, false, (unsigned)splits, s);
   if (rc) return rc;
   const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdiv(M * N / 4, 256), 8192));
   if (c_dtype == PD_DTYPE_F32)
@@ -753,7 +754,7 @@ int grouped_gemm_pair(const void* lhs1, const void* rhsT1, void* out1, const voi
              (const bf16_t*)lhs2, (const bf16_t*)rhsT2, out2};
   if (cdiv(J, CfgDtlRA::BM) + E > 65535) return fail(PD_EUNSUPPORTED, "grouped_gemm_pair: too many rows");
   if (!dtl_fits(J, K, N, K)) return fail(PD_EUNSUPPORTED, "grouped_gemm_pair: operands of 2 GiB or more");
-  if (N >= 512)  // 256x256 tiles: measured faster for the paired N=512 products
+  if (big_tiles_grouped(J, E, N, 2))
     return launch_dtl<CfgDtlBig, MODE_GROUPED>(
         a, out_dtype, K % CfgDtlBig::BK != 0,
         dim3((unsigned)cdiv(N, CfgDtlBig::BN), (unsigned)(cdiv(J, CfgDtlBig::BM) + E), 2), (hipStream_t)stream);
@@ -791,15 +792,19 @@ int grouped_gemm_kcat(const void* lhs1, const void* rhs1, int64_t K1, const void
   q.rs_tok2 = rs2 ? rs2 : rs;
   q.sort_idx = sort_idx;
   q.k = k;
-  if (N >= 512) {  // 256x256 tiles, as for the paired N=512 products
-    const dim3 grid((unsigned)cdiv(N, CfgDtlBig::BN), (unsigned)(cdiv(J, CfgDtlBig::BM) + E), pair ? 2u : 1u);
-    hipLaunchKernelGGL((k_gemm_dtl_kcat<CfgDtlBig, bf16_t, false, false, EpiStore, MODE_GROUPED>), grid,
-                       dim3(CfgDtlBig::NT), 0, (hipStream_t)stream, a, q, EpiStore::Args{});
+#define PD_L(CFG, KE)                                                                                            \
+  hipLaunchKernelGGL((k_gemm_dtl_kcat<CFG, bf16_t, false, false, KE, EpiStore, MODE_GROUPED>),                    \
+                     dim3((unsigned)cdiv(N, CFG::BN), (unsigned)(cdiv(J, CFG::BM) + E), pair ? 2u : 1u),          \
+                     dim3(CFG::NT), 0, (hipStream_t)stream, a, q, EpiStore::Args{})
+  const bool ke = K1 % 64 || K2 % 64;
+  if (big_tiles_grouped(J, E, N, pair ? 2 : 1)) {
+    if (ke) PD_L(CfgDtlBig, true);
+    else PD_L(CfgDtlBig, false);
   } else {
-    const dim3 grid((unsigned)cdiv(N, CfgDtlRA::BN), (unsigned)(cdiv(J, CfgDtlRA::BM) + E), pair ? 2u : 1u);
-    hipLaunchKernelGGL((k_gemm_dtl_kcat<CfgDtlRA, bf16_t, false, false, EpiStore, MODE_GROUPED>), grid,
-                       dim3(CfgDtlRA::NT), 0, (hipStream_t)stream, a, q, EpiStore::Args{});
+    if (ke) PD_L(CfgDtl, true);
+    else PD_L(CfgDtl, false);
   }
+#undef PD_L
   return check_launch("grouped_gemm_kcat");
 }
 
@@ -818,7 +823,7 @@ int grouped_gemm_dw_pair(const void* lhs1, const void* dout1, void* out1, const 
   GemmArgs a{K, N, J, (const bf16_t*)lhs1, K, (const bf16_t*)dout1, N, out1, N, 1.f, 0.f, offsets, E, 0, K * N, 0,
              (const bf16_t*)lhs2, (const bf16_t*)dout2, out2};
   dim3 grid((unsigned)cdiv(N, CfgDtlRA::BN), (unsigned)cdiv(K, CfgDtlRA::BM), (unsigned)(2 * E));
-  return launch_dtl<CfgDtlRA, MODE_GROUPED_K, true, true>(a, out_dtype, true, grid, (hipStream_t)stream);
+  return launch_dtl<CfgDtl, MODE_GROUPED_K, true, true>(a, out_dtype, true, grid, (hipStream_t)stream);
 }
 
 }  // namespace pd
@@ -837,7 +842,7 @@ int pd_grouped_gemm_dw(const void* lhs, const void* dout, const int32_t* offsets
   dim3 grid((unsigned)cdiv(N, CfgSmall::BN), (unsigned)cdiv(K, CfgSmall::BM), (unsigned)E);
   static_assert(CfgDtlRA::BM == CfgSmall::BM && CfgDtlRA::BN == CfgSmall::BN, "one grid shape for both kernels");
   if (dtl_fits_mn(J, K) && dtl_fits_mn(J, N))  // both operands MN-major: rows of lhs / dout are k
-    return launch_dtl<CfgDtlRA, MODE_GROUPED_K, true, true>(a, out_dtype, true, grid, (hipStream_t)stream);
+    return launch_dtl<CfgDtl, MODE_GROUPED_K, true, true>(a, out_dtype, true, grid, (hipStream_t)stream);
   return launch_bf16<CfgSmall, MODE_GROUPED_K>(a, false, false, out_dtype, grid, (hipStream_t)stream);
 }
 

@@ -13,11 +13,22 @@
 // record count ends at the operand's last row, so rows past the operand extent, and
 // chunks past the end of its last row, load as zeros; their outputs are never stored.
 //
-// NS LDS stages form a ring with NS-1 k-tiles in flight: iteration kt waits (vmcnt) until
-// its own tile has landed, one s_barrier makes it visible and frees the stage of tile
-// kt-1, the loads of tile kt+NS-1 go out, then tile kt is consumed. The barrier is a bare
-// s_barrier with compiler-only memory clobbers: a fenced __syncthreads would wait for
-// every load in flight.
+// Two LDS stages, software-pipelined inside a wave (pipe_stage). A stage is four k16 steps;
+// the fragments of step n+1 are read from LDS between the MFMAs of step n (two register
+// sets), and the last step of a stage reads the first fragments of the next one, after the
+// one barrier of the stage: this wave's loads of the next stage have landed (vmcnt) and
+// its reads of this stage are done (lgkmcnt), so behind the barrier the next stage is
+// visible and this one's space is free. The loads of stage kt+2 go out in two halves,
+// between the MFMAs of stage kt's last step and of stage kt+1's first step. The order is
+// pinned by scheduling barriers: left to itself the compiler reads a step's fragments into
+// the registers of the step before, after its MFMAs, so a wave alternates between waiting
+// for LDS and computing. Same products, same k order, so the same bits as the unpipelined
+// loop; 256x256 tiles 4096x3072x4096 with B MN-major 131 -> 104 us (785 -> 994 TFLOP/s),
+// both MN-major 137 -> 104 us, K-major 8192x4096x3072 210 -> 169 us. What bounds the loop
+// now is the LDS port: at 64x128 per wave a k16 step is 48 KB of fragment reads and 16 KB of
+// load writes per CU, 512 clocks at 128 B, as many as its MFMAs take.
+// The barrier is a bare s_barrier with compiler-only memory clobbers: a fenced
+// __syncthreads would wait for every load in flight.
 //
 // The MFMA runs with the operands swapped (B rows as the 32-row "A" input), so each lane
 // ends with 4 consecutive output columns of one row per 4 accumulators; the epilogue
@@ -249,12 +260,10 @@ __device__ inline bool map_tile(const GemmArgs& p, int lane, TileJob& t) {
   return t.m0 < t.M && t.n0 < p.N;
 }
 
-// RA_: read every fragment of a stage from LDS before its first MFMA (false: one k16
-// step ahead of the MFMAs).
-template <int BM_, int BN_, int WM_, int WN_, int NS_, bool RA_ = false>
+// SPLIT: the loads of a stage go out in two halves (see the top of this file).
+template <int BM_, int BN_, int WM_, int WN_, bool SPLIT_>
 struct DtlCfg {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, BK = 64;
-  static constexpr bool READ_ALL = RA_;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = 2, BK = 64;
   static constexpr int NW = WM_ * WN_, NT = NW * 64;
   static constexpr int WTM = BM_ / WM_, WTN = BN_ / WN_;  // wave tile
   static constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -263,11 +272,11 @@ struct DtlCfg {
   static constexpr int STAGE_BYTES = (BM_ + BN_) * ROWB;
   static constexpr int A_INSTS = BM_ / (RPI * NW), B_INSTS = BN_ / (RPI * NW);  // 1 KB loads per wave per stage
   static constexpr int INSTS = A_INSTS + B_INSTS;
+  static constexpr int HALF = SPLIT_ ? INSTS / 2 : INSTS;  // loads in the first half
   static_assert(NW % 2 == 0, "the swizzle parity of a wave's rows must not depend on the load index");
   static_assert(BM_ % (RPI * NW) == 0 && BN_ % (RPI * NW) == 0, "every wave moves whole 1 KB row blocks");
   static_assert(TM >= 1 && TN >= 1 && WTM % 32 == 0 && WTN % 32 == 0, "wave tile is a multiple of 32x32");
-  static_assert(NS_ >= 2 && INSTS * (NS_ - 2) < 64, "vmcnt range");
-  static_assert(NS_ * STAGE_BYTES <= 160 * 1024, "LDS");
+  static_assert(NS * STAGE_BYTES <= 160 * 1024, "LDS");
 };
 
 // s_waitcnt on the vector-memory counter only (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] |
@@ -278,19 +287,8 @@ __device__ inline void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-// Waits until at most `ahead` (<= A) stages of this wave's loads are still in flight.
-template <int INSTS, int A>
-__device__ inline void wait_stages(int ahead) {
-  if constexpr (A > 0) {
-    if (ahead >= A) {
-      wait_vmcnt<A * INSTS>();
-      return;
-    }
-    wait_stages<INSTS, A - 1>(ahead);
-  } else {
-    wait_vmcnt<0>();
-  }
-}
+// Waits for this wave's buffer loads (vmcnt = 0) and its LDS operations (lgkmcnt = 0).
+__device__ inline void wait_loads_and_lds() { __builtin_amdgcn_s_waitcnt(7 << 4); }
 
 // A bare s_barrier: it orders the waves but waits for none of this wave's memory
 // operations (gfx950 inserts no wait before s_barrier). It suffices where the LDS data
@@ -323,14 +321,35 @@ __device__ inline int64_t uni64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// 128x128x64 tiles, 8 waves (4x2, 32x64 per wave), 2 LDS stages (64 KB, two blocks per CU).
-typedef DtlCfg<128, 128, 4, 2, 2> CfgDtl;
-// The same tile reading a whole stage's fragments before its MFMAs: never slower, and
-// 10-19% faster on the K=512 MoE shapes (measured per shape).
-typedef DtlCfg<128, 128, 4, 2, 2, true> CfgDtlRA;
-// 256x256x64 tiles, 8 waves of 64x128 (128 KB of LDS, one block per CU): fewer LDS
-// bytes per MFMA; faster for the paired N=512 products and the paired weight gradients.
-typedef DtlCfg<256, 256, 4, 2, 2> CfgDtlBig;
+// 128x128x64 tiles (64 KB of LDS, two blocks per CU): 8 waves of 32x64, or 4 waves of 64x64,
+// which read 4 fragments for 4 MFMAs instead of 3 for 2 but leave fewer waves to cover a
+// transposing read's or an epilogue's latency. K-major 8192x1024x768 17.6 (4 waves) against
+// 18.6 us, both MN-major 768x4096x4096 51 (8 waves) against 55; loads in two halves: 60.
+typedef DtlCfg<128, 128, 4, 2, false> CfgDtl;
+typedef DtlCfg<128, 128, 2, 2, false> CfgDtlRA;
+// 256x256x64 tiles, 8 waves (128 KB of LDS, one block per CU): fewer LDS bytes per MFMA.
+typedef DtlCfg<256, 256, 2, 4, true> CfgDtlBig;
+template <bool AMN, bool BMN>
+using CfgDtlSmall = std::conditional_t<AMN || BMN, CfgDtl, CfgDtlRA>;
+
+// Whether `rows` x N outputs take 256x256 tiles (one block per CU) rather than 128x128 (two
+// per CU): by the rounds of 256 big or 512 small tiles, a partial round costing 0.8 + 0.2 of
+// its fill and a round of small tiles 0.64 of a round of big ones (half the products at 0.8
+// of the rate). Big against small, us: 192 big tiles (4096x3072x4096) 101 / 117, 384
+// (8192x3072x4864) 238 / 248, 512 (65536x512x512) 46 / 60, 256 (65536x256x512) 28 / 31; 128
+// (8192x1024x768) 21.7 / 17.6, 48 (768x4096x4096) 91 / 51. Grouped rows: J plus half a tile
+// per group for the groups' ragged ends.
+inline bool big_tiles(int64_t rows, int64_t N, int64_t problems = 1) {
+  auto rounds = [](int64_t tiles, int64_t cap) {  // in fifths
+    const int64_t full = tiles / cap, rem = tiles % cap;
+    return 5.0 * full + (rem ? 4.0 + (double)rem / cap : 0.0);
+  };
+  auto up = [](int64_t x, int64_t n) { return (x + n - 1) / n; };
+  return rounds(problems * up(rows, 256) * up(N, 256), 256) <= 0.64 * rounds(problems * up(rows, 128) * up(N, 128), 512);
+}
+inline bool big_tiles_grouped(int64_t J, int E, int64_t N, int64_t problems = 1) {
+  return big_tiles(J + (int64_t)E * 128, N, problems);
+}
 
 // The kernel addresses each operand through a 31-bit buffer record count (rows = M or N
 // for a K-major operand; for an MN-major one, K plus the 128 k-rows a last stage may
@@ -346,34 +365,27 @@ __device__ inline int32_t buf_bytes(int64_t bytes) {
   return bytes > 0x7FFFFFFF ? 0x7FFFFFFF : (bytes < 0 ? 0 : (int32_t)bytes);
 }
 
-// Per-lane byte offsets of a wave's 1 KB row-block loads of one operand tile (relative
-// to the tile's first row, k = 0): lane l fills physical chunk l % 8 of row l / 8 of the
-// block, i.e. logical chunk (l % 8) ^ swz(row); the block of load q starts at row
-// (q * NW + wave) * 8, so swz's parity bit is wave & 1 for every q.
-template <int ROWS, int NW>
-__device__ inline void dtl_offsets(uint32_t (&off)[ROWS / (8 * NW)], int64_t ld, int wave, int lane) {
-  const int rsub = lane >> 3;
-  const int c = (lane & 7) ^ rsub ^ (wave & 1);
-#pragma unroll
-  for (int q = 0; q < ROWS / (8 * NW); ++q) {
-    const int64_t row = (int64_t)(q * NW + wave) * 8 + rsub;
-    off[q] = (uint32_t)((row * ld + c * 8) * 2);
-  }
-}
-
-// Per-lane byte offsets of a wave's 1 KB loads of an MN-major operand tile (R elements
-// per k-row, relative to the tile's first column, k = 0): load q covers k-rows
+// A wave's 1 KB loads of one operand tile: the lane's byte offset of load 0 relative to the
+// tile's first row (K-major) or column (MN-major) at k = 0, and the step from load to load
+// (one scalar: NW row blocks further, so the swizzle of the lane's chunk is the same).
+// K-major: lane l fills physical chunk l % 8 of row l / 8 of the block, i.e. logical chunk
+// (l % 8) ^ swz(row); the block of load q starts at row (q * NW + wave) * 8, so swz's
+// parity bit is wave & 1 for every q. MN-major (R elements per k-row): load q covers k-rows
 // (q * NW + wave) * RPL .. + RPL - 1; lane l fills physical chunk l % CPR of k-row l / CPR.
-template <int R, int NW>
-__device__ inline void dtl_offsets_mn(uint32_t (&off)[R / (8 * NW)], int64_t ld, int wave, int lane) {
-  static_assert(R >= 128 && R <= 512, "an MN-major tile row is 256..1024 bytes");
-  constexpr int CPR = R / 8, RPL = 1024 / (2 * R);
-  const int rsub = lane / CPR, pc = lane % CPR;
-#pragma unroll
-  for (int q = 0; q < R / (8 * NW); ++q) {
-    const int64_t row = (int64_t)(q * NW + wave) * RPL + rsub;
-    const int c = pc ^ (4 * (int)(row & 3));
-    off[q] = (uint32_t)((row * ld + c * 8) * 2);
+struct LaneOff {
+  uint32_t off, step;
+};
+template <bool MN, int R, int NW>
+__device__ inline LaneOff dtl_offsets(int64_t ld, int wave, int lane) {
+  if constexpr (MN) {
+    static_assert(R >= 128 && R <= 512, "an MN-major tile row is 256..1024 bytes");
+    constexpr int CPR = R / 8, RPL = 1024 / (2 * R);
+    static_assert(NW * RPL % 4 == 0, "the swizzle (k-row & 3) must not depend on the load index");
+    const int row = wave * RPL + lane / CPR, c = (lane % CPR) ^ (4 * (row & 3));
+    return {(uint32_t)((row * ld + c * 8) * 2), (uint32_t)uni((int)(NW * RPL * ld * 2))};
+  } else {
+    const int rsub = lane >> 3, c = (lane & 7) ^ rsub ^ (wave & 1);
+    return {(uint32_t)(((wave * 8 + rsub) * ld + c * 8) * 2), (uint32_t)uni((int)(NW * 8 * ld * 2))};
   }
 }
 
@@ -423,17 +435,27 @@ struct FragOffs {
   }
 };
 
-// One stage of one operand at byte offset koff (the stage's k position) within each
-// row. The descriptor spans [base, base + bytes) (stride 0); the whole offset goes in the
-// per-lane register so the record-count check covers it.
-template <int ROWS, int NW>
-__device__ inline void dtl_issue(char* dst, const bf16_t* base, int32_t bytes, const uint32_t* off, uint32_t koff,
-                                 int wave) {
-  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), (short)0, bytes, 0x00020000);
+// Loads LO .. HI-1 of a stage of one operand at byte offset koff (the stage's k position)
+// within each row. The descriptor spans [base, base + bytes) (stride 0); the whole offset
+// goes in the per-lane register so the record-count check covers it (bytes = 0: zeros).
+template <int NW, int LO, int HI>
+__device__ inline void dtl_issue(char* dst, const bf16_t* base, int32_t bytes, LaneOff lo, uint32_t koff, int wave) {
+  if constexpr (LO < HI) {
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), (short)0, bytes, 0x00020000);
 #pragma unroll
-  for (int q = 0; q < ROWS / (8 * NW); ++q)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(dst + (q * NW + wave) * 8 * 128), 16, off[q] + koff,
-                                             0, 0, 0);
+    for (int q = LO; q < HI; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(dst + (q * NW + wave) * 8 * 128), 16,
+                                               lo.off + (koff + q * lo.step), 0, 0, 0);
+  }
+}
+
+// Loads LO .. HI-1 of a stage, counted over A's and then B's, into stage space st.
+template <class CFG, int LO, int HI>
+__device__ inline void dtl_issue_ab(char* st, const bf16_t* a, int32_t abytes, LaneOff offa, uint32_t ka,
+                                    const bf16_t* b, int32_t bbytes, LaneOff offb, uint32_t kb, int wave) {
+  constexpr int NA = CFG::A_INSTS;
+  dtl_issue<CFG::NW, (LO < NA ? LO : NA), (HI < NA ? HI : NA)>(st, a, abytes, offa, ka, wave);
+  dtl_issue<CFG::NW, (LO > NA ? LO - NA : 0), (HI > NA ? HI - NA : 0)>(st + CFG::BM * CFG::ROWB, b, bbytes, offb, kb, wave);
 }
 
 __device__ inline void mask_frag(bf16x8& v, int64_t k, int64_t kmin, int64_t kend) {
@@ -483,22 +505,30 @@ __device__ inline void store1<bf16_t>(bf16_t* C, int64_t idx, float v, float bet
   C[idx] = f32_to_bf16(beta != 0.f ? v + beta * bf16_to_f32(C[idx]) : v);
 }
 
-// Fragment reads of k16 step kk of a stage; EDGE zeroes k outside [kmin, kend).
-template <class CFG, bool EDGE, bool AMN, bool BMN>
-__device__ inline void dtl_read(const char* st, const FragOffs<CFG, AMN, BMN>& fo, int lane, int kk, int64_t k0,
-                                int64_t kmin, int64_t kend, bf16x8 (&af)[CFG::TM], bf16x8 (&bfr)[CFG::TN]) {
+// The fragments of one k16 step.
+template <class CFG>
+struct Frags {
+  bf16x8 a[CFG::TM], b[CFG::TN];
+};
+
+template <class CFG, bool AMN, bool BMN>
+__device__ inline void read_frags(const char* st, const FragOffs<CFG, AMN, BMN>& fo, int lane, int kk,
+                                  Frags<CFG>& f) {
   const int coff = ((2 * kk + (lane >> 5)) ^ fo.sw) << 4;
 #pragma unroll
-  for (int i = 0; i < CFG::TM; ++i) af[i] = frag_load<AMN, CFG::BM>(st, fo.a[i], kk, coff);
+  for (int j = 0; j < CFG::TN; ++j) f.b[j] = frag_load<BMN, CFG::BN>(st, fo.b[j], kk, coff);
 #pragma unroll
-  for (int j = 0; j < CFG::TN; ++j) bfr[j] = frag_load<BMN, CFG::BN>(st, fo.b[j], kk, coff);
-  if (EDGE) {
-    const int64_t kf = k0 + kk * 16 + (lane >> 5) * 8;
+  for (int i = 0; i < CFG::TM; ++i) f.a[i] = frag_load<AMN, CFG::BM>(st, fo.a[i], kk, coff);
+}
+
+// Zeroes the fragments' k outside [kmin, kend); k = the step's first.
+template <class CFG>
+__device__ inline void mask_frags(Frags<CFG>& f, int lane, int64_t k, int64_t kmin, int64_t kend) {
+  const int64_t kf = k + (lane >> 5) * 8;
 #pragma unroll
-    for (int i = 0; i < CFG::TM; ++i) mask_frag(af[i], kf, kmin, kend);
+  for (int i = 0; i < CFG::TM; ++i) mask_frag(f.a[i], kf, kmin, kend);
 #pragma unroll
-    for (int j = 0; j < CFG::TN; ++j) mask_frag(bfr[j], kf, kmin, kend);
-  }
+  for (int j = 0; j < CFG::TN; ++j) mask_frag(f.b[j], kf, kmin, kend);
 }
 
 template <class CFG>
@@ -511,30 +541,43 @@ __device__ inline void dtl_mfma(const bf16x8 (&af)[CFG::TM], const bf16x8 (&bfr)
       acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[j], af[i], acc[i][j], 0, 0, 0);
 }
 
-// Consumes one 64-k stage (4 k16 steps), reading step kk+1's fragments ahead of step
-// kk's MFMAs.
-template <class CFG, bool EDGE, bool AMN, bool BMN>
-__device__ inline void dtl_stage(const char* st, const FragOffs<CFG, AMN, BMN>& fo, int lane, int64_t k0,
-                                 int64_t kmin, int64_t kend, f32x16 (&acc)[CFG::TM][CFG::TN]) {
-  constexpr int TM = CFG::TM, TN = CFG::TN, KK = CFG::KK;
-  if constexpr (CFG::READ_ALL) {
-    // every fragment of the stage in flight at once; each MFMA then waits only for its
-    // own reads, so the LDS latency of later steps hides behind earlier MFMAs
-    bf16x8 af[KK][TM], bfr[KK][TN];
+// Scheduling order of a step: after each of its MFMAS MFMAs, an equal share of its READS LDS
+// reads (sched_group_barrier mask 0x100) and LOADS buffer loads (0x020).
+template <int MFMAS, int READS, int LOADS>
+__device__ inline void spread_step() {
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) dtl_read<CFG, EDGE>(st, fo, lane, kk, k0, kmin, kend, af[kk], bfr[kk]);
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) dtl_mfma<CFG>(af[kk], bfr[kk], acc);
-    return;
+  for (int m = 0; m < MFMAS; ++m) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if ((m + 1) * READS / MFMAS > m * READS / MFMAS)
+      __builtin_amdgcn_sched_group_barrier(0x100, (READS + MFMAS - 1) / MFMAS, 0);
+    if (LOADS > 0 && (m + 1) * LOADS / MFMAS > m * LOADS / MFMAS)
+      __builtin_amdgcn_sched_group_barrier(0x020, (LOADS + MFMAS - 1) / MFMAS, 0);
   }
-  bf16x8 af[2][TM], bfr[2][TN];
-  dtl_read<CFG, EDGE>(st, fo, lane, 0, k0, kmin, kend, af[0], bfr[0]);
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) {
-    if (kk + 1 < KK)
-      dtl_read<CFG, EDGE>(st, fo, lane, kk + 1, k0, kmin, kend, af[(kk + 1) & 1], bfr[(kk + 1) & 1]);
-    dtl_mfma<CFG>(af[kk & 1], bfr[kk & 1], acc);
-  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The stage's four k16 steps (see the top of this file). Before: f[0] holds the stage's
+// step 0. read(kk, f): the stage's step kk; read_next(f): the next stage's step 0;
+// issue(ahead, half): that half of the loads of the stage `ahead` stages on; mfma(kk, f):
+// step kk's products. MFMAS, READS: a step's MFMAs and LDS reads; LOADS0, LOADS3: the loads issued in steps 0 and 3.
+template <int MFMAS, int READS, int LOADS0, int LOADS3, class F, class Read, class ReadNext, class Issue, class Mfma>
+__device__ inline void pipe_stage(F (&f)[2], Read&& read, ReadNext&& read_next, Issue&& issue, Mfma&& mfma) {
+  read(1, f[1]);
+  issue(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+  mfma(0, f[0]);
+  spread_step<MFMAS, READS, LOADS0>();
+  read(2, f[0]);
+  mfma(1, f[1]);
+  spread_step<MFMAS, READS, 0>();
+  read(3, f[1]);
+  mfma(2, f[0]);
+  spread_step<MFMAS, READS, 0>();
+  wait_loads_and_lds();
+  lds_barrier();
+  read_next(f[0]);
+  issue(std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
+  mfma(3, f[1]);
+  spread_step<MFMAS, READS, LOADS3>();
 }
 
 template <class CFG, typename TC>
@@ -687,9 +730,9 @@ struct EpiStore {
 // (ldb) between k-rows.
 template <class CFG, typename TC, int MODE, bool KEDGE, class EPI = EpiStore, bool AMN = false, bool BMN = false>
 __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::Args ea) {
-  constexpr int BM = CFG::BM, BN = CFG::BN, TM = CFG::TM, TN = CFG::TN, NS = CFG::NS, NW = CFG::NW;
-  constexpr int BK = CFG::BK, ROWB = CFG::ROWB;
-  constexpr int LDS = NS * CFG::STAGE_BYTES > EPI::LDS_BYTES ? NS * CFG::STAGE_BYTES : EPI::LDS_BYTES;
+  constexpr int BM = CFG::BM, BN = CFG::BN, TM = CFG::TM, TN = CFG::TN, NW = CFG::NW;
+  constexpr int BK = CFG::BK;
+  constexpr int LDS = CFG::NS * CFG::STAGE_BYTES > EPI::LDS_BYTES ? CFG::NS * CFG::STAGE_BYTES : EPI::LDS_BYTES;
   __shared__ __attribute__((aligned(1024))) char smem[LDS];
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
   const int wm = wave / CFG::WN, wn = wave % CFG::WN;
@@ -708,11 +751,7 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
   const bf16_t* bbase = (const bf16_t*)uni64((int64_t)(BMN ? t.B + n0 : t.B + n0 * p.ldb));
   const int32_t abytes = buf_bytes(AMN ? (p.K * p.lda - m0) * 2 : (p.M - m0) * p.lda * 2);
   const int32_t bbytes = buf_bytes(BMN ? (p.K * p.ldb - n0) * 2 : (p.N - n0) * p.ldb * 2);
-  uint32_t offa[CFG::A_INSTS], offb[CFG::B_INSTS];
-  if constexpr (AMN) dtl_offsets_mn<BM, NW>(offa, p.lda, wave, lane);
-  else dtl_offsets<BM, NW>(offa, p.lda, wave, lane);
-  if constexpr (BMN) dtl_offsets_mn<BN, NW>(offb, p.ldb, wave, lane);
-  else dtl_offsets<BN, NW>(offb, p.ldb, wave, lane);
+  const LaneOff offa = dtl_offsets<AMN, BM, NW>(p.lda, wave, lane), offb = dtl_offsets<BMN, BN, NW>(p.ldb, wave, lane);
   // a stage's k position as a byte offset: along the row (K-major) or down k-rows (MN)
   const uint32_t kstep_a = AMN ? (uint32_t)(p.lda * 2) : 2u, kstep_b = BMN ? (uint32_t)(p.ldb * 2) : 2u;
 
@@ -724,55 +763,53 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  auto issue = [&](int64_t kt) {
-    char* st = smem + (int)(kt % NS) * CFG::STAGE_BYTES;
+  // half h of the loads of stage kt (none past the last stage: its descriptors are empty)
+  auto issue = [&](int64_t kt, auto h) {
+    constexpr int LO = decltype(h)::value ? CFG::HALF : 0, HI = decltype(h)::value ? CFG::INSTS : CFG::HALF;
     const uint32_t kpos = (uint32_t)(kbeg + kt * BK);
-    dtl_issue<BM, NW>(st, abase, abytes, offa, kpos * kstep_a, wave);
-    dtl_issue<BN, NW>(st + BM * ROWB, bbase, bbytes, offb, kpos * kstep_b, wave);
+    const bool in = kt < nk;
+    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & 1) * CFG::STAGE_BYTES, abase, uni(in ? abytes : 0), offa,
+                              kpos * kstep_a, bbase, uni(in ? bbytes : 0), offb, kpos * kstep_b, wave);
   };
-
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < nk) issue(s);
+  issue(0, std::integral_constant<int, 0>{});
+  issue(0, std::integral_constant<int, 1>{});
+  issue(1, std::integral_constant<int, 0>{});
 
   const FragOffs<CFG, AMN, BMN> fo(wm, wn, lane);
-  auto sync = [&](int64_t kt) {  // stage kt has landed and is visible; stage kt+NS-1 goes out
-    const int64_t left = nk - 1 - kt;
-    wait_stages<CFG::INSTS, NS - 2>((int)(left < NS - 2 ? left : NS - 2));
-    lds_barrier();
-    if (kt + NS - 1 < nk) issue(kt + NS - 1);
+  Frags<CFG> f[2];
+  wait_vmcnt<CFG::HALF>();
+  lds_barrier();
+  read_frags<CFG>(smem, fo, lane, 0, f[0]);
+  constexpr int READS = TM * (AMN ? 2 : 1) + TN * (BMN ? 2 : 1);
+  auto stage = [&](int64_t kt, auto edge) {
+    const char* st = smem + (int)(kt & 1) * CFG::STAGE_BYTES;
+    const char* nx = smem + (int)(~kt & 1) * CFG::STAGE_BYTES;
+    pipe_stage<TM * TN, READS, CFG::INSTS - CFG::HALF, CFG::HALF>(
+        f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
+        [&](Frags<CFG>& g) { read_frags<CFG>(nx, fo, lane, 0, g); },
+        [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
+        [&](int kk, Frags<CFG>& g) {
+          if (decltype(edge)::value) mask_frags<CFG>(g, lane, kbeg + kt * BK + kk * 16, kmin, kend);
+          dtl_mfma<CFG>(g.a, g.b, acc);
+        });
   };
-  auto st_of = [&](int64_t kt) { return smem + (int)(kt % NS) * CFG::STAGE_BYTES; };
   if constexpr (KEDGE) {
-    if (nk > 0) {
-      sync(0);
-      dtl_stage<CFG, true>(st_of(0), fo, lane, kbeg, kmin, kend, acc);
-    }
-    for (int64_t kt = 1; kt < nk - 1; ++kt) {
-      sync(kt);
-      dtl_stage<CFG, false>(st_of(kt), fo, lane, kbeg + kt * BK, kmin, kend, acc);
-    }
-    if (nk > 1) {
-      sync(nk - 1);
-      dtl_stage<CFG, true>(st_of(nk - 1), fo, lane, kbeg + (nk - 1) * BK, kmin, kend, acc);
-    }
+    if (nk > 0) stage(0, std::true_type{});
+    for (int64_t kt = 1; kt < nk - 1; ++kt) stage(kt, std::false_type{});
+    if (nk > 1) stage(nk - 1, std::true_type{});
   } else {
-    for (int64_t kt = 0; kt < nk; ++kt) {
-      sync(kt);
-      dtl_stage<CFG, false>(st_of(kt), fo, lane, kbeg + kt * BK, kmin, kend, acc);
-    }
+    for (int64_t kt = 0; kt < nk; ++kt) stage(kt, std::false_type{});
   }
+  wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG, TC>(p, ea, t, wm, wn, tid, acc, smem);
 }
 
 // Two products of one shape in one block, P1 = A @ B^T and P2 = A2 @ B2^T (dense, every
 // operand K-contiguous with the same lda / ldb), for epilogues that need both tiles of the
-// same (row, column) block at once. A stage holds A | B | A2 | B2 (B2 == B shares B's
-// rows and skips their loads; with SHARED_B the caller guarantees B2 == B and a stage
-// has no B2 region). EPI::run(p, ea, tile, wm, wn, tid, acc1, acc2, smem).
+// same (row, column) block at once. A stage holds A | B | A2 | B2 (SHARED_B: the caller
+// guarantees B2 == B, and a stage has no B2 region). EPI::run(p, ea, tile, wm, wn, tid, acc1, acc2, smem).
 template <class CFG, bool KEDGE, class EPI, bool SHARED_B = false>
 __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename EPI::Args ea) {
-  static_assert(CFG::NS == 2, "two LDS stages");
   constexpr int BM = CFG::BM, BN = CFG::BN, TM = CFG::TM, TN = CFG::TN, NW = CFG::NW;
   constexpr int BK = CFG::BK, ROWB = CFG::ROWB;
   constexpr int SB = (SHARED_B ? 2 * BM + BN : 2 * (BM + BN)) * ROWB;
@@ -788,15 +825,13 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
   const int64_t kmin = uni64(t.kbeg), kend = uni64(t.kend);
   const int64_t kbeg = kmin & ~(int64_t)63;
   const int64_t nk = kend > kmin ? (kend - kbeg + BK - 1) / BK : 0;
-  const bool share_b = SHARED_B || p.B2 == p.B;
   const bf16_t* abase = (const bf16_t*)uni64((int64_t)(p.A + m0 * p.lda));
   const bf16_t* a2base = (const bf16_t*)uni64((int64_t)(p.A2 + m0 * p.lda));
   const bf16_t* bbase = (const bf16_t*)uni64((int64_t)(p.B + n0 * p.ldb));
   const bf16_t* b2base = (const bf16_t*)uni64((int64_t)(p.B2 + n0 * p.ldb));
   const int32_t abytes = buf_bytes((p.M - m0) * p.lda * 2), bbytes = buf_bytes((p.N - n0) * p.ldb * 2);
-  uint32_t offa[CFG::A_INSTS], offb[CFG::B_INSTS];
-  dtl_offsets<BM, NW>(offa, p.lda, wave, lane);
-  dtl_offsets<BN, NW>(offb, p.ldb, wave, lane);
+  const LaneOff offa = dtl_offsets<false, BM, NW>(p.lda, wave, lane);
+  const LaneOff offb = dtl_offsets<false, BN, NW>(p.ldb, wave, lane);
 
   f32x16 acc[TM][TN], acc2[TM][TN];
 #pragma unroll
@@ -806,52 +841,76 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = acc2[i][j][v] = 0.f;
 
-  auto issue = [&](int64_t kt) {
+  // half 0: A and B (without SPLIT every load), half 1: A2 (and B2), of stage kt (none past
+  // the last stage)
+  constexpr bool SPLIT = CFG::HALF < CFG::INSTS;
+  constexpr int LOADS1 = SHARED_B ? CFG::A_INSTS : CFG::INSTS;
+  auto issue = [&](int64_t kt, auto h) {
     char* st = smem + (int)(kt & 1) * SB;
     const uint32_t koff = (uint32_t)((kbeg + kt * BK) * 2);
-    dtl_issue<BM, NW>(st, abase, abytes, offa, koff, wave);
-    dtl_issue<BN, NW>(st + BM * ROWB, bbase, bbytes, offb, koff, wave);
-    dtl_issue<BM, NW>(st + (BM + BN) * ROWB, a2base, abytes, offa, koff, wave);
-    if (!share_b) dtl_issue<BN, NW>(st + (2 * BM + BN) * ROWB, b2base, bbytes, offb, koff, wave);
+    const int32_t ab = uni(kt < nk ? abytes : 0), bb = uni(kt < nk ? bbytes : 0);
+    if (decltype(h)::value == 0) {
+      dtl_issue<NW, 0, CFG::A_INSTS>(st, abase, ab, offa, koff, wave);
+      dtl_issue<NW, 0, CFG::B_INSTS>(st + BM * ROWB, bbase, bb, offb, koff, wave);
+    }
+    if (decltype(h)::value == SPLIT) {
+      dtl_issue<NW, 0, CFG::A_INSTS>(st + (BM + BN) * ROWB, a2base, ab, offa, koff, wave);
+      if (!SHARED_B) dtl_issue<NW, 0, CFG::B_INSTS>(st + (2 * BM + BN) * ROWB, b2base, bb, offb, koff, wave);
+    }
   };
-  if (nk > 0) issue(0);
+  issue(0, std::integral_constant<int, 0>{});
+  issue(0, std::integral_constant<int, 1>{});
+  issue(1, std::integral_constant<int, 0>{});
 
   const FragOffs<CFG, false, false> fo(wm, wn, lane);
-  FragOffs<CFG, false, false> fo2 = fo;  // the second problem's A (and B) sit after the first's
+  struct F2 {
+    Frags<CFG> x;
+    bf16x8 a2[TM], b2[SHARED_B ? 1 : TN];
+  } f[2];
+  // the second problem's A (and B) sit after the first's
+  auto read = [&](const char* st, int kk, F2& g) {
+    read_frags<CFG>(st, fo, lane, kk, g.x);
+    const int coff = ((2 * kk + (lane >> 5)) ^ fo.sw) << 4;
 #pragma unroll
-  for (int i = 0; i < TM; ++i) fo2.a[i] += (BM + BN) * ROWB;
+    for (int i = 0; i < TM; ++i) g.a2[i] = frag_load<false, BM>(st, fo.a[i] + (BM + BN) * ROWB, kk, coff);
+    if constexpr (!SHARED_B) {
 #pragma unroll
-  for (int j = 0; j < TN; ++j) fo2.b[j] += share_b ? 0 : (BM + BN) * ROWB;
-  auto sync = [&](int64_t kt) {
-    wait_vmcnt<0>();
-    lds_barrier();
-    if (kt + 1 < nk) issue(kt + 1);
+      for (int j = 0; j < TN; ++j) g.b2[j] = frag_load<false, BN>(st, fo.b[j] + (BM + BN) * ROWB, kk, coff);
+    }
   };
+  wait_vmcnt<CFG::INSTS + (SPLIT ? 0 : LOADS1)>();
+  lds_barrier();
+  read(smem, 0, f[0]);
   auto stage = [&](int64_t kt, auto edge) {
-    constexpr bool E = decltype(edge)::value;
     const char* st = smem + (int)(kt & 1) * SB;
-    dtl_stage<CFG, E>(st, fo, lane, kbeg + kt * BK, kmin, kend, acc);
-    dtl_stage<CFG, E>(st, fo2, lane, kbeg + kt * BK, kmin, kend, acc2);
+    const char* nx = smem + (int)(~kt & 1) * SB;
+    pipe_stage<2 * TM * TN, 2 * TM + (SHARED_B ? 1 : 2) * TN, (SPLIT ? LOADS1 : 0), CFG::INSTS + (SPLIT ? 0 : LOADS1)>(
+        f, [&](int kk, F2& g) { read(st, kk, g); }, [&](F2& g) { read(nx, 0, g); },
+        [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
+        [&](int kk, F2& g) {
+          if (decltype(edge)::value) {
+            const int64_t kf = kbeg + kt * BK + kk * 16;
+            mask_frags<CFG>(g.x, lane, kf, kmin, kend);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) mask_frag(g.a2[i], kf + (lane >> 5) * 8, kmin, kend);
+            if constexpr (!SHARED_B) {
+#pragma unroll
+              for (int j = 0; j < TN; ++j) mask_frag(g.b2[j], kf + (lane >> 5) * 8, kmin, kend);
+            }
+          }
+          dtl_mfma<CFG>(g.x.a, g.x.b, acc);
+          if constexpr (SHARED_B) dtl_mfma<CFG>(g.a2, g.x.b, acc2);
+          else dtl_mfma<CFG>(g.a2, g.b2, acc2);
+        });
   };
   if constexpr (KEDGE) {
-    if (nk > 0) {
-      sync(0);
-      stage(0, std::true_type{});
-    }
-    for (int64_t kt = 1; kt < nk - 1; ++kt) {
-      sync(kt);
-      stage(kt, std::false_type{});
-    }
-    if (nk > 1) {
-      sync(nk - 1);
-      stage(nk - 1, std::true_type{});
-    }
+    if (nk > 0) stage(0, std::true_type{});
+    for (int64_t kt = 1; kt < nk - 1; ++kt) stage(kt, std::false_type{});
+    if (nk > 1) stage(nk - 1, std::true_type{});
   } else {
-    for (int64_t kt = 0; kt < nk; ++kt) {
-      sync(kt);
-      stage(kt, std::false_type{});
-    }
+    for (int64_t kt = 0; kt < nk; ++kt) stage(kt, std::false_type{});
   }
+  wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG>(p, ea, t, wm, wn, tid, acc, acc2, smem);
 }
 
@@ -862,7 +921,8 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
 // rs(t) = routed(t) ? (delta ? delta[t] : 0) : 1, routed(t) = !route || route[t] (delta
 // bf16, or fp32 through delta_f): the
 // blend weight of the target output x @ W^T in the masked linear (and of its cotangent).
-// A1 and A2 are K-contiguous; B1MN / B2MN: the B operand is MN-major. The LDS stage ring
+// A1 and A2 are K-contiguous, K1 and K2 at least 1 (KEDGE: not both multiples of 64);
+// B1MN / B2MN: the B operand is MN-major. The LDS stage ring
 // runs straight through the segment boundary, so the second product's first stages
 // load while the first product's last stage is consumed.
 // MODE_GROUPED (job space of routed experts): rows are jobs sorted by expert, each B is an
@@ -888,11 +948,11 @@ struct KcatArgs {
   const float* delta_f = nullptr;  // fp32 per-row delta (dense mode; preferred over `delta`)
 };
 
-template <class CFG, typename TC, bool B1MN, bool B2MN, class EPI = EpiStore, int MODE = MODE_DENSE>
+template <class CFG, typename TC, bool B1MN, bool B2MN, bool KEDGE, class EPI = EpiStore, int MODE = MODE_DENSE>
 __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs q, typename EPI::Args ea) {
-  constexpr int BM = CFG::BM, BN = CFG::BN, TM = CFG::TM, TN = CFG::TN, NS = CFG::NS, NW = CFG::NW;
-  constexpr int BK = CFG::BK, ROWB = CFG::ROWB;
-  constexpr int LDS = NS * CFG::STAGE_BYTES > EPI::LDS_BYTES ? NS * CFG::STAGE_BYTES : EPI::LDS_BYTES;
+  constexpr int BM = CFG::BM, BN = CFG::BN, TM = CFG::TM, TN = CFG::TN, NW = CFG::NW;
+  constexpr int BK = CFG::BK;
+  constexpr int LDS = CFG::NS * CFG::STAGE_BYTES > EPI::LDS_BYTES ? CFG::NS * CFG::STAGE_BYTES : EPI::LDS_BYTES;
   __shared__ __attribute__((aligned(1024))) char smem[LDS];
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
   const int wm = wave / CFG::WN, wn = wave % CFG::WN;
@@ -921,13 +981,8 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
   const int32_t a1bytes = buf_bytes((p.M - m0) * q.lda1 * 2), a2bytes = buf_bytes((p.M - m0) * p.lda * 2);
   const int32_t b1bytes = buf_bytes(B1MN ? (K1 * q.ldb1 - n0) * 2 : (p.N - n0) * q.ldb1 * 2);
   const int32_t b2bytes = buf_bytes(B2MN ? (K2 * p.ldb - n0) * 2 : (p.N - n0) * p.ldb * 2);
-  uint32_t oa1[CFG::A_INSTS], ob1[CFG::B_INSTS], oa2[CFG::A_INSTS], ob2[CFG::B_INSTS];
-  dtl_offsets<BM, NW>(oa1, q.lda1, wave, lane);
-  dtl_offsets<BM, NW>(oa2, p.lda, wave, lane);
-  if constexpr (B1MN) dtl_offsets_mn<BN, NW>(ob1, q.ldb1, wave, lane);
-  else dtl_offsets<BN, NW>(ob1, q.ldb1, wave, lane);
-  if constexpr (B2MN) dtl_offsets_mn<BN, NW>(ob2, p.ldb, wave, lane);
-  else dtl_offsets<BN, NW>(ob2, p.ldb, wave, lane);
+  const LaneOff oa1 = dtl_offsets<false, BM, NW>(q.lda1, wave, lane), ob1 = dtl_offsets<B1MN, BN, NW>(q.ldb1, wave, lane);
+  const LaneOff oa2 = dtl_offsets<false, BM, NW>(p.lda, wave, lane), ob2 = dtl_offsets<B2MN, BN, NW>(p.ldb, wave, lane);
   const uint32_t ks1 = B1MN ? (uint32_t)(q.ldb1 * 2) : 2u, ks2 = B2MN ? (uint32_t)(p.ldb * 2) : 2u;
 
   f32x16 acc[TM][TN];
@@ -938,44 +993,48 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  // One issue path whose operands are selected value by value: two calls under an
-  // if / else get merged into one call over selected array addresses, which moves the
-  // offset arrays to scratch and the descriptors into vector registers.
-  auto issue = [&](int64_t kt) {
-    char* st = smem + (int)(kt % NS) * CFG::STAGE_BYTES;
-    const bool s1 = kt < nk1;
+  // one issue path whose operands are selected value by value
+  auto issue = [&](int64_t kt, auto h) {
+    constexpr int LO = decltype(h)::value ? CFG::HALF : 0, HI = decltype(h)::value ? CFG::INSTS : CFG::HALF;
+    const bool s1 = kt < nk1, in = kt < nk;
     const uint32_t kpos = (uint32_t)((s1 ? kt : kt - nk1) * BK);
-    uint32_t oa[CFG::A_INSTS], ob[CFG::B_INSTS];
-#pragma unroll
-    for (int i = 0; i < CFG::A_INSTS; ++i) oa[i] = s1 ? oa1[i] : oa2[i];
-#pragma unroll
-    for (int i = 0; i < CFG::B_INSTS; ++i) ob[i] = s1 ? ob1[i] : ob2[i];
-    dtl_issue<BM, NW>(st, s1 ? a1 : a2, s1 ? a1bytes : a2bytes, oa, kpos * 2, wave);
-    dtl_issue<BN, NW>(st + BM * ROWB, s1 ? b1 : b2, s1 ? b1bytes : b2bytes, ob, kpos * (s1 ? ks1 : ks2), wave);
+    const LaneOff oa{s1 ? oa1.off : oa2.off, s1 ? oa1.step : oa2.step};
+    const LaneOff ob{s1 ? ob1.off : ob2.off, s1 ? ob1.step : ob2.step};
+    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & 1) * CFG::STAGE_BYTES, (const bf16_t*)uni64((int64_t)(s1 ? a1 : a2)),
+                              uni(in ? (s1 ? a1bytes : a2bytes) : 0), oa, kpos * 2,
+                              (const bf16_t*)uni64((int64_t)(s1 ? b1 : b2)),
+                              uni(in ? (s1 ? b1bytes : b2bytes) : 0), ob, kpos * (s1 ? ks1 : ks2), wave);
   };
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < nk) issue(s);
+  issue(0, std::integral_constant<int, 0>{});
+  issue(0, std::integral_constant<int, 1>{});
+  issue(1, std::integral_constant<int, 0>{});
 
   const FragOffs<CFG, false, B1MN> fo1(wm, wn, lane);
   const FragOffs<CFG, false, B2MN> fo2(wm, wn, lane);
-  auto sync = [&](int64_t kt) {
-    const int64_t left = nk - 1 - kt;
-    wait_stages<CFG::INSTS, NS - 2>((int)(left < NS - 2 ? left : NS - 2));
-    lds_barrier();
-    if (kt + NS - 1 < nk) issue(kt + NS - 1);
+  Frags<CFG> f[2];
+  wait_vmcnt<CFG::HALF>();
+  lds_barrier();
+  read_frags<CFG>(smem, fo1, lane, 0, f[0]);
+  // stage kt of a segment whose fragments sit at fo, the next stage's at fon; its k range
+  // starts at k0 and ends at kend
+  auto stage = [&](int64_t kt, const auto& fo, const auto& fon, int64_t k0, int64_t kend, auto edge, auto reads) {
+    const char* st = smem + (int)(kt & 1) * CFG::STAGE_BYTES;
+    const char* nx = smem + (int)(~kt & 1) * CFG::STAGE_BYTES;
+    pipe_stage<TM * TN, decltype(reads)::value, CFG::INSTS - CFG::HALF, CFG::HALF>(
+        f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
+        [&](Frags<CFG>& g) { read_frags<CFG>(nx, fon, lane, 0, g); },
+        [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
+        [&](int kk, Frags<CFG>& g) {
+          if (decltype(edge)::value) mask_frags<CFG>(g, lane, k0 + kk * 16, 0, kend);
+          dtl_mfma<CFG>(g.a, g.b, acc);
+        });
   };
-  auto st_of = [&](int64_t kt) { return smem + (int)(kt % NS) * CFG::STAGE_BYTES; };
-  // segment 1 (k tail masked in its last stage)
-  const bool tail1 = (K1 % BK) != 0;
-  for (int64_t kt = 0; kt < nk1 - (tail1 ? 1 : 0); ++kt) {
-    sync(kt);
-    dtl_stage<CFG, false>(st_of(kt), fo1, lane, kt * BK, 0, K1, acc);
-  }
-  if (tail1) {
-    sync(nk1 - 1);
-    dtl_stage<CFG, true>(st_of(nk1 - 1), fo1, lane, (nk1 - 1) * BK, 0, K1, acc);
-  }
+  constexpr std::integral_constant<int, TM + TN * (B1MN ? 2 : 1)> r1{};
+  constexpr std::integral_constant<int, TM + TN * (B2MN ? 2 : 1)> r2{};
+  // segment 1; its last stage reads segment 2's first fragments (KEDGE: and masks its k tail)
+  constexpr bool LAST1 = KEDGE || B1MN != B2MN;
+  for (int64_t kt = 0; kt < nk1 - LAST1; ++kt) stage(kt, fo1, fo1, kt * BK, K1, std::false_type{}, r1);
+  if constexpr (LAST1) stage(nk1 - 1, fo1, fo2, (nk1 - 1) * BK, K1, std::integral_constant<bool, KEDGE>{}, r1);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int64_t row = m0 + wm * CFG::WTM + i * 32 + (lane & 31);
@@ -989,15 +1048,9 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
       for (int v = 0; v < 16; ++v) acc[i][j][v] *= rs;
   }
   // segment 2
-  const bool tail2 = (K2 % BK) != 0;
-  for (int64_t kt = nk1; kt < nk - (tail2 ? 1 : 0); ++kt) {
-    sync(kt);
-    dtl_stage<CFG, false>(st_of(kt), fo2, lane, (kt - nk1) * BK, 0, K2, acc);
-  }
-  if (tail2) {
-    sync(nk - 1);
-    dtl_stage<CFG, true>(st_of(nk - 1), fo2, lane, (nk - 1 - nk1) * BK, 0, K2, acc);
-  }
+  for (int64_t kt = nk1; kt < nk - KEDGE; ++kt) stage(kt, fo2, fo2, (kt - nk1) * BK, K2, std::false_type{}, r2);
+  if constexpr (KEDGE) stage(nk - 1, fo2, fo2, (nk - 1 - nk1) * BK, K2, std::true_type{}, r2);
+  wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG, TC>(p, ea, t, wm, wn, tid, acc, smem);
 }
 
@@ -1007,16 +1060,25 @@ template <class EPI, typename TC, bool BMN = false>
 inline int launch_dense_epi(const GemmArgs& a, const typename EPI::Args& ea, hipStream_t s, const char* what) {
   if (a.M * a.lda * 2 > 0x7FFFFFFF || !(BMN ? dtl_fits_mn(a.K, a.ldb) : a.N * a.ldb * 2 <= 0x7FFFFFFF))
     return fail(PD_EUNSUPPORTED, std::string(what) + ": operands of 2 GiB or more");
-  if ((a.M + CfgDtlRA::BM - 1) / CfgDtlRA::BM > 65535 || (a.N + CfgDtlRA::BN - 1) / CfgDtlRA::BN > 65535)
+  if ((a.M + CfgDtl::BM - 1) / CfgDtl::BM > 65535 || (a.N + CfgDtl::BN - 1) / CfgDtl::BN > 65535)
     return fail(PD_EUNSUPPORTED, std::string(what) + ": too large");
-  const dim3 grid((unsigned)((a.N + CfgDtlRA::BN - 1) / CfgDtlRA::BN), (unsigned)((a.M + CfgDtlRA::BM - 1) / CfgDtlRA::BM));
-  if (a.K % CfgDtlRA::BK)
-    hipLaunchKernelGGL((k_gemm_dtl<CfgDtlRA, TC, MODE_DENSE, true, EPI, false, BMN>), grid, dim3(CfgDtlRA::NT), 0, s,
+  const dim3 grid((unsigned)((a.N + CfgDtl::BN - 1) / CfgDtl::BN), (unsigned)((a.M + CfgDtl::BM - 1) / CfgDtl::BM));
+  if (a.K % CfgDtl::BK)
+    hipLaunchKernelGGL((k_gemm_dtl<CfgDtl, TC, MODE_DENSE, true, EPI, false, BMN>), grid, dim3(CfgDtl::NT), 0, s,
                        a, ea);
   else
-    hipLaunchKernelGGL((k_gemm_dtl<CfgDtlRA, TC, MODE_DENSE, false, EPI, false, BMN>), grid, dim3(CfgDtlRA::NT), 0, s,
+    hipLaunchKernelGGL((k_gemm_dtl<CfgDtl, TC, MODE_DENSE, false, EPI, false, BMN>), grid, dim3(CfgDtl::NT), 0, s,
                        a, ea);
   return check_launch(what);
+}
+
+template <class CFG, class EPI, typename TC, bool B1MN, bool B2MN>
+inline void launch_kcat_cfg(const GemmArgs& a, const KcatArgs& q, const typename EPI::Args& ea, hipStream_t s) {
+  const dim3 grid((unsigned)((a.N + CFG::BN - 1) / CFG::BN), (unsigned)((a.M + CFG::BM - 1) / CFG::BM));
+  if (a.K % CFG::BK || q.K1 % CFG::BK)
+    hipLaunchKernelGGL((k_gemm_dtl_kcat<CFG, TC, B1MN, B2MN, true, EPI>), grid, dim3(CFG::NT), 0, s, a, q, ea);
+  else
+    hipLaunchKernelGGL((k_gemm_dtl_kcat<CFG, TC, B1MN, B2MN, false, EPI>), grid, dim3(CFG::NT), 0, s, a, q, ea);
 }
 
 // C = rs (.) (A1 @ op(B1)) + A2 @ op(B2) (k_gemm_dtl_kcat) with the epilogue policy EPI.
@@ -1029,16 +1091,10 @@ inline int launch_kcat_epi(const GemmArgs& a, const KcatArgs& q, const typename 
     return fail(PD_EUNSUPPORTED, std::string(what) + ": operands of 2 GiB or more");
   if ((a.M + CfgDtlRA::BM - 1) / CfgDtlRA::BM > 65535 || (a.N + CfgDtlRA::BN - 1) / CfgDtlRA::BN > 65535)
     return fail(PD_EUNSUPPORTED, std::string(what) + ": too large");
-  // 256x256 tiles once the grid has at least 256 of them (pd_gemm's rule)
-  const int64_t gbx = (a.N + CfgDtlBig::BN - 1) / CfgDtlBig::BN, gby = (a.M + CfgDtlBig::BM - 1) / CfgDtlBig::BM;
-  if (EPI::LDS_BYTES <= 2 * CfgDtlBig::STAGE_BYTES && gbx * gby >= 256)
-    hipLaunchKernelGGL((k_gemm_dtl_kcat<CfgDtlBig, TC, B1MN, B2MN, EPI>), dim3((unsigned)gbx, (unsigned)gby),
-                       dim3(CfgDtlBig::NT), 0, s, a, q, ea);
+  if (big_tiles(a.M, a.N) && EPI::LDS_BYTES <= 2 * CfgDtlBig::STAGE_BYTES)
+    launch_kcat_cfg<CfgDtlBig, EPI, TC, B1MN, B2MN>(a, q, ea, s);
   else
-    hipLaunchKernelGGL((k_gemm_dtl_kcat<CfgDtlRA, TC, B1MN, B2MN, EPI>),
-                       dim3((unsigned)((a.N + CfgDtlRA::BN - 1) / CfgDtlRA::BN),
-                            (unsigned)((a.M + CfgDtlRA::BM - 1) / CfgDtlRA::BM)),
-                       dim3(CfgDtlRA::NT), 0, s, a, q, ea);
+    launch_kcat_cfg<CfgDtl, EPI, TC, B1MN, B2MN>(a, q, ea, s);
   return check_launch(what);
 }
 

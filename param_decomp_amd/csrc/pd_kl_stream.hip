@@ -397,7 +397,7 @@ static KLFused kl_fused_plan(int64_t N, int64_t d, int64_t V, int n_chunks, char
 // Tiles of the fused passes: with one head for both sides (a tied head, as in the LM
 // step) 128 positions x 256 vocab columns, whose stage (A | B | A2, 64 KB) carries half
 // the operand bytes per MFMA of the 128 x 128 tile; with two heads 128 x 128.
-typedef DtlCfg<128, 256, 4, 2, 2> CfgKLWide;
+typedef DtlCfg<128, 256, 4, 2, false> CfgKLWide;
 static int64_t kl_tiles(const KLChunks& K, int64_t V, int bn) {
   int64_t n = 0;
   for (int64_t c = 0; c < K.nc; ++c) n += cdiv(K.width(c, V), bn);

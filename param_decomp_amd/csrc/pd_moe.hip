@@ -1229,18 +1229,18 @@ static int grouped_gemm_mask_bwd(const bf16_t* lhs, const bf16_t* rhs, bf16_t* o
                                  int64_t K, int64_t N, int pm, float imp_scale, hipStream_t s) {
   const bool pair = lhs2 != nullptr;
   if (J == 0) return PD_OK;
-  if (!dtl_fits(J, K, N, K) || cdiv(J, CfgDtlRA::BM) + E > 65535)
+  if (!dtl_fits(J, K, N, K) || cdiv(J, CfgDtl::BM) + E > 65535)
     return fail(PD_EUNSUPPORTED, "pd_moe_stack_step: d_acts product too large");
   GemmArgs a{J, N, K, lhs, K, rhs, K, out, N, 1.f, 0.f, offsets, E, K * N, 0, 0, lhs2, rhs2, out2};
   // 128x128 tiles for pairs too (unlike the plain paired N=512 products): two blocks per
   // CU keep twice the waves to cover the epilogue's gathered loads (measured faster)
-  const dim3 grid((unsigned)cdiv(N, CfgDtlRA::BN), (unsigned)(cdiv(J, CfgDtlRA::BM) + E), pair ? 2u : 1u);
+  const dim3 grid((unsigned)cdiv(N, CfgDtl::BN), (unsigned)(cdiv(J, CfgDtl::BM) + E), pair ? 2u : 1u);
 #define PD_FM(PMV)                                                                                                    \
   {                                                                                                                   \
     typename EpiMaskBwd<PMV>::Args ea{m0, pair ? *m1 : m0, h0, pair ? h1 : h0, ub0, pair ? ub1 : ub0, d_pre0,         \
                                       pair ? d_pre1 : d_pre0, imp_scale};                                             \
-    hipLaunchKernelGGL((k_gemm_dtl<CfgDtlRA, bf16_t, MODE_GROUPED, false, EpiMaskBwd<PMV>>), grid,                   \
-                       dim3(CfgDtlRA::NT), 0, s, a, ea);                                                              \
+    hipLaunchKernelGGL((k_gemm_dtl<CfgDtl, bf16_t, MODE_GROUPED, false, EpiMaskBwd<PMV>>), grid,                   \
+                       dim3(CfgDtl::NT), 0, s, a, ea);                                                              \
   }
   if (pm == PM_SL0) PD_FM(PM_SL0)
   else if (pm == 2) PD_FM(2)

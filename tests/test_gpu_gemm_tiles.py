@@ -1,0 +1,59 @@
+"""The bf16 products in 256x256 tiles (`big_tiles`): contractions of one partial stage up to
+a few, ragged outputs, ragged and empty groups, and the two-segment product with k tails.
+
+Against fp32 products of the same bf16 operands: an fp32 output's error is the order of an
+fp32 sum over K <= 1000 terms (below 1e-6 of the result's norm), a bf16 output adds one
+rounding (2^-9 of a value at most, 1.7e-3 of the norm for uniform mantissas)."""
+
+import pytest
+import torch
+
+from param_decomp_amd import ops
+from param_decomp_amd.decomposed_linear import SiteWeights, site_forward
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(got, want):
+    return float((got.float() - want).norm() / want.norm())
+
+
+def _rand(device, seed, *shape):
+    g = torch.Generator(device=device).manual_seed(seed)
+    return torch.randn(*shape, device=device, generator=g).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 136, 320])
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+def test_big_tile_short_contractions(device, ta, tb, K):
+    M, N = 3000, 4104
+    a, b = _rand(device, 1, *((K, M) if ta else (M, K))), _rand(device, 2, *((N, K) if tb else (K, N)))
+    want = (a.t() if ta else a).float() @ (b.t() if tb else b).float()
+    assert _rel(ops.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb), out_dtype=torch.float32), want) < 1e-6
+    assert _rel(ops.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb)), want) < 2e-3
+
+
+@pytest.mark.parametrize("K", [72, 256])
+@pytest.mark.parametrize("sizes", [[20000, 0, 1, 300, 257], [4000, 4001, 3999, 4096, 4100]])
+def test_big_tile_groups(device, sizes, K):
+    E, J, N = len(sizes), sum(sizes), 520
+    offs = torch.tensor([0] + sizes, device=device).cumsum(0).to(torch.int32)
+    lhs, rhs = _rand(device, 3, J, K), _rand(device, 4, E, N, K)
+    got = ops.grouped_gemm(lhs, rhs, offs, trans_rhs=True)
+    want = torch.cat([x.float() @ rhs[e].float().t() for e, x in enumerate(lhs.split(sizes))])
+    assert _rel(got, want) < 2e-3
+
+
+@pytest.mark.parametrize("d_in,C", [(200, 136), (64, 72), (8, 128)])
+def test_big_tile_two_segments(device, d_in, C):
+    T, d_out = 4000, 3072
+    x, V, U, W = (_rand(device, 5 + i, *s) for i, s in enumerate([(T, d_in), (d_in, C), (C, d_out), (d_out, d_in)]))
+    m, d = torch.rand(T, C, device=device).to(torch.bfloat16), torch.rand(T, device=device).to(torch.bfloat16)
+    route = torch.arange(T, device=device) % 3 != 0
+    out = site_forward(x, SiteWeights(W, V, U), m, d, route.to(torch.uint8)).output
+    target = x.float() @ W.float().t()
+    xV = (x.float() @ V.float()).to(torch.bfloat16).float()
+    acts = (xV * (m.float() - d.float()[:, None])).to(torch.bfloat16).float()
+    want = torch.where(route[:, None], acts @ U.float() + d.float()[:, None] * target, target)
+    # the stored xV may round to the neighbouring bf16 value in another order of its sum
+    assert _rel(out, want) < 4e-3
