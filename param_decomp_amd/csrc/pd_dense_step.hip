@@ -148,20 +148,29 @@ __global__ __launch_bounds__(SITE_COLS) void k_step_fwd(const T* __restrict__ h,
 // and 7.5e-4 of their scale (worst bin position; sums over tokens average it further),
 // and the table (half as wide in z) by 8.3e-7 for GELU (so |g error| <= 8.3e-7 sum_j
 // |w_out_j|) and 6.9e-5 for its derivative. A component with a wider unit is flagged by
-// the table pass, and both passes evaluate its gate exactly, element by element, as the
-// fp32 step does.
+// the table pass, and its gate is evaluated exactly, element by element, as the fp32 step
+// does, in work of its own (a flagged component on one lane of the binned passes held its
+// whole wave for 64 and 256 serial tokens: with the handful of flagged components that
+// Kaiming gates of C = 4096 have, the 768 -> 3072 step took 1170 us, now 660).
 static constexpr int GATE_TBINS = 32;    // table bins over [min h, max h]
 static constexpr int GATE_MBINS = 16;    // moment bins (pairs of table bins)
 static constexpr int GATE_NC = 8;        // degree-7 table polynomials, 8 Chebyshev moments
 static constexpr int GATE_MOM = GATE_MBINS * GATE_NC;  // moment slots per component (>= 49)
 static constexpr float GATE_DZ_MAX = 3.f;
 static constexpr int RANGE_ROWS = 256;   // tokens per block of the range pass
+static constexpr int RANGE_COLS = 128;   // components per block of the range pass
 static constexpr int FWD_WAVES = 8;      // waves per binned-forward block (each 64 tokens)
 static constexpr int BWD_COLS = 32;      // components per binned-backward block
 static constexpr int BWD_WAVES = 4;      // waves per binned-backward block
 static constexpr int BWD_ROWS = 256;     // tokens per half-wave stream of the backward
 static constexpr int BWD_BLOCK_ROWS = 2 * BWD_WAVES * BWD_ROWS;  // tokens per backward block
-static_assert(GATE_MOM >= 49, "the exact-gate sums share the moment slots");
+static constexpr int EXACT_TOKENS = 2;   // tokens per thread of the flagged components' backward
+static constexpr int EXACT_ROWS = 256 * EXACT_TOKENS;  // tokens per block of it
+// More flagged components than this among 64 go one per lane instead of one token per lane
+// (per wave and component an element and its share of the sums, against 64 or 128 elements
+// whatever the count). All 4096 flagged: 1.28 ms per step, with one token per lane 2.31 ms.
+static constexpr int EXACT_LANES = 32;
+static_assert(GATE_MOM >= 49, "the finalize pass holds a flagged component's 49 sums in its moment slots");
 
 // The Chebyshev nodes x_k = cos((2k+1) pi / 16), k < 8 (T_m(x_k) = cos(m (2k+1) pi / 16)
 // follows by the recurrence T_{m+1} = 2 x T_m - T_{m-1}).
@@ -169,32 +178,48 @@ __constant__ float kChebNode[GATE_NC] = {0.980785280f,  0.831469612f,  0.5555702
                                          -0.195090322f, -0.555570233f, -0.831469612f, -0.980785280f};
 
 // Partial per-component min/max of h over RANGE_ROWS tokens: rng_part[chunk][c] = (min, max).
+// Block = RANGE_COLS components x RANGE_ROWS tokens, 8 components of a row per thread in one
+// 16-byte load (C % 8 == 0, the bf16 products' rule): a pass over h at HBM rate, 22.9 ->
+// 11 us at [4096, 4096] (2-byte loads per lane reached 1.5 TB/s).
 __global__ __launch_bounds__(256) void k_gate_range(const bf16_t* __restrict__ h, int64_t T, int64_t C,
                                                     float2* __restrict__ rng_part) {
-  __shared__ float2 red[4][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t c = (int64_t)blockIdx.x * 64 + lane;
-  const int64_t t0 = (int64_t)blockIdx.y * RANGE_ROWS;
-  float lo = INFINITY, hi = -INFINITY;
+  __shared__ float2 red[16][RANGE_COLS];
+  const int cc = threadIdx.x & 15, rr = threadIdx.x >> 4;
+  const int64_t c = (int64_t)blockIdx.x * RANGE_COLS + cc * 8;
+  const int64_t t0 = (int64_t)blockIdx.y * RANGE_ROWS, t1 = t0 + RANGE_ROWS < T ? t0 + RANGE_ROWS : T;
+  float lo[8], hi[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    lo[e] = INFINITY;
+    hi[e] = -INFINITY;
+  }
   if (c < C)
-    for (int64_t tb = t0 + w * 8; tb < t0 + RANGE_ROWS && tb < T; tb += 32) {  // 8 rows' loads at a time
-      float v[8];
+    for (int64_t tb = t0 + rr; tb < t1; tb += 64) {  // 4 rows' loads at a time
+      uint4 v[4];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = tb + e < T ? bf16_to_f32(h[(tb + e) * C + c]) : v[0];
+      for (int k = 0; k < 4; ++k) v[k] = *(const uint4*)(h + (tb + 16 * k < t1 ? tb + 16 * k : tb) * C + c);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        lo = fminf(lo, v[e]);
-        hi = fmaxf(hi, v[e]);
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = bf16_to_f32((bf16_t)(w[e >> 1] >> (16 * (e & 1))));
+          lo[e] = fminf(lo[e], x);
+          hi[e] = fmaxf(hi[e], x);
+        }
       }
     }
-  red[w][lane] = make_float2(lo, hi);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) red[rr][cc * 8 + e] = make_float2(lo[e], hi[e]);
   __syncthreads();
-  if (w == 0 && c < C) {
-    for (int k = 1; k < 4; ++k) {
-      lo = fminf(lo, red[k][lane].x);
-      hi = fmaxf(hi, red[k][lane].y);
+  const int64_t cw = (int64_t)blockIdx.x * RANGE_COLS + threadIdx.x;
+  if (threadIdx.x < RANGE_COLS && cw < C) {
+    float2 r = red[0][threadIdx.x];
+    for (int k = 1; k < 16; ++k) {
+      r.x = fminf(r.x, red[k][threadIdx.x].x);
+      r.y = fmaxf(r.y, red[k][threadIdx.x].y);
     }
-    rng_part[(int64_t)blockIdx.y * C + c] = make_float2(lo, hi);
+    rng_part[(int64_t)blockIdx.y * C + cw] = r;
   }
 }
 
@@ -347,16 +372,16 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void k_step_fwd_tab(
   const int nc = (int)(s.C - c0 < 64 ? s.C - c0 : 64);
   for (int i = threadIdx.x; i < 64 * GATE_TBINS * 2; i += blockDim.x)
     if ((i & 63) < nc) lt[i] = tab[(c0 + (i & 63)) * GATE_TBINS * 2 + (i >> 6)];
-  if (w == 0 && lane < nc) gate_weights_load(c0 + lane, w_in, b_in, w_out, b_out, wl + lane, 64);
-  __syncthreads();
   const int64_t c = c0 + lane;
+  const float4 rg = rng[c < s.C ? c : c0];
+  const bool exact = c < s.C && rg.w != 0.f;
+  if (w == 0 && exact) gate_weights_load(c, w_in, b_in, w_out, b_out, wl + lane, 64);
+  __syncthreads();
   const int64_t r0 = ((int64_t)blockIdx.y * FWD_WAVES + w) * 64;
   const int64_t r1 = r0 + 64 < s.T ? r0 + 64 : s.T;
   float imp = 0.f, col = 0.f;
-  if (c < s.C && r0 < s.T) {
-    const float4 rg = rng[c];
-    const bool exact = rg.w != 0.f;
-    const int64_t n = s.T * s.C;
+  const int64_t n = s.T * s.C;
+  if (c < s.C && r0 < s.T && !exact) {
     // 8 tokens per step: their h loads go out together, then the 8 elements are computed
     for (int64_t t8 = r0; t8 < r1; t8 += 8) {
       float hv8[8];
@@ -367,12 +392,7 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void k_step_fwd_tab(
         const int64_t t = t8 + e, i = t * s.C + c;
         const float hv = hv8[e];
         const GateCoord q = gate_coord(hv, rg);
-        float g = gate_poly(lt[(2 * q.b) * 64 + lane], lt[(2 * q.b + 1) * 64 + lane], q.tau).x;
-        if (exact) {
-          GeluOut go[16];
-          float gp;
-          g = gate_exact(wl + lane, 64, hv, go, gp);
-        }
+        const float g = gate_poly(lt[(2 * q.b) * 64 + lane], lt[(2 * q.b + 1) * 64 + lane], q.tau).x;
         const float lo = lower_fwd(g);
         const float iv = step_imp(s, upper_fwd(g));
         imp += iv;
@@ -383,6 +403,37 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void k_step_fwd_tab(
       }
     }
     if (s.sl0) s.colpart[(r0 / 64) * s.C + c] = col;
+  }
+  // the block's flagged components: a few one at a time, a wave's 64 tokens on its 64 lanes;
+  // many one per lane
+  auto element = [&](int l, int64_t t) {
+    const int64_t i = t * s.C + c0 + l;
+    const float hv = bf16_to_f32(h[i]);
+    GeluOut go[16];
+    float gp;
+    const float g = gate_exact(wl + l, 64, hv, go, gp);
+    const float lo = lower_fwd(g);
+    const float m = lo + (1.f - lo) * step_uniform_fwd(s, i, n);
+    acts[i] = f32_to_bf16(hv * (m - step_delta(s, t)));
+    return step_imp(s, upper_fwd(g));
+  };
+  unsigned long long left = __ballot(exact);
+  if (__popcll(left) > EXACT_LANES) {
+    left = 0;
+    if (exact && r0 < s.T) {
+      for (int64_t t = r0; t < r1; ++t) col += element(lane, t);
+      imp += col;
+      if (s.sl0) s.colpart[(r0 / 64) * s.C + c] = col;
+    }
+  }
+  for (; left && r0 < s.T; left &= left - 1) {
+    const int l = __ffsll(left) - 1;
+    float iv = r0 + lane < s.T ? element(l, r0 + lane) : 0.f;
+    imp += iv;
+    if (s.sl0) {
+      iv = wave_sum(iv);
+      if (lane == 0) s.colpart[(r0 / 64) * s.C + c0 + l] = iv;
+    }
   }
   imp = wave_sum(imp);
   if (lane == 0) red[w] = imp;
@@ -477,20 +528,17 @@ __global__ __launch_bounds__(SITE_COLS) void k_step_bwd(const T* __restrict__ da
 
 // The bf16 backward with the binned gate. Block = BWD_COLS components x BWD_BLOCK_ROWS
 // tokens in BWD_WAVES waves; lane l of wave w takes component l % 32 and token stream
-// 2w + l / 32 (BWD_ROWS consecutive tokens). Per element: g and dg/dh from the table
-// (exactly, for a flagged component), the squashing pullback dg, dh = da (m - d) + dg g'
+// 2w + l / 32 (BWD_ROWS consecutive tokens). Per element: g and dg/dh from the table,
+// the squashing pullback dg, dh = da (m - d) + dg g'
 // written token-major, and dg T_m(tau_m), m < 8, added into the lane's own LDS slots of its
 // moment bin mb (two 16-byte read-add-writes; one writer per slot and LDS operations of a
-// wave run in order, so the sums are deterministic). A flagged component's lanes keep the
-// 49 exact gate-parameter sums in registers and store them into their first 49 slots at
-// the end. The block then adds its 8 streams per slot in a fixed order: partial[row
-// block][q][c], q < GATE_MOM. LDS: the 32 components' tables (32 KB) and the 4 waves'
+// wave run in order, so the sums are deterministic). A flagged component's lanes do
+// nothing (k_step_bwd_exact). The block then adds its 8 streams per slot in a fixed
+// order: partial[row block][q][c], q < GATE_MOM. LDS: the 32 components' tables (32 KB) and the 4 waves'
 // slots (128 KB).
 __global__ __launch_bounds__(64 * BWD_WAVES) void k_step_bwd_tab(
     const bf16_t* __restrict__ da, const bf16_t* __restrict__ h, const float4* __restrict__ tab,
-    const float4* __restrict__ rng, const float* __restrict__ w_in, const float* __restrict__ b_in,
-    const float* __restrict__ w_out, const float* __restrict__ b_out, StepParams s, bf16_t* __restrict__ dh,
-    float* __restrict__ partial) {
+    const float4* __restrict__ rng, StepParams s, bf16_t* __restrict__ dh, float* __restrict__ partial) {
   __shared__ float4 lt[GATE_TBINS * 2 * BWD_COLS];
   __shared__ float4 mom[BWD_WAVES * GATE_MOM / 4 * 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, cl = lane & (BWD_COLS - 1);
@@ -510,9 +558,8 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_step_bwd_tab(
   __syncthreads();
   const int64_t r0 = (int64_t)by * BWD_BLOCK_ROWS + (2 * w + (lane >> 5)) * BWD_ROWS;
   const int64_t r1 = r0 + BWD_ROWS < s.T ? r0 + BWD_ROWS : s.T;
-  if (c < s.C && r0 < s.T) {
-    const float4 rg = rng[c];
-    const bool exact = rg.w != 0.f;
+  const float4 rg = rng[c < s.C ? c : c0];
+  if (c < s.C && r0 < s.T && rg.w == 0.f) {
     const float dtau_dh = 2.f * rg.y;
     const bool ubyte = s.draw_dtype == PD_DTYPE_BF16;
     const int64_t n = s.T * s.C;
@@ -550,29 +597,27 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_step_bwd_tab(
           u = draw_uniform(s.mk0, s.mk1, i, n, s.draw_dtype, s.layout);
         const float m = lo + (1.f - lo) * u;
         const float dg = lower_vjp(g, dav * hv * (1.f - u)) + upper_vjp(g, step_dimp(s, c, upper_fwd(g)));
-        dh[i] = f32_to_bf16(fmaf(dg, gp, dav * (m - d8[e])));  // a flagged lane rewrites it below
-        if (!exact) {
-          // moment bin mb = b / 2 and its coordinate tau_m = s - 2 mb - 1 in [-1, 1]
-          const int mb = q.b >> 1;
-          const float tm = q.s - (float)(2 * mb) - 1.f, t2 = tm + tm;
-          float p[GATE_NC];
-          p[0] = dg;
-          p[1] = dg * tm;
+        dh[i] = f32_to_bf16(fmaf(dg, gp, dav * (m - d8[e])));
+        // moment bin mb = b / 2 and its coordinate tau_m = s - 2 mb - 1 in [-1, 1]
+        const int mb = q.b >> 1;
+        const float tm = q.s - (float)(2 * mb) - 1.f, t2 = tm + tm;
+        float p[GATE_NC];
+        p[0] = dg;
+        p[1] = dg * tm;
 #pragma unroll
-          for (int k = 2; k < GATE_NC; ++k) p[k] = fmaf(t2, p[k - 1], -p[k - 2]);
-          float4* slot = my + (2 * mb) * 64;
-          float4 a = slot[0], b = slot[64];
-          a.x += p[0];
-          a.y += p[1];
-          a.z += p[2];
-          a.w += p[3];
-          b.x += p[4];
-          b.y += p[5];
-          b.z += p[6];
-          b.w += p[7];
-          slot[0] = a;
-          slot[64] = b;
-        }
+        for (int k = 2; k < GATE_NC; ++k) p[k] = fmaf(t2, p[k - 1], -p[k - 2]);
+        float4* slot = my + (2 * mb) * 64;
+        float4 a = slot[0], b = slot[64];
+        a.x += p[0];
+        a.y += p[1];
+        a.z += p[2];
+        a.w += p[3];
+        b.x += p[4];
+        b.y += p[5];
+        b.z += p[6];
+        b.w += p[7];
+        slot[0] = a;
+        slot[64] = b;
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -581,37 +626,6 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_step_bwd_tab(
         d8[e] = dln[e];
         ub8[e] = ubn[e];
       }
-    }
-    if (exact) {
-      // flagged component: the exact gate, element by element, rewriting dh, with the 49
-      // gate-parameter sums in registers, stored into the lane's first 49 slots
-      float wv[49], acc[49];
-      gate_weights_load(c, w_in, b_in, w_out, b_out, wv, 1);
-#pragma unroll
-      for (int k = 0; k < 49; ++k) acc[k] = 0.f;
-      for (int64_t t = r0; t < r1; ++t) {
-        const int64_t i = t * s.C + c;
-        const float hv = bf16_to_f32(h[i]), dav = bf16_to_f32(da[i]);
-        GeluOut go[16];
-        float gp;
-        const float g = gate_exact(wv, 1, hv, go, gp);
-        const float lo = lower_fwd(g);
-        const float u = step_uniform_bwd(s, i, n);
-        const float m = lo + (1.f - lo) * u;
-        const float dg = lower_vjp(g, dav * hv * (1.f - u)) + upper_vjp(g, step_dimp(s, c, upper_fwd(g)));
-        dh[i] = f32_to_bf16(fmaf(dg, gp, dav * (m - step_delta(s, t))));
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const float dz = dg * wv[32 + j] * go[j].grad;
-          acc[j] = fmaf(dz, hv, acc[j]);
-          acc[16 + j] += dz;
-          acc[32 + j] = fmaf(dg, go[j].gelu, acc[32 + j]);
-        }
-        acc[48] += dg;
-      }
-      float* mf = (float*)(mom + w * (GATE_MOM / 4) * 64);
-#pragma unroll
-      for (int k = 0; k < 49; ++k) mf[mom_index(k, lane)] = acc[k];
     }
   }
   __syncthreads();
@@ -641,15 +655,92 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_step_bwd_tab(
   }
 }
 
+// The backward of the flagged components. Block = 64 components (one flag per lane; without
+// a flagged one it ends there) x EXACT_ROWS tokens. A few flagged components go one at a
+// time with one token per lane, EXACT_TOKENS per thread; many one per lane, a quarter of the
+// block's tokens per wave. Per flagged component dh and the 49 gate-parameter sums, added
+// over the block in a fixed order: xpart[row block][49][c]. Bound by the exact gate's 16
+// erf and exp per element; a launch with nothing flagged is its launch (4.7 us).
+__global__ __launch_bounds__(256) void k_step_bwd_exact(
+    const bf16_t* __restrict__ da, const bf16_t* __restrict__ h, const float4* __restrict__ rng,
+    const float* __restrict__ w_in, const float* __restrict__ b_in, const float* __restrict__ w_out,
+    const float* __restrict__ b_out, StepParams s, bf16_t* __restrict__ dh, float* __restrict__ xpart) {
+  __shared__ float red[49][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t c0 = (int64_t)blockIdx.x * 64, n = s.T * s.C, t0 = (int64_t)blockIdx.y * EXACT_ROWS;
+  float wv[49], acc[49];
+  auto element = [&](int64_t c, int64_t t) {
+    const int64_t i = t * s.C + c;
+    const float hv = bf16_to_f32(h[i]), dav = bf16_to_f32(da[i]);
+    GeluOut go[16];
+    float gp;
+    const float g = gate_exact(wv, 1, hv, go, gp);
+    const float lo = lower_fwd(g);
+    const float u = step_uniform_bwd(s, i, n);
+    const float m = lo + (1.f - lo) * u;
+    const float dg = lower_vjp(g, dav * hv * (1.f - u)) + upper_vjp(g, step_dimp(s, c, upper_fwd(g)));
+    dh[i] = f32_to_bf16(fmaf(dg, gp, dav * (m - step_delta(s, t))));
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const float dz = dg * wv[32 + j] * go[j].grad;
+      acc[j] = fmaf(dz, hv, acc[j]);
+      acc[16 + j] += dz;
+      acc[32 + j] = fmaf(dg, go[j].gelu, acc[32 + j]);
+    }
+    acc[48] += dg;
+  };
+  const bool exact = c0 + lane < s.C && rng[c0 + lane < s.C ? c0 + lane : c0].w != 0.f;
+  unsigned long long left = __ballot(exact);
+  if (__popcll(left) > EXACT_LANES) {
+    const int64_t c = c0 + lane, ta = t0 + w * (EXACT_ROWS / 4);
+#pragma unroll
+    for (int k = 0; k < 49; ++k) acc[k] = 0.f;
+    if (exact) {
+      gate_weights_load(c, w_in, b_in, w_out, b_out, wv, 1);
+      for (int64_t t = ta; t < ta + EXACT_ROWS / 4 && t < s.T; ++t) element(c, t);
+    }
+    for (int k = 0; k < 4; ++k) {  // the waves' sums in token order
+      if (w == k) {
+#pragma unroll
+        for (int q = 0; q < 49; ++q) red[q][lane] = k ? red[q][lane] + acc[q] : acc[q];
+      }
+      __syncthreads();
+    }
+    if (exact)
+      for (int q = w; q < 49; q += 4) xpart[((int64_t)blockIdx.y * 49 + q) * s.C + c] = red[q][lane];
+    return;
+  }
+  for (; left; left &= left - 1) {
+    const int64_t c = c0 + __ffsll(left) - 1;
+    gate_weights_load(c, w_in, b_in, w_out, b_out, wv, 1);
+#pragma unroll
+    for (int k = 0; k < 49; ++k) acc[k] = 0.f;
+    for (int e = 0; e < EXACT_TOKENS; ++e)
+      if (t0 + e * 256 + threadIdx.x < s.T) element(c, t0 + e * 256 + threadIdx.x);
+#pragma unroll
+    for (int k = 0; k < 49; ++k) {
+      const float v = wave_sum(acc[k]);
+      if (lane == 0) red[k][w] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 49) {
+      const float* r = red[threadIdx.x];
+      xpart[((int64_t)blockIdx.y * 49 + threadIdx.x) * s.C + c] = ((r[0] + r[1]) + r[2]) + r[3];
+    }
+    __syncthreads();
+  }
+}
+
 // Gate-parameter gradients from the binned backward's slots. Block = FIN_COLS components;
 // thread = (component, hidden unit j, node quarter). Slots are summed over the row blocks
-// in order. A flagged component's slots hold its exact sums. Otherwise slot (mb, m) holds
+// in order. A flagged component takes its exact sums (xpart). Otherwise slot (mb, m) holds
 // the Chebyshev moment M_m of moment bin mb; its node weights w_k make 128 virtual tokens
 // (h_v, w_v), and each thread takes the exact pullback (GELU with the A&S 7.1.26 erf,
 // |error| <= 1.5e-7) of the 32 in its quarter; the quarters are added in order. db_out =
 // sum over bins of M_0 = sum_t dg_t.
 static constexpr int FIN_COLS = 4;
-__global__ __launch_bounds__(256) void k_gate_finalize(const float* __restrict__ partial, int64_t nchunk, int64_t C,
+__global__ __launch_bounds__(256) void k_gate_finalize(const float* __restrict__ partial, int64_t nchunk,
+                                                       const float* __restrict__ xpart, int64_t nx, int64_t C,
                                                        const float4* __restrict__ rng, const float* __restrict__ w_in,
                                                        const float* __restrict__ b_in, const float* __restrict__ w_out,
                                                        float* __restrict__ dw_in, float* __restrict__ db_in,
@@ -664,7 +755,12 @@ __global__ __launch_bounds__(256) void k_gate_finalize(const float* __restrict__
   const int64_t c0 = (int64_t)lb * FIN_COLS;
   for (int i = threadIdx.x; i < FIN_COLS * GATE_MOM; i += blockDim.x) {
     const int cc = i % FIN_COLS, q = i / FIN_COLS;
-    M[cc][q] = c0 + cc < C ? pd_ordered_sum(partial + (int64_t)q * C + c0 + cc, nchunk, (int64_t)GATE_MOM * C) : 0.f;
+    float v = 0.f;
+    if (c0 + cc < C) {
+      if (rng[c0 + cc].w == 0.f) v = pd_ordered_sum(partial + (int64_t)q * C + c0 + cc, nchunk, (int64_t)GATE_MOM * C);
+      else if (q < 49) v = pd_ordered_sum(xpart + (int64_t)q * C + c0 + cc, nx, 49 * C);
+    }
+    M[cc][q] = v;
   }
   __syncthreads();
   for (int i = threadIdx.x; i < FIN_COLS * GATE_MOM; i += blockDim.x) {
@@ -789,7 +885,7 @@ __global__ void k_step_losses(const float* __restrict__ rec_part, int64_t n_rec,
 }
 
 struct StepWorkspace {
-  size_t yt, h, graw, acts, y, dy, da, dh, imp, rec, gate, delta, ubits, rng_part, rng, tab, sl0_col, sl0_slope,
+  size_t yt, h, graw, acts, y, dy, da, dh, imp, rec, gate, xgate, delta, ubits, rng_part, rng, tab, sl0_col, sl0_slope,
       sl0_act, sl0_freq, sl0_fb, total;
 };
 
@@ -815,6 +911,7 @@ static StepWorkspace step_layout(int dtype, int64_t T, int64_t d_in, int64_t d_o
   take(w.imp, 4 * cdiv(T, SITE_ROWS) * cdiv(C, SITE_COLS));
   take(w.rec, 4 * cdiv(T, TP) * cdiv(d_out, TP));
   take(w.gate, bf ? 4 * cdiv(T, BWD_BLOCK_ROWS) * GATE_MOM * C : 4 * cdiv(T, SITE_ROWS) * 49 * C);
+  take(w.xgate, bf ? 4 * cdiv(T, EXACT_ROWS) * 49 * C : 0);
   take(w.delta, 4 * T);
   take(w.ubits, (size_t)T * C);
   take(w.rng_part, 8 * cdiv(T, RANGE_ROWS) * C);
@@ -860,6 +957,7 @@ static int dense_step_impl(int dtype, int64_t T, int64_t d_in, int64_t d_out, in
   float* imp_part = (float*)(ws + L.imp);
   float* rec_part = (float*)(ws + L.rec);
   float* gate_part = (float*)(ws + L.gate);
+  float* xpart = (float*)(ws + L.xgate);
   const bool bf = dtype == PD_DTYPE_BF16;
   float* delta = use_delta ? (float*)(ws + L.delta) : nullptr;
   const bool sl0 = imp.kind == PD_IMPMIN_SMOOTH_L0;
@@ -888,7 +986,7 @@ static int dense_step_impl(int dtype, int64_t T, int64_t d_in, int64_t d_out, in
   if (bf) {
     float2* rng_part = (float2*)(ws + L.rng_part);
     const int nchunk = (int)cdiv(T, RANGE_ROWS);
-    hipLaunchKernelGGL(k_gate_range, dim3((unsigned)cdiv(C, 64), (unsigned)nchunk), dim3(256), 0, s, (const bf16_t*)h,
+    hipLaunchKernelGGL(k_gate_range, dim3((unsigned)cdiv(C, RANGE_COLS), (unsigned)nchunk), dim3(256), 0, s, (const bf16_t*)h,
                        T, C, rng_part);
     hipLaunchKernelGGL(k_gate_table, dim3((unsigned)cdiv(C * GATE_TBINS, 256)), dim3(256), 0, s, rng_part, nchunk, C,
                        w_in, b_in, w_out, b_out, (float*)tab, rng);
@@ -932,16 +1030,20 @@ static int dense_step_impl(int dtype, int64_t T, int64_t d_in, int64_t d_out, in
   if ((rc = pd_gemm(dtype, T, C, d_out, dy, d_out, 0, U, d_out, 1, da, C, dtype, 1.f, 0.f, stream))) return rc;
   PD_MARK(9);
   const dim3 bgrid((unsigned)cdiv(C, BWD_COLS), (unsigned)cdiv(T, BWD_BLOCK_ROWS));
-  if (bf)
+  if (bf) {
     hipLaunchKernelGGL(k_step_bwd_tab, bgrid, dim3(64 * BWD_WAVES), 0, s, (const bf16_t*)da, (const bf16_t*)h,
-                       (const float4*)tab, (const float4*)rng, w_in, b_in, w_out, b_out, sp, (bf16_t*)dh, gate_part);
-  else
+                       (const float4*)tab, (const float4*)rng, sp, (bf16_t*)dh, gate_part);
+    hipLaunchKernelGGL(k_step_bwd_exact, dim3((unsigned)cdiv(C, 64), (unsigned)cdiv(T, EXACT_ROWS)), dim3(256), 0, s,
+                       (const bf16_t*)da, (const bf16_t*)h, (const float4*)rng, w_in, b_in, w_out, b_out, sp,
+                       (bf16_t*)dh, xpart);
+  } else
     hipLaunchKernelGGL((k_step_bwd<float, true>), cgrid, dim3(SITE_COLS), 0, s, (const float*)da, (const float*)h,
                        graw, w_in, b_in, w_out, sp, (float*)dh, gate_part);
   if ((rc = check_launch("pd_dense_step bwd"))) return rc;
   PD_MARK(10);
   if (bf)
-    hipLaunchKernelGGL(k_gate_finalize, dim3((unsigned)cdiv(C, FIN_COLS)), dim3(256), 0, s, gate_part, (int64_t)bgrid.y, C,
+    hipLaunchKernelGGL(k_gate_finalize, dim3((unsigned)cdiv(C, FIN_COLS)), dim3(256), 0, s, gate_part, (int64_t)bgrid.y,
+                       (const float*)xpart, cdiv(T, EXACT_ROWS), C,
                        (const float4*)rng, w_in, b_in, w_out, dw_in, db_in, dw_out, db_out);
   else
     hipLaunchKernelGGL(k_step_gate_reduce, dim3((unsigned)cdiv(49 * C, 256)), dim3(256), 0, s, gate_part,
