@@ -582,7 +582,7 @@ int pd_lm_stack_step_timed(int64_t B, int64_t T, int d, int n_head, int n_kv_hea
  * [n_tokens, dims[0]]; weights[i] bf16 [dims[i], dims[i+1]] (the reference's "i o"
  * layout); biases[i] bf16 [dims[i+1]]; preact bf16 [n_tokens, dims[n]]. bf16 compute
  * with fp32 accumulation, every product, bias sum and GELU rounded to bf16 as the
- * engine's bf16 compute cast does. The forward keeps W^T copies and every hidden z_i and
+ * engine's bf16 compute cast does. The forward keeps every hidden z_i and
  * a_i in the workspace; pd_ci_mlp_bwd reads them, so it takes the forward's workspace
  * unchanged. dims, weights, biases, d_weights and d_biases are HOST arrays of device
  * pointers. All tensors 16-byte aligned. n_layers <= 16. */

@@ -64,82 +64,96 @@ static void ci_transpose(const bf16_t* src, int64_t R, int64_t Cc, bf16_t* dst, 
                      Cc, dst, ldd);
 }
 
+// A tile's bf16(acc) through the staged LDS image, 8 consecutive columns of a row at a time:
+// f(row, col, v) with v the 8 rounded values (N % 8 == 0). From the MFMA layout each store
+// instruction would write 16 bytes into 32 rows; through the image whole lines.
+template <class CFG, class F>
+__device__ inline void staged_rows(const GemmArgs& p, const TileJob& t, int wm, int wn, int tid,
+                                   f32x16 (&acc)[CFG::TM][CFG::TN], char* smem, F&& f) {
+  typedef StagedStore<CFG, 2> SS;
+  constexpr int CPR = CFG::BN / 8, RPP = CFG::NT / CPR;
+  static_assert(SS::OK && CFG::NT % CPR == 0 && SS::ROWS % RPP == 0, "image passes");
+  const int rr = tid / CPR, cc = tid % CPR;
+  const int64_t col = t.n0 + cc * 8;
+#pragma unroll
+  for (int q = 0; q < SS::PASSES; ++q) {
+    staged_image_pass<CFG, 2>(1.f, q, wm, wn, tid & 63, acc, smem);
+#pragma unroll 2
+    for (int r = rr; r < SS::ROWS; r += RPP) {
+      const int64_t row = t.m0 + q * SS::ROWS + r;
+      if (row >= t.M || col >= p.N) continue;
+      const uint4 w = *(const uint4*)(smem + r * SS::RSB + cc * 16);
+      const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = bf16_to_f32((bf16_t)(ww[e >> 1] >> (16 * (e & 1))));
+      f(row, col, v);
+    }
+  }
+}
+__device__ inline void load_bf16x8(const bf16_t* p, float* v) {
+  const uint4 w = *(const uint4*)p;
+  const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = bf16_to_f32((bf16_t)(ww[e >> 1] >> (16 * (e & 1))));
+}
+__device__ inline void store_bf16x8(bf16_t* p, const float* v) {
+  *(uint4*)p = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                          pack_bf16x2(v[6], v[7]));
+}
+
 // Epilogue of L_i: z = bf16(bf16(acc) + b); a hidden layer stores z to zsave and
-// bf16(GELU(z)) to C, the head stores z to C. N % 4 == 0.
+// bf16(GELU(z)) to C, the head stores z to C. N % 8 == 0.
 struct EpiBiasGelu {
   static constexpr int LDS_BYTES = 0;
+  static constexpr bool BIG_OK = true;
   struct Args {
     const bf16_t* bias;
     bf16_t* zsave;  // NULL for the head
   };
   template <class CFG, typename TC>
   __device__ static void run(const GemmArgs& p, const Args& a, const TileJob& t, int wm, int wn, int tid,
-                             f32x16 (&acc)[CFG::TM][CFG::TN], char*) {
-    const int lane = tid & 63;
+                             f32x16 (&acc)[CFG::TM][CFG::TN], char* smem) {
     bf16_t* C = (bf16_t*)t.C;
+    const int64_t bc = t.n0 + (tid % (CFG::BN / 8)) * 8;
+    float b[8] = {};
+    if (bc < p.N) load_bf16x8(a.bias + bc, b);
+    staged_rows<CFG>(p, t, wm, wn, tid, acc, smem, [&](int64_t row, int64_t col, float* v) {
+      const int64_t idx = row * p.ldc + col;
 #pragma unroll
-    for (int i = 0; i < CFG::TM; ++i) {
-      const int64_t row = t.m0 + wm * CFG::WTM + i * 32 + (lane & 31);
-      if (row >= t.M) continue;
+      for (int e = 0; e < 8; ++e) v[e] = bfr(v[e] + b[e]);
+      if (a.zsave) {
+        store_bf16x8(a.zsave + idx, v);
 #pragma unroll
-      for (int j = 0; j < CFG::TN; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * g + 4 * (lane >> 5);
-          if (col >= p.N) continue;
-          const uint2 bw = *(const uint2*)(a.bias + col);
-          const float b[4] = {bf16_to_f32((bf16_t)(bw.x & 0xFFFF)), bf16_to_f32((bf16_t)(bw.x >> 16)),
-                              bf16_to_f32((bf16_t)(bw.y & 0xFFFF)), bf16_to_f32((bf16_t)(bw.y >> 16))};
-          float z[4], o[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            z[e] = bfr(bfr(acc[i][j][4 * g + e]) + b[e]);
-            o[e] = a.zsave ? gelu_and_grad<true>(z[e]).gelu : z[e];
-          }
-          const int64_t idx = row * p.ldc + col;
-          if (a.zsave) *(uint2*)(a.zsave + idx) = make_uint2(pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3]));
-          *(uint2*)(C + idx) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-        }
-    }
+        for (int e = 0; e < 8; ++e) v[e] = gelu_and_grad<true>(v[e]).gelu;
+      }
+      store_bf16x8(C + idx, v);
+    });
   }
 };
 
 // Epilogue of d_a = d_z @ W^T: d_a = bf16(acc); with z given, C = bf16(d_a * GELU'(z)),
-// else C = d_a. N % 4 == 0.
+// else C = d_a. N % 8 == 0.
 struct EpiGeluGrad {
   static constexpr int LDS_BYTES = 0;
+  static constexpr bool BIG_OK = true;
   struct Args {
     const bf16_t* z;  // saved pre-activations [M, N] (ld = ldc), or NULL
   };
   template <class CFG, typename TC>
   __device__ static void run(const GemmArgs& p, const Args& a, const TileJob& t, int wm, int wn, int tid,
-                             f32x16 (&acc)[CFG::TM][CFG::TN], char*) {
-    const int lane = tid & 63;
+                             f32x16 (&acc)[CFG::TM][CFG::TN], char* smem) {
     bf16_t* C = (bf16_t*)t.C;
+    staged_rows<CFG>(p, t, wm, wn, tid, acc, smem, [&](int64_t row, int64_t col, float* v) {
+      const int64_t idx = row * p.ldc + col;
+      if (a.z) {
+        float z[8];
+        load_bf16x8(a.z + idx, z);
 #pragma unroll
-    for (int i = 0; i < CFG::TM; ++i) {
-      const int64_t row = t.m0 + wm * CFG::WTM + i * 32 + (lane & 31);
-      if (row >= t.M) continue;
-#pragma unroll
-      for (int j = 0; j < CFG::TN; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * g + 4 * (lane >> 5);
-          if (col >= p.N) continue;
-          const int64_t idx = row * p.ldc + col;
-          float o[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = bfr(acc[i][j][4 * g + e]);
-          if (a.z) {
-            const uint2 zw = *(const uint2*)(a.z + idx);
-            const float z[4] = {bf16_to_f32((bf16_t)(zw.x & 0xFFFF)), bf16_to_f32((bf16_t)(zw.x >> 16)),
-                                bf16_to_f32((bf16_t)(zw.y & 0xFFFF)), bf16_to_f32((bf16_t)(zw.y >> 16))};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] *= gelu_and_grad<true>(z[e]).grad;
-          }
-          *(uint2*)(C + idx) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-        }
-    }
+        for (int e = 0; e < 8; ++e) v[e] *= gelu_and_grad<true>(z[e]).grad;
+      }
+      store_bf16x8(C + idx, v);
+    });
   }
 };
 
@@ -206,13 +220,23 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ par
   if (w == 0 && j < n) out[j] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
+// Contraction slices of a weight gradient (1: none): where fewer than 192 128x128 tiles
+// leave CUs idle, enough for about 384 blocks, each at least 512 tokens deep. 768x1024 over
+// 4096 tokens 50 -> 16 us in 8 slices; at 256 tiles two slices gain nothing over their sum.
+static int mlp_dw_splits(int64_t din, int64_t dout, int64_t N) {
+  const int64_t tiles = cdiv(din, 128) * cdiv(dout, 128);
+  if (tiles >= 192 || !dtl_fits_mn(N, din) || !dtl_fits_mn(N, dout)) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(384 / tiles, N / 512), 16));
+}
+
 // ---------------------------------------------------------------- MLP workspace
 struct MlpPlan {
-  bf16_t* WT[MLP_MAX_LAYERS];  // W_i^T [d_i+1, d_i]
+  bf16_t* WT;                  // a weight's transposed copy, where one is needed
   bf16_t* Z[MLP_MAX_LAYERS];   // hidden pre-activations [N, d_i+1]
   bf16_t* A[MLP_MAX_LAYERS];   // hidden activations [N, d_i+1]
   bf16_t *dz_a, *dz_b;         // backward ping-pong [N, max d]
-  bf16_t *aT, *dzT;            // K-contiguous copies [max d, Np], Np = N rounded up to 8
+  float* sk;                   // the weight gradients' contraction slices
+  size_t sk_bytes;
   float* part;                 // column-sum partials [N / MLP_SUM_ROWS, max d]
   size_t total;
 };
@@ -227,16 +251,19 @@ static MlpPlan mlp_plan(int L, const int64_t* dims, int64_t N, char* base) {
   };
   int64_t mx = 0;
   for (int i = 0; i <= L; ++i) mx = std::max(mx, dims[i]);
-  for (int i = 0; i < L; ++i) P.WT[i] = (bf16_t*)take(2 * (size_t)dims[i] * dims[i + 1]);
+  size_t wt = 0;
+  for (int i = 0; i < L; ++i) {
+    if (!dtl_fits_mn(dims[i], dims[i + 1])) wt = std::max(wt, 2 * (size_t)dims[i] * dims[i + 1]);
+    P.sk_bytes = std::max(P.sk_bytes, gemm_splitk_ws_bytes(dims[i], dims[i + 1], N, mlp_dw_splits(dims[i], dims[i + 1], N)));
+  }
+  P.WT = (bf16_t*)take(wt);
   for (int i = 0; i + 1 < L; ++i) {
     P.Z[i] = (bf16_t*)take(2 * (size_t)N * dims[i + 1]);
     P.A[i] = (bf16_t*)take(2 * (size_t)N * dims[i + 1]);
   }
   P.dz_a = (bf16_t*)take(2 * (size_t)N * mx);
   P.dz_b = (bf16_t*)take(2 * (size_t)N * mx);
-  const int64_t Np = (N + 7) & ~(int64_t)7;
-  P.aT = (bf16_t*)take(2 * (size_t)Np * mx);
-  P.dzT = (bf16_t*)take(2 * (size_t)Np * mx);
+  P.sk = (float*)take(P.sk_bytes);
   P.part = (float*)take(4 * (size_t)cdiv(N, MLP_SUM_ROWS) * mx);
   P.total = off;
   return P;
@@ -516,13 +543,18 @@ int pd_ci_mlp_fwd(int n_layers, const int64_t* dims, int64_t n_tokens, const voi
   const bf16_t* a = (const bf16_t*)x;
   for (int i = 0; i < n_layers; ++i) {
     const int64_t din = dims[i], dout = dims[i + 1];
-    ci_transpose((const bf16_t*)weights[i], din, dout, P.WT[i], din, s);
     const bool head = i + 1 == n_layers;
     bf16_t* out = head ? (bf16_t*)preact : P.A[i];
-    GemmArgs g{n_tokens, dout, din, a, din, P.WT[i], din, out, dout, 1.f, 0.f, nullptr, 0, 0, 0, 0,
-               nullptr, nullptr, nullptr};
+    // W_i [din, dout] as stored (MN-major); only a weight whose last stage would reach past
+    // the kernel's 31-bit range goes through a transposed copy
+    const bool mn = dtl_fits_mn(din, dout);
+    if (!mn) ci_transpose((const bf16_t*)weights[i], din, dout, P.WT, din, s);
+    GemmArgs g{n_tokens, dout, din, a, din, mn ? (const bf16_t*)weights[i] : P.WT, mn ? dout : din, out, dout, 1.f, 0.f,
+               nullptr, 0, 0, 0, 0, nullptr, nullptr, nullptr};
     EpiBiasGelu::Args ea{(const bf16_t*)biases[i], head ? nullptr : P.Z[i]};
-    if ((rc = launch_dense_epi<EpiBiasGelu, bf16_t>(g, ea, s, "pd_ci_mlp_fwd"))) return rc;
+    rc = mn ? launch_dense_epi<EpiBiasGelu, bf16_t, true>(g, ea, s, "pd_ci_mlp_fwd")
+            : launch_dense_epi<EpiBiasGelu, bf16_t>(g, ea, s, "pd_ci_mlp_fwd");
+    if (rc) return rc;
     a = out;
   }
   return PD_OK;
@@ -543,7 +575,7 @@ int pd_ci_mlp_bwd(int n_layers, const int64_t* dims, int64_t n_tokens, const voi
     return fail(PD_EWORKSPACE, "pd_ci_mlp_bwd: workspace too small");
   const MlpPlan P = mlp_plan(n_layers, dims, n_tokens, (char*)workspace);
   hipStream_t s = (hipStream_t)stream;
-  const int64_t N = n_tokens, Np = (N + 7) & ~(int64_t)7, nchunk = cdiv(N, MLP_SUM_ROWS);
+  const int64_t N = n_tokens, nchunk = cdiv(N, MLP_SUM_ROWS);
   const bf16_t* dz = (const bf16_t*)d_preact;
   for (int i = n_layers - 1; i >= 0; --i) {
     const int64_t din = dims[i], dout = dims[i + 1];
@@ -553,11 +585,9 @@ int pd_ci_mlp_bwd(int n_layers, const int64_t* dims, int64_t n_tokens, const voi
                        P.part);
     hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)cdiv(dout, 64)), dim3(256), 0, s, P.part, nchunk, dout,
                        d_biases[i]);
-    // dW_i [din, dout] = a^T [din, N] @ (d_z^T [dout, N])^T
-    ci_transpose(ain, N, din, P.aT, Np, s);
-    ci_transpose(dz, N, dout, P.dzT, Np, s);
-    if ((rc = pd_gemm(PD_DTYPE_BF16, din, dout, Np, P.aT, Np, 0, P.dzT, Np, 1, d_weights[i], dout, PD_DTYPE_F32, 1.f,
-                      0.f, stream)))
+    // dW_i [din, dout] = a^T @ d_z, both as stored (token rows are the contraction)
+    if ((rc = gemm_splitk(din, dout, N, ain, din, 1, dz, dout, 0, d_weights[i], dout, PD_DTYPE_F32, 0.f, P.sk,
+                          P.sk_bytes, stream, mlp_dw_splits(din, dout, N))))
       return rc;
     // d_a = d_z @ W_i^T (B = W_i stored [din, dout]: [N, K] K-contiguous), then the GELU
     // pullback of layer i-1, or the input gradient

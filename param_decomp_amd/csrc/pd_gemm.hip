@@ -546,7 +546,7 @@ static int launch_dtl(const GemmArgs& a, int c_dtype, bool kedge, dim3 grid, hip
 }
 
 // Any operand layout through the buffer-fed kernel (a_kmaj / b_kmaj: K-contiguous), in 256x256
-// or 128x128 tiles.
+// (`big`) or 128x128 tiles.
 template <int MODE, bool BIG_OK>
 static int launch_dtl_any(const GemmArgs& a, bool a_kmaj, bool b_kmaj, int c_dtype, bool kedge, bool big,
                           unsigned batch, hipStream_t s) {
@@ -556,6 +556,8 @@ static int launch_dtl_any(const GemmArgs& a, bool a_kmaj, bool b_kmaj, int c_dty
   {                                                                                                 \
     if constexpr (BIG_OK)                                                                           \
       if (big) return launch_dtl<CfgDtlBig, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);            \
+    if constexpr (MODE == MODE_DENSE && !(AMN) && !(BMN))                                           \
+      if (deep_ring(a.M, a.N, a.K)) return launch_dtl<CfgDtlDeep, MODE>(a, c_dtype, kedge, grid, s); \
     return launch_dtl<CfgDtlSmall<AMN, BMN>, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);           \
   }
   if (a_kmaj && b_kmaj) PD_L(false, false)

@@ -13,7 +13,7 @@
 // record count ends at the operand's last row, so rows past the operand extent, and
 // chunks past the end of its last row, load as zeros; their outputs are never stored.
 //
-// Two LDS stages, software-pipelined inside a wave (pipe_stage). A stage is four k16 steps;
+// Two (or four) LDS stages, software-pipelined inside a wave (pipe_stage). A stage is four k16 steps;
 // the fragments of step n+1 are read from LDS between the MFMAs of step n (two register
 // sets), and the last step of a stage reads the first fragments of the next one, after the
 // one barrier of the stage: this wave's loads of the next stage have landed (vmcnt) and
@@ -260,10 +260,11 @@ __device__ inline bool map_tile(const GemmArgs& p, int lane, TileJob& t) {
   return t.m0 < t.M && t.n0 < p.N;
 }
 
-// SPLIT: the loads of a stage go out in two halves (see the top of this file).
-template <int BM_, int BN_, int WM_, int WN_, bool SPLIT_>
+// SPLIT: the loads of a stage go out in two halves; NS: LDS stages, a power of two (see the
+// top of this file).
+template <int BM_, int BN_, int WM_, int WN_, bool SPLIT_, int NS_ = 2>
 struct DtlCfg {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = 2, BK = 64;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, BK = 64;
   static constexpr int NW = WM_ * WN_, NT = NW * 64;
   static constexpr int WTM = BM_ / WM_, WTN = BN_ / WN_;  // wave tile
   static constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -276,7 +277,10 @@ struct DtlCfg {
   static_assert(NW % 2 == 0, "the swizzle parity of a wave's rows must not depend on the load index");
   static_assert(BM_ % (RPI * NW) == 0 && BN_ % (RPI * NW) == 0, "every wave moves whole 1 KB row blocks");
   static_assert(TM >= 1 && TN >= 1 && WTM % 32 == 0 && WTN % 32 == 0, "wave tile is a multiple of 32x32");
-  static_assert(NS * STAGE_BYTES <= 160 * 1024, "LDS");
+  static_assert((NS & (NS - 1)) == 0 && NS * STAGE_BYTES <= 160 * 1024, "LDS");
+  static_assert(NS == 2 || !SPLIT_, "split loads are written for two stages");
+  // loads in flight that a stage's readers need not wait for: those of the later stages
+  static constexpr int AHEAD = (NS - 2) * INSTS;
 };
 
 // s_waitcnt on the vector-memory counter only (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] |
@@ -287,8 +291,13 @@ __device__ inline void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-// Waits for this wave's buffer loads (vmcnt = 0) and its LDS operations (lgkmcnt = 0).
-__device__ inline void wait_loads_and_lds() { __builtin_amdgcn_s_waitcnt(7 << 4); }
+// Waits until at most N of this wave's buffer loads are in flight and for its LDS operations
+// (lgkmcnt = 0).
+template <int N>
+__device__ inline void wait_loads_and_lds() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
+}
 
 // A bare s_barrier: it orders the waves but waits for none of this wave's memory
 // operations (gfx950 inserts no wait before s_barrier). It suffices where the LDS data
@@ -327,6 +336,15 @@ __device__ inline int64_t uni64(int64_t v) {
 // 18.6 us, both MN-major 768x4096x4096 51 (8 waves) against 55; loads in two halves: 60.
 typedef DtlCfg<128, 128, 4, 2, false> CfgDtl;
 typedef DtlCfg<128, 128, 2, 2, false> CfgDtlRA;
+// The same tile with a four-stage ring (one block per CU), for launches of at most one block
+// per CU over a long contraction: a lone block waits out the latency of loads issued only
+// one stage ahead. 3001x768x4096 41.6 -> 31.3 us, 4096x1024x768 12.5 -> 11.1; with an
+// MN-major operand (bound by its transposing reads) 52 -> 52, over K = 384 5.6 -> 6.3, and
+// with more tiles than CUs the second block is worth more (8192x1024x768 17.6 -> 19.4).
+typedef DtlCfg<128, 128, 4, 2, false, 4> CfgDtlDeep;
+inline bool deep_ring(int64_t M, int64_t N, int64_t K) {
+  return ((M + 127) / 128) * ((N + 127) / 128) <= 256 && K >= 768;
+}
 // 256x256x64 tiles, 8 waves (128 KB of LDS, one block per CU): fewer LDS bytes per MFMA.
 typedef DtlCfg<256, 256, 2, 4, true> CfgDtlBig;
 template <bool AMN, bool BMN>
@@ -558,9 +576,10 @@ __device__ inline void spread_step() {
 
 // The stage's four k16 steps (see the top of this file). Before: f[0] holds the stage's
 // step 0. read(kk, f): the stage's step kk; read_next(f): the next stage's step 0;
-// issue(ahead, half): that half of the loads of the stage `ahead` stages on; mfma(kk, f):
+// issue(ahead, half): that half of the loads of the stage `ahead` stages
+// on (NS stages, AHEAD loads of the later ones left in flight); mfma(kk, f):
 // step kk's products. MFMAS, READS: a step's MFMAs and LDS reads; LOADS0, LOADS3: the loads issued in steps 0 and 3.
-template <int MFMAS, int READS, int LOADS0, int LOADS3, class F, class Read, class ReadNext, class Issue, class Mfma>
+template <int MFMAS, int READS, int LOADS0, int LOADS3, int NS, int AHEAD, class F, class Read, class ReadNext, class Issue, class Mfma>
 __device__ inline void pipe_stage(F (&f)[2], Read&& read, ReadNext&& read_next, Issue&& issue, Mfma&& mfma) {
   read(1, f[1]);
   issue(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
@@ -572,10 +591,10 @@ __device__ inline void pipe_stage(F (&f)[2], Read&& read, ReadNext&& read_next, 
   read(3, f[1]);
   mfma(2, f[0]);
   spread_step<MFMAS, READS, 0>();
-  wait_loads_and_lds();
+  wait_loads_and_lds<AHEAD>();
   lds_barrier();
   read_next(f[0]);
-  issue(std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
+  issue(std::integral_constant<int, NS>{}, std::integral_constant<int, 0>{});
   mfma(3, f[1]);
   spread_step<MFMAS, READS, LOADS3>();
 }
@@ -768,23 +787,26 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
     constexpr int LO = decltype(h)::value ? CFG::HALF : 0, HI = decltype(h)::value ? CFG::INSTS : CFG::HALF;
     const uint32_t kpos = (uint32_t)(kbeg + kt * BK);
     const bool in = kt < nk;
-    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & 1) * CFG::STAGE_BYTES, abase, uni(in ? abytes : 0), offa,
+    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES, abase, uni(in ? abytes : 0), offa,
                               kpos * kstep_a, bbase, uni(in ? bbytes : 0), offb, kpos * kstep_b, wave);
   };
-  issue(0, std::integral_constant<int, 0>{});
-  issue(0, std::integral_constant<int, 1>{});
-  issue(1, std::integral_constant<int, 0>{});
+#pragma unroll
+  for (int st = 0; st < CFG::NS - 1; ++st) {
+    issue(st, std::integral_constant<int, 0>{});
+    issue(st, std::integral_constant<int, 1>{});
+  }
+  issue(CFG::NS - 1, std::integral_constant<int, 0>{});
 
   const FragOffs<CFG, AMN, BMN> fo(wm, wn, lane);
   Frags<CFG> f[2];
-  wait_vmcnt<CFG::HALF>();
+  wait_vmcnt<CFG::AHEAD + CFG::HALF>();
   lds_barrier();
   read_frags<CFG>(smem, fo, lane, 0, f[0]);
   constexpr int READS = TM * (AMN ? 2 : 1) + TN * (BMN ? 2 : 1);
   auto stage = [&](int64_t kt, auto edge) {
-    const char* st = smem + (int)(kt & 1) * CFG::STAGE_BYTES;
-    const char* nx = smem + (int)(~kt & 1) * CFG::STAGE_BYTES;
-    pipe_stage<TM * TN, READS, CFG::INSTS - CFG::HALF, CFG::HALF>(
+    const char* st = smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES;
+    const char* nx = smem + (int)((kt + 1) & (CFG::NS - 1)) * CFG::STAGE_BYTES;
+    pipe_stage<TM * TN, READS, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD>(
         f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
         [&](Frags<CFG>& g) { read_frags<CFG>(nx, fo, lane, 0, g); },
         [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
@@ -884,7 +906,7 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
   auto stage = [&](int64_t kt, auto edge) {
     const char* st = smem + (int)(kt & 1) * SB;
     const char* nx = smem + (int)(~kt & 1) * SB;
-    pipe_stage<2 * TM * TN, 2 * TM + (SHARED_B ? 1 : 2) * TN, (SPLIT ? LOADS1 : 0), CFG::INSTS + (SPLIT ? 0 : LOADS1)>(
+    pipe_stage<2 * TM * TN, 2 * TM + (SHARED_B ? 1 : 2) * TN, (SPLIT ? LOADS1 : 0), CFG::INSTS + (SPLIT ? 0 : LOADS1), 2, 0>(
         f, [&](int kk, F2& g) { read(st, kk, g); }, [&](F2& g) { read(nx, 0, g); },
         [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
         [&](int kk, F2& g) {
@@ -1000,27 +1022,30 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
     const uint32_t kpos = (uint32_t)((s1 ? kt : kt - nk1) * BK);
     const LaneOff oa{s1 ? oa1.off : oa2.off, s1 ? oa1.step : oa2.step};
     const LaneOff ob{s1 ? ob1.off : ob2.off, s1 ? ob1.step : ob2.step};
-    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & 1) * CFG::STAGE_BYTES, (const bf16_t*)uni64((int64_t)(s1 ? a1 : a2)),
+    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES, (const bf16_t*)uni64((int64_t)(s1 ? a1 : a2)),
                               uni(in ? (s1 ? a1bytes : a2bytes) : 0), oa, kpos * 2,
                               (const bf16_t*)uni64((int64_t)(s1 ? b1 : b2)),
                               uni(in ? (s1 ? b1bytes : b2bytes) : 0), ob, kpos * (s1 ? ks1 : ks2), wave);
   };
-  issue(0, std::integral_constant<int, 0>{});
-  issue(0, std::integral_constant<int, 1>{});
-  issue(1, std::integral_constant<int, 0>{});
+#pragma unroll
+  for (int st = 0; st < CFG::NS - 1; ++st) {
+    issue(st, std::integral_constant<int, 0>{});
+    issue(st, std::integral_constant<int, 1>{});
+  }
+  issue(CFG::NS - 1, std::integral_constant<int, 0>{});
 
   const FragOffs<CFG, false, B1MN> fo1(wm, wn, lane);
   const FragOffs<CFG, false, B2MN> fo2(wm, wn, lane);
   Frags<CFG> f[2];
-  wait_vmcnt<CFG::HALF>();
+  wait_vmcnt<CFG::AHEAD + CFG::HALF>();
   lds_barrier();
   read_frags<CFG>(smem, fo1, lane, 0, f[0]);
   // stage kt of a segment whose fragments sit at fo, the next stage's at fon; its k range
   // starts at k0 and ends at kend
   auto stage = [&](int64_t kt, const auto& fo, const auto& fon, int64_t k0, int64_t kend, auto edge, auto reads) {
-    const char* st = smem + (int)(kt & 1) * CFG::STAGE_BYTES;
-    const char* nx = smem + (int)(~kt & 1) * CFG::STAGE_BYTES;
-    pipe_stage<TM * TN, decltype(reads)::value, CFG::INSTS - CFG::HALF, CFG::HALF>(
+    const char* st = smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES;
+    const char* nx = smem + (int)((kt + 1) & (CFG::NS - 1)) * CFG::STAGE_BYTES;
+    pipe_stage<TM * TN, decltype(reads)::value, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD>(
         f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
         [&](Frags<CFG>& g) { read_frags<CFG>(nx, fon, lane, 0, g); },
         [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
@@ -1054,21 +1079,27 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
   EPI::template run<CFG, TC>(p, ea, t, wm, wn, tid, acc, smem);
 }
 
+template <class CFG, class EPI, typename TC, bool BMN>
+inline void launch_epi_cfg(const GemmArgs& a, const typename EPI::Args& ea, hipStream_t s) {
+  const dim3 grid((unsigned)((a.N + CFG::BN - 1) / CFG::BN), (unsigned)((a.M + CFG::BM - 1) / CFG::BM));
+  if (a.K % CFG::BK)
+    hipLaunchKernelGGL((k_gemm_dtl<CFG, TC, MODE_DENSE, true, EPI, false, BMN>), grid, dim3(CFG::NT), 0, s, a, ea);
+  else
+    hipLaunchKernelGGL((k_gemm_dtl<CFG, TC, MODE_DENSE, false, EPI, false, BMN>), grid, dim3(CFG::NT), 0, s, a, ea);
+}
+
 // Dense C = A [M, K] @ B^T (B stored [N, K], both K-contiguous, lda/ldb % 8 == 0, 16-byte
-// aligned) with the epilogue policy EPI (its Args carry everything beyond C's tile).
+// aligned; BMN: B stored [K, N]) with the epilogue policy EPI (its Args carry everything
+// beyond C's tile; EPI::BIG_OK: it takes 256x256 tiles too).
 template <class EPI, typename TC, bool BMN = false>
 inline int launch_dense_epi(const GemmArgs& a, const typename EPI::Args& ea, hipStream_t s, const char* what) {
   if (a.M * a.lda * 2 > 0x7FFFFFFF || !(BMN ? dtl_fits_mn(a.K, a.ldb) : a.N * a.ldb * 2 <= 0x7FFFFFFF))
     return fail(PD_EUNSUPPORTED, std::string(what) + ": operands of 2 GiB or more");
   if ((a.M + CfgDtl::BM - 1) / CfgDtl::BM > 65535 || (a.N + CfgDtl::BN - 1) / CfgDtl::BN > 65535)
     return fail(PD_EUNSUPPORTED, std::string(what) + ": too large");
-  const dim3 grid((unsigned)((a.N + CfgDtl::BN - 1) / CfgDtl::BN), (unsigned)((a.M + CfgDtl::BM - 1) / CfgDtl::BM));
-  if (a.K % CfgDtl::BK)
-    hipLaunchKernelGGL((k_gemm_dtl<CfgDtl, TC, MODE_DENSE, true, EPI, false, BMN>), grid, dim3(CfgDtl::NT), 0, s,
-                       a, ea);
-  else
-    hipLaunchKernelGGL((k_gemm_dtl<CfgDtl, TC, MODE_DENSE, false, EPI, false, BMN>), grid, dim3(CfgDtl::NT), 0, s,
-                       a, ea);
+  if (EPI::BIG_OK && big_tiles(a.M, a.N)) launch_epi_cfg<CfgDtlBig, EPI, TC, BMN>(a, ea, s);
+  else if (!BMN && deep_ring(a.M, a.N, a.K)) launch_epi_cfg<CfgDtlDeep, EPI, TC, BMN>(a, ea, s);
+  else launch_epi_cfg<CfgDtl, EPI, TC, BMN>(a, ea, s);
   return check_launch(what);
 }
 
@@ -1093,6 +1124,8 @@ inline int launch_kcat_epi(const GemmArgs& a, const KcatArgs& q, const typename 
     return fail(PD_EUNSUPPORTED, std::string(what) + ": too large");
   if (big_tiles(a.M, a.N) && EPI::LDS_BYTES <= 2 * CfgDtlBig::STAGE_BYTES)
     launch_kcat_cfg<CfgDtlBig, EPI, TC, B1MN, B2MN>(a, q, ea, s);
+  else if (!B1MN && !B2MN && deep_ring(a.M, a.N, a.K + q.K1))
+    launch_kcat_cfg<CfgDtlDeep, EPI, TC, B1MN, B2MN>(a, q, ea, s);
   else
     launch_kcat_cfg<CfgDtl, EPI, TC, B1MN, B2MN>(a, q, ea, s);
   return check_launch(what);

@@ -149,6 +149,7 @@ __device__ inline void epi_groups(const GemmArgs& p, const TileJob& t, int wm, i
 // C = xV (bf16); acts = routed ? xV * (m - d) : 0
 struct EpiActs {
   static constexpr int LDS_BYTES = 0;
+  static constexpr bool BIG_OK = false;
   struct Args {
     const bf16_t* mask;
     const bf16_t* delta;
@@ -177,6 +178,7 @@ struct EpiActs {
 // da = g @ U^T rounded; dmask = routed ? da * xV : 0 (if wanted); C = dxV = routed ? da * (m - d) : 0
 struct EpiMaskedBwd {
   static constexpr int LDS_BYTES = 0;
+  static constexpr bool BIG_OK = false;
   struct Args {
     const bf16_t* xV;
     const bf16_t* mask;
