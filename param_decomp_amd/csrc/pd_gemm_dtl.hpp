@@ -260,8 +260,8 @@ __device__ inline bool map_tile(const GemmArgs& p, int lane, TileJob& t) {
   return t.m0 < t.M && t.n0 < p.N;
 }
 
-// SPLIT: the loads of a stage go out in two halves; NS: LDS stages, a power of two (see the
-// top of this file).
+// SPLIT: the loads of a stage go out in two halves; NS: LDS stages (see the top of this
+// file).
 template <int BM_, int BN_, int WM_, int WN_, bool SPLIT_, int NS_ = 2>
 struct DtlCfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, BK = 64;
@@ -277,7 +277,8 @@ struct DtlCfg {
   static_assert(NW % 2 == 0, "the swizzle parity of a wave's rows must not depend on the load index");
   static_assert(BM_ % (RPI * NW) == 0 && BN_ % (RPI * NW) == 0, "every wave moves whole 1 KB row blocks");
   static_assert(TM >= 1 && TN >= 1 && WTM % 32 == 0 && WTN % 32 == 0, "wave tile is a multiple of 32x32");
-  static_assert((NS & (NS - 1)) == 0 && NS * STAGE_BYTES <= 160 * 1024, "LDS");
+  static_assert(NS >= 2 && NS * STAGE_BYTES <= 160 * 1024, "LDS");
+  static __device__ __host__ int ring(int64_t kt) { return (int)((uint32_t)kt % (uint32_t)NS); }  // stage kt's space
   static_assert(NS == 2 || !SPLIT_, "split loads are written for two stages");
   // loads in flight that a stage's readers need not wait for: those of the later stages
   static constexpr int AHEAD = (NS - 2) * INSTS;
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
     constexpr int LO = decltype(h)::value ? CFG::HALF : 0, HI = decltype(h)::value ? CFG::INSTS : CFG::HALF;
     const uint32_t kpos = (uint32_t)(kbeg + kt * BK);
     const bool in = kt < nk;
-    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES, abase, uni(in ? abytes : 0), offa,
+    dtl_issue_ab<CFG, LO, HI>(smem + CFG::ring(kt) * CFG::STAGE_BYTES, abase, uni(in ? abytes : 0), offa,
                               kpos * kstep_a, bbase, uni(in ? bbytes : 0), offb, kpos * kstep_b, wave);
   };
 #pragma unroll
@@ -804,8 +805,8 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
   read_frags<CFG>(smem, fo, lane, 0, f[0]);
   constexpr int READS = TM * (AMN ? 2 : 1) + TN * (BMN ? 2 : 1);
   auto stage = [&](int64_t kt, auto edge) {
-    const char* st = smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES;
-    const char* nx = smem + (int)((kt + 1) & (CFG::NS - 1)) * CFG::STAGE_BYTES;
+    const char* st = smem + CFG::ring(kt) * CFG::STAGE_BYTES;
+    const char* nx = smem + CFG::ring(kt + 1) * CFG::STAGE_BYTES;
     pipe_stage<TM * TN, READS, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD>(
         f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
         [&](Frags<CFG>& g) { read_frags<CFG>(nx, fo, lane, 0, g); },
@@ -828,25 +829,28 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
 
 // Two products of one shape in one block, P1 = A @ B^T and P2 = A2 @ B2^T (dense, every
 // operand K-contiguous with the same lda / ldb), for epilogues that need both tiles of the
-// same (row, column) block at once. A stage holds A | B | A2 | B2 (SHARED_B: the caller
-// guarantees B2 == B, and a stage has no B2 region). EPI::run(p, ea, tile, wm, wn, tid, acc1, acc2, smem).
+// same (row, column) block at once. EPI::run(p, ea, tile, wm, wn, tid, acc1, acc2, smem).
+// SHARED_B (the caller guarantees B2 == B): one k loop, a stage holding A | B | A2, so B's
+// rows and fragments are read once for both. Otherwise one k loop after the other through
+// the same ring of A | B stages: both products side by side would need 128x128 tiles for
+// their stages to fit (2048 x 16759 x 768 twice with the KL epilogue: 186 against 150 us;
+// with two stages instead of three 167).
 template <class CFG, bool KEDGE, class EPI, bool SHARED_B = false>
 __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename EPI::Args ea) {
   constexpr int BM = CFG::BM, BN = CFG::BN, TM = CFG::TM, TN = CFG::TN, NW = CFG::NW;
   constexpr int BK = CFG::BK, ROWB = CFG::ROWB;
-  constexpr int SB = (SHARED_B ? 2 * BM + BN : 2 * (BM + BN)) * ROWB;
-  constexpr int LDS = 2 * SB > EPI::LDS_BYTES ? 2 * SB : EPI::LDS_BYTES;
-  static_assert(2 * SB <= 160 * 1024, "LDS");
+  static_assert(CFG::HALF == CFG::INSTS && (!SHARED_B || CFG::NS == 2), "loads in one go; two stages of A | B | A2");
+  constexpr int SB = (SHARED_B ? 2 * BM + BN : BM + BN) * ROWB, NS = CFG::NS;
+  constexpr int LDS = NS * SB > EPI::template lds_bytes<CFG>() ? NS * SB : EPI::template lds_bytes<CFG>();
+  static_assert(LDS <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(1024))) char smem[LDS];
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
   const int wm = wave / CFG::WN, wn = wave % CFG::WN;
 
   TileJob t;
   if (!map_tile<BM, BN, MODE_DENSE, float>(p, lane, t)) return;
-  const int64_t m0 = uni64(t.m0), n0 = uni64(t.n0);
-  const int64_t kmin = uni64(t.kbeg), kend = uni64(t.kend);
-  const int64_t kbeg = kmin & ~(int64_t)63;
-  const int64_t nk = kend > kmin ? (kend - kbeg + BK - 1) / BK : 0;
+  const int64_t m0 = uni64(t.m0), n0 = uni64(t.n0), K = p.K;
+  const int64_t nk = (K + BK - 1) / BK;
   const bf16_t* abase = (const bf16_t*)uni64((int64_t)(p.A + m0 * p.lda));
   const bf16_t* a2base = (const bf16_t*)uni64((int64_t)(p.A2 + m0 * p.lda));
   const bf16_t* bbase = (const bf16_t*)uni64((int64_t)(p.B + n0 * p.ldb));
@@ -862,75 +866,85 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = acc2[i][j][v] = 0.f;
+  const FragOffs<CFG, false, false> fo(wm, wn, lane);
 
-  // half 0: A and B (without SPLIT every load), half 1: A2 (and B2), of stage kt (none past
-  // the last stage)
-  constexpr bool SPLIT = CFG::HALF < CFG::INSTS;
-  constexpr int LOADS1 = SHARED_B ? CFG::A_INSTS : CFG::INSTS;
-  auto issue = [&](int64_t kt, auto h) {
-    char* st = smem + (int)(kt & 1) * SB;
-    const uint32_t koff = (uint32_t)((kbeg + kt * BK) * 2);
-    const int32_t ab = uni(kt < nk ? abytes : 0), bb = uni(kt < nk ? bbytes : 0);
-    if (decltype(h)::value == 0) {
+  if constexpr (SHARED_B) {
+    auto issue = [&](int64_t kt, auto h) {  // none past the last stage
+      if (decltype(h)::value) return;
+      char* st = smem + (int)(kt & 1) * SB;
+      const uint32_t koff = (uint32_t)(kt * BK * 2);
+      const int32_t ab = uni(kt < nk ? abytes : 0), bb = uni(kt < nk ? bbytes : 0);
       dtl_issue<NW, 0, CFG::A_INSTS>(st, abase, ab, offa, koff, wave);
       dtl_issue<NW, 0, CFG::B_INSTS>(st + BM * ROWB, bbase, bb, offb, koff, wave);
-    }
-    if (decltype(h)::value == SPLIT) {
       dtl_issue<NW, 0, CFG::A_INSTS>(st + (BM + BN) * ROWB, a2base, ab, offa, koff, wave);
-      if (!SHARED_B) dtl_issue<NW, 0, CFG::B_INSTS>(st + (2 * BM + BN) * ROWB, b2base, bb, offb, koff, wave);
-    }
-  };
-  issue(0, std::integral_constant<int, 0>{});
-  issue(0, std::integral_constant<int, 1>{});
-  issue(1, std::integral_constant<int, 0>{});
-
-  const FragOffs<CFG, false, false> fo(wm, wn, lane);
-  struct F2 {
-    Frags<CFG> x;
-    bf16x8 a2[TM], b2[SHARED_B ? 1 : TN];
-  } f[2];
-  // the second problem's A (and B) sit after the first's
-  auto read = [&](const char* st, int kk, F2& g) {
-    read_frags<CFG>(st, fo, lane, kk, g.x);
-    const int coff = ((2 * kk + (lane >> 5)) ^ fo.sw) << 4;
+    };
+    constexpr int LOADS = 2 * CFG::A_INSTS + CFG::B_INSTS;
+    struct F2 {
+      Frags<CFG> x;
+      bf16x8 a2[TM];
+    } f[2];
+    auto read = [&](const char* st, int kk, F2& g) {
+      read_frags<CFG>(st, fo, lane, kk, g.x);
+      const int coff = ((2 * kk + (lane >> 5)) ^ fo.sw) << 4;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) g.a2[i] = frag_load<false, BM>(st, fo.a[i] + (BM + BN) * ROWB, kk, coff);
-    if constexpr (!SHARED_B) {
+      for (int i = 0; i < TM; ++i) g.a2[i] = frag_load<false, BM>(st, fo.a[i] + (BM + BN) * ROWB, kk, coff);
+    };
+    issue(0, std::integral_constant<int, 0>{});
+    issue(1, std::integral_constant<int, 0>{});
+    wait_vmcnt<LOADS>();
+    lds_barrier();
+    read(smem, 0, f[0]);
+    auto stage = [&](int64_t kt, auto edge) {
+      const char* st = smem + (int)(kt & 1) * SB;
+      const char* nx = smem + (int)(~kt & 1) * SB;
+      pipe_stage<2 * TM * TN, 2 * TM + TN, 0, LOADS, 2, 0>(
+          f, [&](int kk, F2& g) { read(st, kk, g); }, [&](F2& g) { read(nx, 0, g); },
+          [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
+          [&](int kk, F2& g) {
+            if (decltype(edge)::value) {
+              const int64_t kf = kt * BK + kk * 16;
+              mask_frags<CFG>(g.x, lane, kf, 0, K);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) g.b2[j] = frag_load<false, BN>(st, fo.b[j] + (BM + BN) * ROWB, kk, coff);
-    }
-  };
-  wait_vmcnt<CFG::INSTS + (SPLIT ? 0 : LOADS1)>();
-  lds_barrier();
-  read(smem, 0, f[0]);
-  auto stage = [&](int64_t kt, auto edge) {
-    const char* st = smem + (int)(kt & 1) * SB;
-    const char* nx = smem + (int)(~kt & 1) * SB;
-    pipe_stage<2 * TM * TN, 2 * TM + (SHARED_B ? 1 : 2) * TN, (SPLIT ? LOADS1 : 0), CFG::INSTS + (SPLIT ? 0 : LOADS1), 2, 0>(
-        f, [&](int kk, F2& g) { read(st, kk, g); }, [&](F2& g) { read(nx, 0, g); },
-        [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
-        [&](int kk, F2& g) {
-          if (decltype(edge)::value) {
-            const int64_t kf = kbeg + kt * BK + kk * 16;
-            mask_frags<CFG>(g.x, lane, kf, kmin, kend);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) mask_frag(g.a2[i], kf + (lane >> 5) * 8, kmin, kend);
-            if constexpr (!SHARED_B) {
-#pragma unroll
-              for (int j = 0; j < TN; ++j) mask_frag(g.b2[j], kf + (lane >> 5) * 8, kmin, kend);
+              for (int i = 0; i < TM; ++i) mask_frag(g.a2[i], kf + (lane >> 5) * 8, 0, K);
             }
-          }
-          dtl_mfma<CFG>(g.x.a, g.x.b, acc);
-          if constexpr (SHARED_B) dtl_mfma<CFG>(g.a2, g.x.b, acc2);
-          else dtl_mfma<CFG>(g.a2, g.b2, acc2);
-        });
-  };
-  if constexpr (KEDGE) {
-    if (nk > 0) stage(0, std::true_type{});
-    for (int64_t kt = 1; kt < nk - 1; ++kt) stage(kt, std::false_type{});
-    if (nk > 1) stage(nk - 1, std::true_type{});
+            dtl_mfma<CFG>(g.x.a, g.x.b, acc);
+            dtl_mfma<CFG>(g.a2, g.x.b, acc2);
+          });
+    };
+    for (int64_t kt = 0; kt < nk - KEDGE; ++kt) stage(kt, std::false_type{});
+    if constexpr (KEDGE) stage(nk - 1, std::true_type{});
   } else {
-    for (int64_t kt = 0; kt < nk; ++kt) stage(kt, std::false_type{});
+    auto issue = [&](int64_t kt, auto h) {  // stages nk .. 2 nk - 1 are the second product's
+      if (decltype(h)::value) return;
+      const bool s1 = kt < nk, in = kt < 2 * nk;
+      const uint32_t koff = (uint32_t)((s1 ? kt : kt - nk) * BK * 2);
+      dtl_issue_ab<CFG, 0, CFG::INSTS>(smem + CFG::ring(kt) * SB,
+                                       (const bf16_t*)uni64((int64_t)(s1 ? abase : a2base)), uni(in ? abytes : 0), offa,
+                                       koff, (const bf16_t*)uni64((int64_t)(s1 ? bbase : b2base)),
+                                       uni(in ? bbytes : 0), offb, koff, wave);
+    };
+    Frags<CFG> f[2];
+#pragma unroll
+    for (int st = 0; st < NS; ++st) issue(st, std::integral_constant<int, 0>{});
+    wait_vmcnt<CFG::AHEAD + CFG::INSTS>();
+    lds_barrier();
+    read_frags<CFG>(smem, fo, lane, 0, f[0]);
+    auto stage = [&](int64_t kt, int64_t k0, auto edge, f32x16 (&ac)[TM][TN]) {
+      const char* st = smem + CFG::ring(kt) * SB;
+      const char* nx = smem + CFG::ring(kt + 1) * SB;
+      pipe_stage<TM * TN, TM + TN, 0, CFG::INSTS, NS, CFG::AHEAD>(
+          f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
+          [&](Frags<CFG>& g) { read_frags<CFG>(nx, fo, lane, 0, g); },
+          [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
+          [&](int kk, Frags<CFG>& g) {
+            if (decltype(edge)::value) mask_frags<CFG>(g, lane, k0 + kk * 16, 0, K);
+            dtl_mfma<CFG>(g.a, g.b, ac);
+          });
+    };
+    for (int64_t kt = 0; kt < nk - KEDGE; ++kt) stage(kt, 0, std::false_type{}, acc);
+    if constexpr (KEDGE) stage(nk - 1, (nk - 1) * BK, std::true_type{}, acc);
+    for (int64_t kt = nk; kt < 2 * nk - KEDGE; ++kt) stage(kt, 0, std::false_type{}, acc2);
+    if constexpr (KEDGE) stage(2 * nk - 1, (nk - 1) * BK, std::true_type{}, acc2);
   }
   wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG>(p, ea, t, wm, wn, tid, acc, acc2, smem);
@@ -1022,7 +1036,7 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
     const uint32_t kpos = (uint32_t)((s1 ? kt : kt - nk1) * BK);
     const LaneOff oa{s1 ? oa1.off : oa2.off, s1 ? oa1.step : oa2.step};
     const LaneOff ob{s1 ? ob1.off : ob2.off, s1 ? ob1.step : ob2.step};
-    dtl_issue_ab<CFG, LO, HI>(smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES, (const bf16_t*)uni64((int64_t)(s1 ? a1 : a2)),
+    dtl_issue_ab<CFG, LO, HI>(smem + CFG::ring(kt) * CFG::STAGE_BYTES, (const bf16_t*)uni64((int64_t)(s1 ? a1 : a2)),
                               uni(in ? (s1 ? a1bytes : a2bytes) : 0), oa, kpos * 2,
                               (const bf16_t*)uni64((int64_t)(s1 ? b1 : b2)),
                               uni(in ? (s1 ? b1bytes : b2bytes) : 0), ob, kpos * (s1 ? ks1 : ks2), wave);
@@ -1043,8 +1057,8 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
   // stage kt of a segment whose fragments sit at fo, the next stage's at fon; its k range
   // starts at k0 and ends at kend
   auto stage = [&](int64_t kt, const auto& fo, const auto& fon, int64_t k0, int64_t kend, auto edge, auto reads) {
-    const char* st = smem + (int)(kt & (CFG::NS - 1)) * CFG::STAGE_BYTES;
-    const char* nx = smem + (int)((kt + 1) & (CFG::NS - 1)) * CFG::STAGE_BYTES;
+    const char* st = smem + CFG::ring(kt) * CFG::STAGE_BYTES;
+    const char* nx = smem + CFG::ring(kt + 1) * CFG::STAGE_BYTES;
     pipe_stage<TM * TN, decltype(reads)::value, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD>(
         f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
         [&](Frags<CFG>& g) { read_frags<CFG>(nx, fon, lane, 0, g); },

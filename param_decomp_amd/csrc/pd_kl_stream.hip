@@ -187,9 +187,10 @@ __device__ inline float kl_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44
 
 // Forward epilogue: the tile's partial (m_p, s_p, a, m_q, s_q) of each position over the
 // tile's vocab columns, to part[(row * n_tiles + tile) * 5]. Rows are summed across the
-// lane pair (lane, lane ^ 32) and the two waves of a row in a fixed order.
+// lane pair (lane, lane ^ 32) and the waves of a row in a fixed order.
 struct EpiKLStats {
-  static constexpr int LDS_BYTES = 0;
+  template <class CFG>
+  static constexpr int lds_bytes() { return CFG::WN * CFG::BM * 3 * 4; }
   struct Args {
     float* part;
     int64_t n_tiles, tile_base;
@@ -197,77 +198,106 @@ struct EpiKLStats {
   template <class CFG>
   __device__ static void run(const GemmArgs& p, const Args& a, const TileJob& t, int wm, int wn, int tid,
                              f32x16 (&zp)[CFG::TM][CFG::TN], f32x16 (&zq)[CFG::TM][CFG::TN], char* smem) {
-    static_assert(CFG::TM == 1 && CFG::WN == 2 && CFG::WTM == 32, "one 32-row MFMA tile per wave, two waves across N");
-    const int lane = tid & 63;
-    float mp = -INFINITY, mq = -INFINITY;
+    // a tile with no column past N (all but a chunk's last) skips the column tests
+    if (t.n0 + CFG::BN <= p.N) run_t<CFG, true>(p, a, t, wm, wn, tid, zp, zq, smem);
+    else run_t<CFG, false>(p, a, t, wm, wn, tid, zp, zq, smem);
+  }
+  template <class CFG, bool FULL>
+  __device__ static void run_t(const GemmArgs& p, const Args& a, const TileJob& t, int wm, int wn, int tid,
+                               f32x16 (&zp)[CFG::TM][CFG::TN], f32x16 (&zq)[CFG::TM][CFG::TN], char* smem) {
+    const int lane = tid & 63, rl = lane & 31;
+    float* red = (float*)smem;  // [WN][BM][3]
+    auto slot = [&](int w, int i) { return red + (w * CFG::BM + wm * CFG::WTM + i * 32 + rl) * 3; };
+    lds_write_barrier();  // the k loop's stage buffers are free
 #pragma unroll
-    for (int j = 0; j < CFG::TN; ++j)
+    for (int i = 0; i < CFG::TM; ++i) {
+      float mp = -INFINITY, mq = -INFINITY;
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
+      for (int j = 0; j < CFG::TN; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * g + 4 * (lane >> 5) + e;
-          if (col < p.N) {
-            mp = fmaxf(mp, zp[0][j][4 * g + e]);
-            mq = fmaxf(mq, zq[0][j][4 * g + e]);
+        for (int v = 0; v < 16; ++v) {
+          const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+          if (FULL || col < p.N) {
+            mp = fmaxf(mp, zp[i][j][v]);
+            mq = fmaxf(mq, zq[i][j][v]);
           }
         }
-    mp = fmaxf(mp, __shfl_xor(mp, 32, 64));
-    mq = fmaxf(mq, __shfl_xor(mq, 32, 64));
-    float* red = (float*)smem;  // [WM][2][32][3]
-    lds_write_barrier();        // the k loop's stage buffers are free
-    if (lane < 32) {
-      red[((wm * 2 + wn) * 32 + lane) * 3 + 0] = mp;
-      red[((wm * 2 + wn) * 32 + lane) * 3 + 1] = mq;
+      mp = fmaxf(mp, __shfl_xor(mp, 32, 64));
+      mq = fmaxf(mq, __shfl_xor(mq, 32, 64));
+      if (lane < 32) {
+        slot(wn, i)[0] = mp;
+        slot(wn, i)[1] = mq;
+      }
     }
     lds_write_barrier();
-    const int rl = lane & 31;
-    mp = fmaxf(red[((wm * 2) * 32 + rl) * 3 + 0], red[((wm * 2 + 1) * 32 + rl) * 3 + 0]);
-    mq = fmaxf(red[((wm * 2) * 32 + rl) * 3 + 1], red[((wm * 2 + 1) * 32 + rl) * 3 + 1]);
-    float sp = 0.f, sa = 0.f, sq = 0.f;
+    float mp[CFG::TM], mq[CFG::TM];
 #pragma unroll
-    for (int j = 0; j < CFG::TN; ++j)
+    for (int i = 0; i < CFG::TM; ++i) {
+      mp[i] = mq[i] = -INFINITY;
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
+      for (int w = 0; w < CFG::WN; ++w) {
+        mp[i] = fmaxf(mp[i], slot(w, i)[0]);
+        mq[i] = fmaxf(mq[i], slot(w, i)[1]);
+      }
+    }
+    lds_write_barrier();
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * g + 4 * (lane >> 5) + e;
-          if (col < p.N) {
-            const float x = zp[0][j][4 * g + e], y = zq[0][j][4 * g + e];
-            const float ex = kl_exp(x - mp);
+    for (int i = 0; i < CFG::TM; ++i) {
+      float sp = 0.f, sa = 0.f, sq = 0.f;
+#pragma unroll
+      for (int j = 0; j < CFG::TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+          if (FULL || col < p.N) {
+            const float x = zp[i][j][v], y = zq[i][j][v];
+            const float ex = kl_exp(x - mp[i]);
             sp += ex;
             sa = fmaf(ex, x - y, sa);
-            sq += kl_exp(y - mq);
+            sq += kl_exp(y - mq[i]);
           }
         }
-    sp += __shfl_xor(sp, 32, 64);
-    sa += __shfl_xor(sa, 32, 64);
-    sq += __shfl_xor(sq, 32, 64);
-    lds_write_barrier();
-    if (lane < 32) {
-      red[((wm * 2 + wn) * 32 + lane) * 3 + 0] = sp;
-      red[((wm * 2 + wn) * 32 + lane) * 3 + 1] = sa;
-      red[((wm * 2 + wn) * 32 + lane) * 3 + 2] = sq;
+      sp += __shfl_xor(sp, 32, 64);
+      sa += __shfl_xor(sa, 32, 64);
+      sq += __shfl_xor(sq, 32, 64);
+      if (lane < 32) {
+        float* r = slot(wn, i);
+        r[0] = sp;
+        r[1] = sa;
+        r[2] = sq;
+      }
     }
     lds_write_barrier();
-    const int64_t row = t.m0 + wm * 32 + rl;
-    if (wn == 0 && lane < 32 && row < t.M) {
-      const float* r0 = red + ((wm * 2) * 32 + rl) * 3;
-      const float* r1 = red + ((wm * 2 + 1) * 32 + rl) * 3;
-      float* dst = a.part + (row * a.n_tiles + a.tile_base + t.n0 / CFG::BN) * 5;
-      dst[0] = mp;
-      dst[1] = r0[0] + r1[0];
-      dst[2] = r0[1] + r1[1];
-      dst[3] = mq;
-      dst[4] = r0[2] + r1[2];
+    if (wn == 0 && lane < 32) {
+#pragma unroll
+      for (int i = 0; i < CFG::TM; ++i) {
+        const int64_t row = t.m0 + wm * CFG::WTM + i * 32 + rl;
+        if (row >= t.M) continue;
+        float o[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < CFG::WN; ++w)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) o[k] = w ? o[k] + slot(w, i)[k] : slot(w, i)[k];
+        float* dst = a.part + (row * a.n_tiles + a.tile_base + t.n0 / CFG::BN) * 5;
+        dst[0] = mp[i];
+        dst[1] = o[0];
+        dst[2] = o[1];
+        dst[3] = mq[i];
+        dst[4] = o[2];
+      }
     }
   }
 };
 
 // Backward epilogue: G[row, col] = (e^{z_q - logZ_q} - e^{z_p - logZ_p}) g[row] in bf16 for
-// col < width, zero for width <= col < kpad (the contraction padding).
+// col < width, zero for width <= col < kpad (the contraction padding; kpad and ldg are
+// multiples of 8). The tile goes through a row-major LDS image, so G's lines are written
+// whole.
 struct EpiKLGrad {
-  static constexpr int LDS_BYTES = 0;
+  template <class CFG>
+  static constexpr int rsb() { return CFG::BN * 2 + 16; }  // LDS bytes per image row
+  template <class CFG>
+  static constexpr int lds_bytes() { return CFG::BM * rsb<CFG>(); }
   struct Args {
     const float* stats;
     const float* g;
@@ -276,26 +306,44 @@ struct EpiKLGrad {
   };
   template <class CFG>
   __device__ static void run(const GemmArgs& p, const Args& a, const TileJob& t, int wm, int wn, int tid,
-                             f32x16 (&zp)[CFG::TM][CFG::TN], f32x16 (&zq)[CFG::TM][CFG::TN], char*) {
-    static_assert(CFG::TM == 1 && CFG::WTM == 32, "one 32-row MFMA tile per wave");
+                             f32x16 (&zp)[CFG::TM][CFG::TN], f32x16 (&zq)[CFG::TM][CFG::TN], char* smem) {
+    if (t.n0 + CFG::BN <= a.width) run_t<CFG, true>(p, a, t, wm, wn, tid, zp, zq, smem);
+    else run_t<CFG, false>(p, a, t, wm, wn, tid, zp, zq, smem);
+  }
+  template <class CFG, bool FULL>
+  __device__ static void run_t(const GemmArgs& p, const Args& a, const TileJob& t, int wm, int wn, int tid,
+                               f32x16 (&zp)[CFG::TM][CFG::TN], f32x16 (&zq)[CFG::TM][CFG::TN], char* smem) {
     const int lane = tid & 63;
-    const int64_t row = t.m0 + wm * 32 + (lane & 31);
-    if (row >= t.M) return;
-    const float* st = a.stats + row * 5;
-    const float lzp = st[0] + logf(st[1]), lzq = st[3] + logf(st[4]);
-    const float gn = a.g[row];
+    lds_write_barrier();  // the k loop's stage buffers are free
 #pragma unroll
-    for (int j = 0; j < CFG::TN; ++j)
+    for (int i = 0; i < CFG::TM; ++i) {
+      const int rl = wm * CFG::WTM + i * 32 + (lane & 31);
+      const int64_t row = t.m0 + rl;
+      const float* st = a.stats + (row < t.M ? row : t.m0) * 5;
+      const float lzp = st[0] + logf(st[1]), lzq = st[3] + logf(st[4]);
+      const float gn = a.g[row < t.M ? row : t.m0];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int64_t col = t.n0 + wn * CFG::WTN + j * 32 + 8 * g + 4 * (lane >> 5);
-        if (col >= a.kpad) continue;
-        float v[4];
+      for (int j = 0; j < CFG::TN; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          v[e] = col + e < a.width ? (kl_exp(zq[0][j][4 * g + e] - lzq) - kl_exp(zp[0][j][4 * g + e] - lzp)) * gn : 0.f;
-        *(uint2*)(a.G + row * a.ldg + col) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-      }
+        for (int g = 0; g < 4; ++g) {
+          const int c = wn * CFG::WTN + j * 32 + 8 * g + 4 * (lane >> 5);
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[e] = FULL || t.n0 + c + e < a.width
+                       ? (kl_exp(zq[i][j][4 * g + e] - lzq) - kl_exp(zp[i][j][4 * g + e] - lzp)) * gn
+                       : 0.f;
+          *(uint2*)(smem + rl * rsb<CFG>() + c * 2) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        }
+    }
+    lds_write_barrier();
+    constexpr int CPR = CFG::BN / 8, RPP = CFG::NT / CPR;
+    static_assert(CFG::NT % CPR == 0 && CFG::BM % RPP == 0, "store passes");
+    const int cc = tid % CPR;
+    const int64_t col = t.n0 + cc * 8;
+    for (int r = tid / CPR; r < CFG::BM; r += RPP)
+      if (t.m0 + r < t.M && col < a.kpad)
+        *(uint4*)(a.G + (t.m0 + r) * a.ldg + col) = *(const uint4*)(smem + r * rsb<CFG>() + cc * 16);
   }
 };
 
@@ -340,6 +388,16 @@ __global__ __launch_bounds__(256) void k_kl_transpose(const bf16_t* __restrict__
   }
 }
 
+// Tiles of the fused passes: 128 positions x 256 vocab columns, 8 waves of 64x64. With one
+// head for both sides (a tied head, as in the LM step) a stage holds A | B | A2 and both
+// products share the head's fragments; two heads take one k loop after the other.
+typedef DtlCfg<128, 256, 2, 4, false> CfgKL;
+typedef DtlCfg<128, 256, 2, 4, false, 3> CfgKLTwo;
+static int64_t kl_tiles(const KLChunks& K, int64_t V, int bn) {
+  int64_t n = 0;
+  for (int64_t c = 0; c < K.nc; ++c) n += cdiv(K.width(c, V), bn);
+  return n;
+}
 struct KLFused {
   float* part;  // [N, n_tiles, 5]
   bf16_t* G;    // [N, cw]
@@ -374,8 +432,7 @@ static KLFused kl_fused_plan(int64_t N, int64_t d, int64_t V, int n_chunks, char
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const KLChunks K = kl_chunks(PD_DTYPE_BF16, V, n_chunks);
   KLFused P;
-  P.n_tiles = 0;
-  for (int64_t c = 0; c < K.nc; ++c) P.n_tiles += cdiv(K.width(c, V), CfgDtl::BN);
+  P.n_tiles = kl_tiles(K, V, CfgKL::BN);
   P.Vp = (V + 7) & ~(int64_t)7;
   size_t off = 0;
   P.part = (float*)(base + off);
@@ -394,20 +451,18 @@ static KLFused kl_fused_plan(int64_t N, int64_t d, int64_t V, int n_chunks, char
   return P;
 }
 
-// Tiles of the fused passes: with one head for both sides (a tied head, as in the LM
-// step) 128 positions x 256 vocab columns, whose stage (A | B | A2, 64 KB) carries half
-// the operand bytes per MFMA of the 128 x 128 tile; with two heads 128 x 128.
-typedef DtlCfg<128, 256, 4, 2, false> CfgKLWide;
-static int64_t kl_tiles(const KLChunks& K, int64_t V, int bn) {
-  int64_t n = 0;
-  for (int64_t c = 0; c < K.nc; ++c) n += cdiv(K.width(c, V), bn);
-  return n;
-}
-template <class CFG, bool SHARED, class EPI>
+template <class EPI>
 static void kl_dual_launch(const GemmArgs& a, const typename EPI::Args& ea, int64_t d, hipStream_t s) {
-  const dim3 grid((unsigned)cdiv(a.N, CFG::BN), (unsigned)cdiv(a.M, CFG::BM));
-  if (d % CFG::BK) hipLaunchKernelGGL((k_gemm_dtl_dual<CFG, true, EPI, SHARED>), grid, dim3(CFG::NT), 0, s, a, ea);
-  else hipLaunchKernelGGL((k_gemm_dtl_dual<CFG, false, EPI, SHARED>), grid, dim3(CFG::NT), 0, s, a, ea);
+  const dim3 grid((unsigned)cdiv(a.N, CfgKL::BN), (unsigned)cdiv(a.M, CfgKL::BM));
+#define PD_L(CFG, KE, SH) hipLaunchKernelGGL((k_gemm_dtl_dual<CFG, KE, EPI, SH>), grid, dim3(CFG::NT), 0, s, a, ea)
+  if (a.B == a.B2) {
+    if (d % CfgKL::BK) PD_L(CfgKL, true, true);
+    else PD_L(CfgKL, false, true);
+  } else {
+    if (d % CfgKL::BK) PD_L(CfgKLTwo, true, false);
+    else PD_L(CfgKLTwo, false, false);
+  }
+#undef PD_L
 }
 
 static int kl_fused_fits(int64_t N, int64_t d, int64_t V) {
@@ -439,9 +494,7 @@ int pd_streamed_kl_fwd(int dtype, int64_t N, int64_t d, int64_t V, int n_chunks,
     if (!workspace || workspace_bytes < kl_fused_plan(N, d, V, n_chunks, nullptr).total)
       return fail(PD_EWORKSPACE, "pd_streamed_kl_fwd: workspace too small");
     const KLFused F = kl_fused_plan(N, d, V, n_chunks, (char*)workspace);
-    const bool shared = head_masked == head_clean;
-    const int bn = shared ? CfgKLWide::BN : CfgDtl::BN;
-    const int64_t n_tiles = kl_tiles(K, V, bn);  // <= F.n_tiles (the plan counts 128-wide tiles)
+    const int64_t n_tiles = kl_tiles(K, V, CfgKL::BN);
     int64_t tile_base = 0;
     for (int64_t c = 0; c < K.nc; ++c) {
       const int64_t w = K.width(c, V);
@@ -450,9 +503,8 @@ int pd_streamed_kl_fwd(int dtype, int64_t N, int64_t d, int64_t V, int n_chunks,
       GemmArgs a{N, w, d, (const bf16_t*)act_clean, d, hc, d, nullptr, 0, 1.f, 0.f, nullptr, 0, 0, 0, 0,
                  (const bf16_t*)act_masked, hm, nullptr};
       const EpiKLStats::Args ea{F.part, n_tiles, tile_base};
-      if (shared) kl_dual_launch<CfgKLWide, true, EpiKLStats>(a, ea, d, s);
-      else kl_dual_launch<CfgDtl, false, EpiKLStats>(a, ea, d, s);
-      tile_base += cdiv(w, bn);
+      kl_dual_launch<EpiKLStats>(a, ea, d, s);
+      tile_base += cdiv(w, CfgKL::BN);
     }
     hipLaunchKernelGGL(k_kl_merge, dim3((unsigned)cdiv(N, 4)), dim3(256), 0, s, F.part, N, n_tiles, stats,
                        position_kl);
@@ -501,8 +553,7 @@ int pd_streamed_kl_bwd(int dtype, int64_t N, int64_t d, int64_t V, int n_chunks,
       GemmArgs a{N, w, d, (const bf16_t*)act_clean, d, hc, d, nullptr, 0, 1.f, 0.f, nullptr, 0, 0, 0, 0,
                  (const bf16_t*)act_masked, hm, nullptr};
       const EpiKLGrad::Args ea{stats, g_position, F.G, K.cw, w, kpad};
-      if (head_masked == head_clean) kl_dual_launch<CfgKLWide, true, EpiKLGrad>(a, ea, d, s);
-      else kl_dual_launch<CfgDtl, false, EpiKLGrad>(a, ea, d, s);
+      kl_dual_launch<EpiKLGrad>(a, ea, d, s);
       // d_act (+)= G [N, kpad] @ (head^T [d, c cw + kpad))^T
       if ((rc = gemm_splitk(N, d, kpad, F.G, K.cw, 0, F.hT + c * K.cw, F.Vp, 1, d_act_masked, d, PD_DTYPE_F32,
                             c == 0 ? 0.f : 1.f, F.sk, F.sk_bytes, stream, F.splits)))
