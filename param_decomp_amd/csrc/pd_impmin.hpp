@@ -77,6 +77,21 @@ __device__ inline int row_group(const int32_t* __restrict__ off, int G, int64_t 
   return lo - 1;
 }
 
+// row_group of the 64 sorted rows j0 .. j0 + 63, one per lane of a whole wave: a lane counts
+// the group starts at or below its row from one coalesced load of the offsets, where a
+// search per row is a chain of log2(G) dependent loads.
+__device__ inline int wave_row_groups(const int32_t* __restrict__ off, int G, int64_t j0, int lane) {
+  int g = 0;
+  for (int b = 1; b < G; b += 64) {
+    const bool in = b + lane < G;
+    const int o = in ? off[b + lane] : 0;
+    g += __popcll(__ballot(in && o <= j0));  // starts no row of the tile precedes
+    for (unsigned long long m = __ballot(in && o > j0 && o <= j0 + 63); m; m &= m - 1)
+      g += __builtin_amdgcn_readlane(o, __ffsll(m) - 1) <= j0 + lane ? 1 : 0;
+  }
+  return g;
+}
+
 // LDS of the in-tile column sums: psi of the 64x64 tile and each row's group (-1 = no row).
 struct Sl0Tile {
   float ps[64][65];
@@ -89,25 +104,32 @@ struct NoSl0Tile {};  // the LDS slot of the other imp-min modes
 // every row below n_rows when off is NULL (one group: a dense site).
 __device__ inline void sl0_tile_groups(Sl0Tile& L, const int32_t* off, int G, int64_t j0, int64_t n_rows, int tid) {
   if (tid < 64) {
-    const int64_t j = j0 + tid;
-    L.grp[tid] = j < n_rows ? (off ? row_group(off, G, j) : 0) : -1;
+    const int g = off ? wave_row_groups(off, G, j0, tid) : 0;
+    L.grp[tid] = j0 + tid < n_rows ? g : -1;
   }
 }
 
-// After a barrier that made L.ps / L.grp visible: thread col (< 64) walks the tile's rows
-// in order and writes each group's column sum (rows grouped consecutively).
+// After a barrier that made L.ps / L.grp visible: lane col of the first wave adds the
+// tile's rows in order and writes each group's column sum (rows grouped consecutively, the
+// rows there are first). The runs of equal groups come from one ballot, so a run's rows are
+// read without a test between them, eight in flight.
 __device__ inline void sl0_tile_colsums(const Sl0Tile& L, int64_t tile, int q0, int C, float* __restrict__ colpart,
                                         int tid) {
-  if (tid >= 64 || q0 + tid >= C) return;
-  float acc = 0.f;
-  for (int r = 0; r < 64; ++r) {
-    const int g = L.grp[r];
-    if (g < 0) break;
-    acc += L.ps[r][tid];
-    if (r == 63 || L.grp[r + 1] != g) {
-      colpart[(tile + g) * C + q0 + tid] = acc;
-      acc = 0.f;
+  if (tid >= 64) return;
+  const int g = L.grp[tid], gn = tid < 63 ? L.grp[tid + 1] : -1;
+  int r = 0;
+  for (unsigned long long m = __ballot(g >= 0 && g != gn); m; m &= m - 1) {
+    const int last = __ffsll(m) - 1, grp = __builtin_amdgcn_readlane(g, last);
+    float acc = 0.f;
+    for (; r + 8 <= last + 1; r += 8) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = L.ps[r + i][tid];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc += v[i];
     }
+    for (; r <= last; ++r) acc += L.ps[r][tid];
+    if (q0 + tid < C) colpart[(tile + grp) * C + q0 + tid] = acc;
   }
 }
 
@@ -130,8 +152,18 @@ static __global__ __launch_bounds__(256) void k_sl0_finalize(const float* __rest
     const int g = (int)(i / C), col = (int)(i % C);
     const int64_t lo = off ? off[g] : 0, hi = off ? off[g + 1] : n_rows;
     float F = 0.f;
-    if (hi > lo)
-      for (int64_t t = lo / 64; t <= (hi - 1) / 64; ++t) F += colpart[(t + g) * C + col];
+    if (hi > lo) {
+      const float* q = colpart + (lo / 64 + g) * (int64_t)C + col;
+      int64_t n = (hi - 1) / 64 - lo / 64 + 1;
+      for (; n >= 8; n -= 8, q += 8 * (int64_t)C) {  // eight loads in flight, added in order
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = q[e * (int64_t)C];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) F += v[e];
+      }
+      for (; n > 0; --n, q += C) F += *q;
+    }
     const float f = F * inv_n;
     float sl = coeff;
     if (ref_count > 0.f) {

@@ -244,6 +244,24 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
     if (tid < TILE) srow[tid] = n0 + tid < a.N ? (int)((n0 + tid) / a.rps) : 0;
     __syncthreads();
   }
+  // the four passes' loads go out together
+  uint2 pws[4], hws[4];
+  float dts[4];
+  bool rts[4];
+  uint4 tws[LAYOUT == MASK_SRC ? 4 : 1];
+#pragma unroll
+  for (int pass = 0; pass < 4; ++pass) {
+    const int r = PD_LM_ROW(pass);
+    const int64_t n = n0 + r;
+    if (n < a.N && qok) {
+      const int64_t idx = n * a.C + q0 + q4;
+      pws[pass] = *(const uint2*)(a.ci_pre + idx);
+      hws[pass] = *(const uint2*)(xV + idx);
+      dts[pass] = a.delta ? a.delta[n] : 0.f;
+      rts[pass] = !a.route || a.route[n];
+      if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)srow[r] * a.C + q0 + q4);
+    }
+  }
   float imp = 0.f;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
@@ -252,12 +270,13 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
     bf16_t o[4] = {0, 0, 0, 0};
     if (n < a.N && qok) {
       const int64_t idx = n * a.C + q0 + q4;
-      const float dt = a.delta ? a.delta[n] : 0.f;
-      const bool routed = !a.route || a.route[n];
-      const uint2 pw = *(const uint2*)(a.ci_pre + idx);
-      const uint2 hw = *(const uint2*)(xV + idx);
+      const float dt = dts[pass];
+      const bool routed = rts[pass];
+      const uint2 pw = pws[pass], hw = hws[pass];
       const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
       const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
+      float uv[4];
+      if constexpr (LAYOUT == MASK_SRC) src_quad_values(tws[pass], a.src_dtype, uv);
       uint32_t ub = 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -266,7 +285,7 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
         else imp += powp<PM>(upper_fwd(pre[e]), a.p);
         float u;
         if constexpr (LAYOUT == MASK_SRC) {
-          u = src_value(a.src, a.src_dtype, (int64_t)srow[r] * a.C + q0 + q4 + e);
+          u = uv[e];
         } else {
           const uint32_t kb = (draw_bits(a.k0, a.k1, idx + e, total, 8, LAYOUT) & 0xFFu) >> 1;
           ub |= kb << (8 * e);
@@ -312,63 +331,92 @@ __global__ __launch_bounds__(256) void k_lm_mask_bwd(LMMaskArgs a, const bf16_t*
     if (tid < 64) SG.grp[tid] = n0 + tid < a.N ? (int)((n0 + tid) / a.rps) : -1;  // each row's source row
     __syncthreads();
   }
+  // the loads of two passes go out together (of all four: half the waves, and slower)
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
-    const int r = PD_LM_ROW(pass);
-    const int64_t n = n0 + r;
-    bf16_t o[4] = {0, 0, 0, 0};
-    float dmsum = 0.f;
-    if (n < a.N && qok) {
-      const int64_t idx = n * a.C + q0 + q4;
-      const float dt = a.delta ? a.delta[n] : 0.f;
-      const uint2 pw = *(const uint2*)(a.ci_pre + idx);
-      const uint2 hw = *(const uint2*)(xV + idx);
-      const uint2 dw = (!a.route || a.route[n]) ? *(const uint2*)(d_acts + idx) : make_uint2(0u, 0u);
-      const uint32_t ub = SRC ? 0u : *(const uint32_t*)(ubits + idx);
-      const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
-      const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
-      const float da[4] = {bf_lo(dw.x), bf_hi(dw.x), bf_lo(dw.y), bf_hi(dw.y)};
-      bf16_t dp[4];
-      float slope4[4] = {imp_scale, imp_scale, imp_scale, imp_scale};
-      if constexpr (PM == PM_SL0) {
-        const float4 sl = *(const float4*)(a.slope + q0 + q4);
-        slope4[0] = sl.x;
-        slope4[1] = sl.y;
-        slope4[2] = sl.z;
-        slope4[3] = sl.w;
+  for (int half = 0; half < 4; half += 2) {
+    uint2 pws[4], hws[4], dws[4];
+    uint32_t ubs[4];
+    float dts[4];
+    uint4 tws[SRC ? 4 : 1];
+#pragma unroll
+    for (int pass = half; pass < half + 2; ++pass) {
+      const int r = PD_LM_ROW(pass);
+      const int64_t n = n0 + r;
+      if (n < a.N && qok) {
+        const int64_t idx = n * a.C + q0 + q4;
+        pws[pass] = *(const uint2*)(a.ci_pre + idx);
+        hws[pass] = *(const uint2*)(xV + idx);
+        dws[pass] = (!a.route || a.route[n]) ? *(const uint2*)(d_acts + idx) : make_uint2(0u, 0u);
+        dts[pass] = a.delta ? a.delta[n] : 0.f;
+        ubs[pass] = SRC ? 0u : *(const uint32_t*)(ubits + idx);
+        if constexpr (SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)SG.grp[r] * a.C + q0 + q4);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = lower_fwd(pre[e]), up = upper_fwd(pre[e]);
-        float u;
-        if constexpr (SRC) u = src_value(a.src, a.src_dtype, (int64_t)SG.grp[r] * a.C + q0 + q4 + e);
-        else u = (float)((ub >> (8 * e)) & 0xFFu) * (1.f / 128.f);
-        const float m = lo + (1.f - lo) * u - dt;
-        float dimp;
-        if constexpr (PM == PM_SL0) dimp = slope4[e] * sl0_dpsi(up, a.g2, a.psis);
-        else dimp = imp_scale * dpowp<PM>(up, a.p);
-        const float dm = da[e] * hv[e];
-        dp[e] = f32_to_bf16(lower_vjp(pre[e], dm * (1.f - u)) + upper_vjp(pre[e], dimp));
-        o[e] = f32_to_bf16(da[e] * m);
-        if constexpr (SRC) {
-          dmsum += dm;
-          const float gs = dm * (1.f - lo);
-          if (a.rps == 1) a.dsrc[idx + e] = gs;
-          else SG.ps[r][q4 + e] = gs;
-        }
-      }
-      *(uint2*)(d_pre + idx) = make_uint2(bf_pack(dp[0], dp[1]), bf_pack(dp[2], dp[3]));
-      *(uint2*)(d_xV + n * a.ld + q0 + q4) = make_uint2(bf_pack(o[0], o[1]), bf_pack(o[2], o[3]));
-    } else if constexpr (SRC) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) SG.ps[r][q4 + e] = 0.f;
     }
-    if constexpr (SRC) {  // the 16 lanes of a row add their columns in a fixed tree (all lanes)
-      dmsum += __shfl_xor(dmsum, 1, 64);
-      dmsum += __shfl_xor(dmsum, 2, 64);
-      dmsum += __shfl_xor(dmsum, 4, 64);
-      dmsum += __shfl_xor(dmsum, 8, 64);
-      if (n < a.N && (tid & 15) == 0 && a.rowdm) a.rowdm[n * gridDim.x + blockIdx.x] = dmsum;
+#pragma unroll
+    for (int pass = half; pass < half + 2; ++pass) {
+      const int r = PD_LM_ROW(pass);
+      const int64_t n = n0 + r;
+      bf16_t o[4] = {0, 0, 0, 0};
+      float dmsum = 0.f;
+      if (n < a.N && qok) {
+        const int64_t idx = n * a.C + q0 + q4;
+        const float dt = dts[pass];
+        const uint2 pw = pws[pass], hw = hws[pass], dw = dws[pass];
+        const uint32_t ub = ubs[pass];
+        const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
+        const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
+        const float da[4] = {bf_lo(dw.x), bf_hi(dw.x), bf_lo(dw.y), bf_hi(dw.y)};
+        bf16_t dp[4];
+        float uv[4], gs[4];
+        if constexpr (SRC) src_quad_values(tws[pass], a.src_dtype, uv);
+        float slope4[4] = {imp_scale, imp_scale, imp_scale, imp_scale};
+        if constexpr (PM == PM_SL0) {
+          const float4 sl = *(const float4*)(a.slope + q0 + q4);
+          slope4[0] = sl.x;
+          slope4[1] = sl.y;
+          slope4[2] = sl.z;
+          slope4[3] = sl.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = lower_fwd(pre[e]), up = upper_fwd(pre[e]);
+          float u;
+          if constexpr (SRC) u = uv[e];
+          else u = (float)((ub >> (8 * e)) & 0xFFu) * (1.f / 128.f);
+          const float m = lo + (1.f - lo) * u - dt;
+          float dimp;
+          if constexpr (PM == PM_SL0) dimp = slope4[e] * sl0_dpsi(up, a.g2, a.psis);
+          else dimp = imp_scale * dpowp<PM>(up, a.p);
+          const float dm = da[e] * hv[e];
+          dp[e] = f32_to_bf16(lower_vjp(pre[e], dm * (1.f - u)) + upper_vjp(pre[e], dimp));
+          o[e] = f32_to_bf16(da[e] * m);
+          if constexpr (SRC) {
+            dmsum += dm;
+            gs[e] = dm * (1.f - lo);
+          }
+        }
+        if constexpr (SRC) {
+          if (a.rps == 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a.dsrc[idx + e] = gs[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) SG.ps[r][q4 + e] = gs[e];
+          }
+        }
+        *(uint2*)(d_pre + idx) = make_uint2(bf_pack(dp[0], dp[1]), bf_pack(dp[2], dp[3]));
+        *(uint2*)(d_xV + n * a.ld + q0 + q4) = make_uint2(bf_pack(o[0], o[1]), bf_pack(o[2], o[3]));
+      } else if constexpr (SRC) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) SG.ps[r][q4 + e] = 0.f;
+      }
+      if constexpr (SRC) {  // the 16 lanes of a row add their columns in a fixed tree (all lanes)
+        dmsum += __shfl_xor(dmsum, 1, 64);
+        dmsum += __shfl_xor(dmsum, 2, 64);
+        dmsum += __shfl_xor(dmsum, 4, 64);
+        dmsum += __shfl_xor(dmsum, 8, 64);
+        if (n < a.N && (tid & 15) == 0 && a.rowdm) a.rowdm[n * gridDim.x + blockIdx.x] = dmsum;
+      }
     }
   }
   if constexpr (SRC) {

@@ -291,22 +291,29 @@ struct MaskRow {
   int32_t ej;
   int64_t srow;
 };
+// GROUP: `groups` (when not NULL) receives each row's (expert, source row) group, by which
+// the rows are sorted (-1: no row).
 template <bool GROUP>
-__device__ inline void fill_mask_rows(MaskRow* rows, const SiteMaskArgs& a, int64_t j0, int tid) {
+__device__ inline void fill_mask_rows(MaskRow* rows, const SiteMaskArgs& a, int64_t j0, int tid,
+                                      int* groups = nullptr) {
   if (tid >= TILE) return;
   const int64_t j = j0 + tid;
   MaskRow v{0, 0.f, 0, 0, 0};
+  int grp = -1;
+  if constexpr (GROUP) v.ej = wave_row_groups(a.offsets, a.E, j0, tid);
   if (j < a.J) {
     const int32_t slot = a.sort_idx[j], tok = slot / a.k;
     v.slot = slot;
     v.dt = a.delta ? a.delta[tok] : 0.f;
     v.routed = !a.route || a.route[tok] ? 1 : 0;
     if constexpr (GROUP) {
-      v.ej = row_group(a.offsets, a.E, j);
-      v.srow = ((int64_t)tok / a.rps) * a.E + v.ej;
+      const int64_t srow = (int64_t)tok / a.rps;
+      v.srow = srow * a.E + v.ej;
+      grp = v.ej * (int)a.S + (int)srow;
     }
   }
   rows[tid] = v;
+  if (groups) groups[tid] = grp;
 }
 
 
@@ -334,6 +341,18 @@ __global__ __launch_bounds__(256) void k_mask_fwd_tile(SiteMaskArgs a, const bf1
   if constexpr (PM == PM_SL0) sl0_tile_groups(SLv, a.offsets, a.E, j0, a.J, tid);
   fill_mask_rows<LAYOUT == MASK_SRC>(rows, a, j0, tid);
   __syncthreads();
+  // the four passes' loads go out together
+  uint2 pws[4], hws[4];
+  uint4 tws[LAYOUT == MASK_SRC ? 4 : 1];
+#pragma unroll
+  for (int pass = 0; pass < 4; ++pass) {
+    const int r = PD_TILE4_ROW(pass);
+    if (j0 + r < a.J && qok) {
+      pws[pass] = *(const uint2*)(a.ci_pre + (int64_t)rows[r].slot * a.c + q0 + q4);
+      hws[pass] = *(const uint2*)(h + (j0 + r) * a.c + q0 + q4);
+      if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, rows[r].srow * a.c + q0 + q4);
+    }
+  }
   float imp = 0.f;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
@@ -343,14 +362,14 @@ __global__ __launch_bounds__(256) void k_mask_fwd_tile(SiteMaskArgs a, const bf1
     if (j < a.J && qok) {
       const int64_t idx = j * a.c + q0 + q4;
       const MaskRow row = rows[r];
-      const int32_t slot = row.slot;
-      const int64_t src = (int64_t)slot * a.c + q0 + q4;
+      const int64_t src = (int64_t)row.slot * a.c + q0 + q4;
       const float dt = row.dt;
       const bool routed = row.routed != 0;
-      const uint2 pw = *(const uint2*)(a.ci_pre + src);
-      const uint2 hw = *(const uint2*)(h + idx);
+      const uint2 pw = pws[pass], hw = hws[pass];
       const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
       const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
+      float uv[4];
+      if constexpr (LAYOUT == MASK_SRC) src_quad_values(tws[pass], a.src_dtype, uv);
       uint32_t ub = 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -361,7 +380,7 @@ __global__ __launch_bounds__(256) void k_mask_fwd_tile(SiteMaskArgs a, const bf1
         if constexpr (LAYOUT == MASK_CONST) {
           u = a.uconst;
         } else if constexpr (LAYOUT == MASK_SRC) {
-          u = src_value(a.src, a.src_dtype, row.srow * a.c + q0 + q4 + e);
+          u = uv[e];
         } else {
           const uint32_t kb = (draw_bits(a.k0, a.k1, src + e, n, 8, LAYOUT) & 0xFFu) >> 1;
           ub |= kb << (8 * e);
@@ -403,74 +422,93 @@ __global__ __launch_bounds__(256) void k_mask_bwd_tile(SiteMaskArgs a, const bf1
   const int64_t j0 = (int64_t)blockIdx.y * TILE;
   const int q0 = blockIdx.x * TILE, q4 = PD_TILE4_COL;
   const bool qok = q0 + q4 < a.c;
-  if constexpr (SRC) {
-    if (tid < 64) {  // each row's (expert, source row) group; rows are sorted by it
-      const int64_t j = j0 + tid;
-      SG.grp[tid] = j < a.J ? row_group(a.offsets, a.E, j) * (int)a.S + (int)((a.sort_idx[j] / a.k) / a.rps) : -1;
-    }
-  }
-  fill_mask_rows<SRC || PM == PM_SL0>(rows, a, j0, tid);
+  if constexpr (SRC) fill_mask_rows<true>(rows, a, j0, tid, SG.grp);
+  else fill_mask_rows<PM == PM_SL0>(rows, a, j0, tid);
   __syncthreads();
+  // the loads of two passes go out together (of four: 91 us at 65536 x 512, half the waves)
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
-    const int r = PD_TILE4_ROW(pass);
-    const int64_t j = j0 + r;
-    bf16_t o[4] = {0, 0, 0, 0};
-    float dmsum = 0.f;
-    if (j < a.J && qok) {
-      const int64_t idx = j * a.c + q0 + q4;
-      const MaskRow row = rows[r];
-      const int32_t slot = row.slot;
-      const int64_t src = (int64_t)slot * a.c + q0 + q4;
-      const float dt = row.dt;
-      const uint2 pw = *(const uint2*)(a.ci_pre + src);
-      const uint2 hw = *(const uint2*)(h + idx);
-      const uint2 dw = row.routed ? *(const uint2*)(d_acts + idx) : make_uint2(0u, 0u);
-      const uint32_t ub = !SRC && a.uconst < 0.f ? *(const uint32_t*)(ubits + idx) : 0u;
-      const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
-      const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
-      const float da[4] = {bf_lo(dw.x), bf_hi(dw.x), bf_lo(dw.y), bf_hi(dw.y)};
-      bf16_t dp[4];
-      float slope4[4] = {imp_scale, imp_scale, imp_scale, imp_scale};
-      if constexpr (PM == PM_SL0) {
-        const float4 sl = *(const float4*)(a.slope + (int64_t)row.ej * a.c + q0 + q4);
-        slope4[0] = sl.x;
-        slope4[1] = sl.y;
-        slope4[2] = sl.z;
-        slope4[3] = sl.w;
+  for (int half = 0; half < 4; half += 2) {
+    uint2 pws[4], hws[4], dws[4];
+    uint4 tws[SRC ? 4 : 1];
+#pragma unroll
+    for (int pass = half; pass < half + 2; ++pass) {
+      const int r = PD_TILE4_ROW(pass);
+      if (j0 + r < a.J && qok) {
+        const int64_t idx = (j0 + r) * a.c + q0 + q4;
+        pws[pass] = *(const uint2*)(a.ci_pre + (int64_t)rows[r].slot * a.c + q0 + q4);
+        hws[pass] = *(const uint2*)(h + idx);
+        dws[pass] = *(const uint2*)(d_acts + idx);
+        if constexpr (SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, rows[r].srow * a.c + q0 + q4);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = lower_fwd(pre[e]), up = upper_fwd(pre[e]);
-        float u;
-        if constexpr (SRC) u = src_value(a.src, a.src_dtype, row.srow * a.c + q0 + q4 + e);
-        else u = a.uconst < 0.f ? (float)((ub >> (8 * e)) & 0xFFu) * (1.f / 128.f) : a.uconst;
-        const float m = lo + (1.f - lo) * u - dt;
-        float dimp;
-        if constexpr (PM == PM_SL0) dimp = slope4[e] * sl0_dpsi(up, a.g2, a.psis);
-        else dimp = imp_scale * dpowp<PM>(up, a.p);
-        const float dm = da[e] * hv[e];
-        dp[e] = f32_to_bf16(lower_vjp(pre[e], dm * (1.f - u)) + upper_vjp(pre[e], dimp));
-        o[e] = f32_to_bf16(da[e] * m);
-        if constexpr (SRC) {
-          dmsum += dm;
-          const float gs = dm * (1.f - lo);
-          if (a.rps == 1) a.dsrc[row.srow * a.c + q0 + q4 + e] = gs;
-          else SG.ps[r][q4 + e] = gs;
-        }
-      }
-      *(uint2*)(d_pre + src) = make_uint2(bf_pack(dp[0], dp[1]), bf_pack(dp[2], dp[3]));
-      *(uint2*)(d_acts + idx) = make_uint2(bf_pack(o[0], o[1]), bf_pack(o[2], o[3]));
-    } else if constexpr (SRC) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) SG.ps[r][q4 + e] = 0.f;
     }
-    if constexpr (SRC) {  // the 16 lanes of a row add their columns in a fixed tree (all lanes)
-      dmsum += __shfl_xor(dmsum, 1, 64);
-      dmsum += __shfl_xor(dmsum, 2, 64);
-      dmsum += __shfl_xor(dmsum, 4, 64);
-      dmsum += __shfl_xor(dmsum, 8, 64);
-      if (j < a.J && (tid & 15) == 0) a.rowdm[j * gridDim.x + blockIdx.x] = dmsum;
+#pragma unroll
+    for (int pass = half; pass < half + 2; ++pass) {
+      const int r = PD_TILE4_ROW(pass);
+      const int64_t j = j0 + r;
+      bf16_t o[4] = {0, 0, 0, 0};
+      float dmsum = 0.f;
+      if (j < a.J && qok) {
+        const int64_t idx = j * a.c + q0 + q4;
+        const MaskRow row = rows[r];
+        const int64_t src = (int64_t)row.slot * a.c + q0 + q4;
+        const float dt = row.dt;
+        const uint2 pw = pws[pass], hw = hws[pass];
+        const uint2 dw = row.routed ? dws[pass] : make_uint2(0u, 0u);
+        const uint32_t ub = !SRC && a.uconst < 0.f ? *(const uint32_t*)(ubits + idx) : 0u;
+        const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
+        const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
+        const float da[4] = {bf_lo(dw.x), bf_hi(dw.x), bf_lo(dw.y), bf_hi(dw.y)};
+        bf16_t dp[4];
+        float uv[4], gs[4];
+        if constexpr (SRC) src_quad_values(tws[pass], a.src_dtype, uv);
+        float slope4[4] = {imp_scale, imp_scale, imp_scale, imp_scale};
+        if constexpr (PM == PM_SL0) {
+          const float4 sl = *(const float4*)(a.slope + (int64_t)row.ej * a.c + q0 + q4);
+          slope4[0] = sl.x;
+          slope4[1] = sl.y;
+          slope4[2] = sl.z;
+          slope4[3] = sl.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = lower_fwd(pre[e]), up = upper_fwd(pre[e]);
+          float u;
+          if constexpr (SRC) u = uv[e];
+          else u = a.uconst < 0.f ? (float)((ub >> (8 * e)) & 0xFFu) * (1.f / 128.f) : a.uconst;
+          const float m = lo + (1.f - lo) * u - dt;
+          float dimp;
+          if constexpr (PM == PM_SL0) dimp = slope4[e] * sl0_dpsi(up, a.g2, a.psis);
+          else dimp = imp_scale * dpowp<PM>(up, a.p);
+          const float dm = da[e] * hv[e];
+          dp[e] = f32_to_bf16(lower_vjp(pre[e], dm * (1.f - u)) + upper_vjp(pre[e], dimp));
+          o[e] = f32_to_bf16(da[e] * m);
+          if constexpr (SRC) {
+            dmsum += dm;
+            gs[e] = dm * (1.f - lo);
+          }
+        }
+        if constexpr (SRC) {
+          if (a.rps == 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a.dsrc[row.srow * a.c + q0 + q4 + e] = gs[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) SG.ps[r][q4 + e] = gs[e];
+          }
+        }
+        *(uint2*)(d_pre + src) = make_uint2(bf_pack(dp[0], dp[1]), bf_pack(dp[2], dp[3]));
+        *(uint2*)(d_acts + idx) = make_uint2(bf_pack(o[0], o[1]), bf_pack(o[2], o[3]));
+      } else if constexpr (SRC) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) SG.ps[r][q4 + e] = 0.f;
+      }
+      if constexpr (SRC) {  // the 16 lanes of a row add their columns in a fixed tree (all lanes)
+        dmsum += __shfl_xor(dmsum, 1, 64);
+        dmsum += __shfl_xor(dmsum, 2, 64);
+        dmsum += __shfl_xor(dmsum, 4, 64);
+        dmsum += __shfl_xor(dmsum, 8, 64);
+        if (j < a.J && (tid & 15) == 0) a.rowdm[j * gridDim.x + blockIdx.x] = dmsum;
+      }
     }
   }
   if constexpr (SRC) {
@@ -1126,27 +1164,44 @@ __global__ __launch_bounds__(256) void k_job_delta_cot(const bf16_t* __restrict_
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc = fmaf(a[e], b[e], acc);
   }
-  acc = wave_sum(acc);
-  if (lane == 0) {
-    float dm = 0.f;
-    for (int p = 0; p < n_parts; ++p) dm += rowdm[j * n_parts + p];
-    q[j] = acc - dm;
-  }
+  float dm = 0.f;
+  for (int p = lane; p < n_parts; p += 64) dm += rowdm[j * n_parts + p];
+  acc = wave_sum(acc - dm);
+  if (lane == 0) q[j] = acc;
 }
 
-// d_src_delta[row] = sum over the row's tokens t of sum_s q[inv[t*k + s]]. One wave per
-// source row, a fixed order (lane-strided tokens, then the wave tree).
+// d_src_delta[row] = sum over the row's tokens t of sum_s q[inv[t*k + s]], WAVES waves a row
+// (blocks of 4 waves): a row of many tokens takes a whole block, since its gathers are what
+// the time is (16 rows of 512 tokens, k = 8: 28 us with a wave a row, 6 with a block). Fixed order
+// (the lanes' strided jobs, the wave tree, the waves).
+template <int WAVES>
 __global__ __launch_bounds__(256) void k_src_delta_grad(const float* __restrict__ q, const int32_t* __restrict__ inv,
                                                         int64_t S, int64_t rps, int k,
                                                         float* __restrict__ d_src_delta) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + wave_id();
+  static_assert(WAVES == 1 || WAVES == 4, "a wave or a block per row");
+  const int64_t row = WAVES == 1 ? (int64_t)blockIdx.x * 4 + wave_id() : (int64_t)blockIdx.x;
   if (row >= S) return;
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, first = WAVES == 1 ? lane : (int)threadIdx.x;
+  const int64_t n = rps * k, base = row * n;
   float acc = 0.f;
-  for (int64_t t = row * rps + lane; t < (row + 1) * rps; t += 64)
-    for (int s = 0; s < k; ++s) acc += q[inv[t * k + s]];
+  int64_t i = first;
+  for (; i + 7 * 64 * WAVES < n; i += 8 * 64 * WAVES) {  // eight gathers in flight
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = q[inv[base + i + e * 64 * WAVES]];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc += v[e];
+  }
+  for (; i < n; i += 64 * WAVES) acc += q[inv[base + i]];
   acc = wave_sum(acc);
-  if (lane == 0) d_src_delta[row] = acc;
+  if constexpr (WAVES == 1) {
+    if (lane == 0) d_src_delta[row] = acc;
+  } else {
+    __shared__ float red[4];
+    if (lane == 0) red[wave_id()] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) d_src_delta[row] = (red[0] + red[1]) + (red[2] + red[3]);
+  }
 }
 
 // out[0, n) = 0.
@@ -1902,7 +1957,11 @@ static int moe_step_impl(int64_t T, int d, int f, int E, int k, int c, int L, co
       if (use_delta) {
         hipLaunchKernelGGL(k_job_delta_cot, dim3((unsigned)cdiv(J, 4)), dim3(256), 0, s, gout, frozen, P.rowdm,
                            (int)cdiv(c, TILE), J, width, P.qjob);
-        hipLaunchKernelGGL(k_src_delta_grad, dim3((unsigned)cdiv(D.S, 4)), dim3(256), 0, s, P.qjob, S.inv, D.S,
+        if (srcs->rps * k > 512)  // more than eight jobs a lane: a block per source row
+          hipLaunchKernelGGL(k_src_delta_grad<4>, dim3((unsigned)D.S), dim3(256), 0, s, P.qjob, S.inv, D.S,
+                           srcs->rps, k, srcs->d_src_delta + ((size_t)l * 3 + si) * D.S);
+        else
+          hipLaunchKernelGGL(k_src_delta_grad<1>, dim3((unsigned)cdiv(D.S, 4)), dim3(256), 0, s, P.qjob, S.inv, D.S,
                            srcs->rps, k, srcs->d_src_delta + ((size_t)l * 3 + si) * D.S);
       }
     };
