@@ -72,6 +72,32 @@ size_t gemm_splitk_ws_bytes(int64_t M, int64_t N, int64_t K, int splits = 0);
 int gemm_splitk(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int trans_a, const void* B, int64_t ldb,
                 int trans_b, void* C, int64_t ldc, int c_dtype, float beta, void* ws, size_t ws_bytes, void* stream,
                 int splits = 0);
+
+// One fp32 product C = op(A) op(B) of the direct form in pd_gemm.hip, row-major like C; `post` on
+// the element v of C: 0 none, 1 max(v, 0), 2 v where `Cin` (C's shape and ldc) is positive
+// and 0 elsewhere. With Cin and post < 2, C = Cin + the product (Cin may be C).
+struct F32Prod {
+  int64_t M, N, K;
+  const float* A;
+  int64_t lda;
+  int32_t ta;
+  const float* B;
+  int64_t ldb;
+  int32_t tb;
+  float* C;
+  int64_t ldc;
+  const float* Cin;
+  int32_t post;
+};
+// The product through the direct form, or false (nothing launched) where pd_gemm would take
+// another form.
+bool gemm_f32_direct(const F32Prod& p, hipStream_t s);
+// Up to F32_GROUP products with one `ta` in one launch, for outputs too small to fill the
+// GPU alone. splits > 1 cuts every contraction into that many slices, each written to its
+// own [M, N] slab from C on (ldc = N, no Cin or post). False (nothing launched) where an
+// operand reaches 2^31 bytes.
+static constexpr int F32_GROUP = 6;
+bool gemm_f32_group(const F32Prod* p, int n, int splits, hipStream_t s);
 int gemm_nt_splitk(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* Bt, int64_t ldb, void* C,
                    int64_t ldc, int c_dtype, float beta, void* ws, size_t ws_bytes, void* stream);
 

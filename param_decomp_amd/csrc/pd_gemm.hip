@@ -330,96 +330,117 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // LDS stage. Within each 16-k batch the two lane halves take different k: half h supplies
 // k = kc + 8h + s on MFMA step s (the two k slots of v_mfma_f32_32x32x2_f32), so
 //   an MN-contiguous operand is one coalesced dword per lane and step (32 consecutive
-//     floats per half), loaded through a buffer descriptor: an element outside the matrix
-//     or the wave's k range gets an offset past the descriptor's end, which the hardware
-//     returns as 0, so no value select follows a load and nothing waits for one until the
-//     MFMA that reads it;
-//   a K-contiguous operand is 8 consecutive floats per lane: two 16-byte loads when
-//     `vec` says rows are 16-byte aligned and K % 4 == 0 (each 4-run then lies wholly
-//     inside or outside the k range), else 8 dwords through the descriptor.
-// The next batch's loads are in flight during this batch's 8 MFMAs. Block forms as in
-// k_gemm_f32 (KW waves splitting the contraction of a 32x32 tile, or 4 waves of a 64x64
-// tile); the summation order is fixed. Measured at the residual-MLP target's products
-// (2048 rows, d 1000 / 100 / 50) it takes 0.35-0.6x the time of the LDS-staged form: those
-// launches hold one or two waves per SIMD, and the LDS round trip per 16-k chunk was
-// exposed latency there. Each operand must span fewer than 2^31 bytes (checked on the host).
+//     floats per half);
+//   a K-contiguous operand is 8 consecutive floats per lane, loaded 4, 2 or 1 at a time
+//     (`vec`: A's width + 16 times B's): as many as divide K, so that each run lies wholly
+//     inside or outside the k range, and as every row's start is aligned to. Each such load
+//     touches one cache line per lane, so it costs the same at any width.
+// Every load goes through a buffer descriptor and is issued without a branch: an element
+// outside the matrix or the wave's k range gets an offset past the descriptor's end, which
+// the hardware returns as 0. Behind a branch the compiler has to assume that the loads were
+// not issued and waits for every load in flight before each batch's MFMAs. F32_AHEAD batches
+// are in flight: these launches hold one or two blocks per CU, so the load latency is what
+// bounds them, and a fourth batch spills at 16 waves per block (128 registers).
+// Block forms as in k_gemm_f32 (KW waves splitting the contraction of a 32x32 tile, or 4
+// waves of a 64x64 tile); the summation order is fixed. Each operand must span fewer than
+// 2^31 bytes (checked on the host). 2048x1000 over 50, both K-contiguous at row stride 50,
+// 17.6 us in dword loads (and a 3.6 us copy before it), 14.5 in 8-byte
+// loads; the whole residual-MLP step 296 -> 223 us with the grouped launches below.
+constexpr int F32_AHEAD = 3;
+
 template <int KW, bool TA, bool TB>
-__global__ __launch_bounds__(KW > 1 ? 64 * KW : 256) void k_gemm_f32_direct(
-    int64_t M, int64_t N, int64_t K, const float* __restrict__ A, int64_t lda, const float* __restrict__ B,
-    int64_t ldb, float* __restrict__ C, int64_t ldc, float alpha, float beta, int64_t sA, int64_t sB, int64_t sC,
-    int32_t bytes_a, int32_t bytes_b, int vec) {
+__device__ inline void f32_direct_tile(const F32Prod& p, int bm, int bn, int kbeg, int kend, int32_t bytes_a,
+                                       int32_t bytes_b, int vec, float alpha, float beta, float (*red)[FT * FT]) {
   constexpr bool SPLIT = KW > 1;
-  constexpr int NWV = SPLIT ? KW : 4, NT = 64 * NWV, S = 8;
-  __shared__ float red[SPLIT ? KW : 1][SPLIT ? FT * FT : 1];
-  A += (int64_t)blockIdx.z * sA;
-  B += (int64_t)blockIdx.z * sB;
-  C += (int64_t)blockIdx.z * sC;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5;
+  constexpr int NWV = SPLIT ? KW : 4, NT = 64 * NWV, S = 8, D = F32_AHEAD;
+  const float *A = p.A, *B = p.B, *Cin = p.Cin;
+  float* C = p.C;
+  const int64_t M = p.M, N = p.N, ldc = p.ldc;
+  // the wave index as a scalar, so that a batch's position is one and each load's offset is
+  // one lane register plus a scalar
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
   const int64_t bt = SPLIT ? FT : 2 * FT;
-  const int64_t m0 = (int64_t)blockIdx.y * bt + (SPLIT ? 0 : (w >> 1) * FT);
-  const int64_t n0 = (int64_t)blockIdx.x * bt + (SPLIT ? 0 : (w & 1) * FT);
-  int kb = 0, ke = (int)K;
+  const int64_t m0 = bm * bt + (SPLIT ? 0 : (w >> 1) * FT);
+  const int64_t n0 = bn * bt + (SPLIT ? 0 : (w & 1) * FT);
+  int kb = kbeg, ke = kend;
   if (SPLIT) {
-    const int kq = (int)((K + KW * FK - 1) / (KW * FK) * FK);
-    kb = w * kq;
+    const int kq = (kend - kbeg + KW * FK - 1) / (KW * FK) * FK;
+    kb = kbeg + w * kq;
     ke = kb + kq < ke ? kb + kq : ke;
   }
   const uint32_t m = (uint32_t)(m0 + (lane & 31)), n = (uint32_t)(n0 + (lane & 31));
-  const bool mok = m < M, nok = n < N;
-  const uint32_t la = (uint32_t)lda, lb = (uint32_t)ldb;
+  const uint32_t sta = TA ? (uint32_t)p.lda : 1u, stb = TB ? 1u : (uint32_t)p.ldb;  // elements from k to k + 1
   const auto rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), (short)0, bytes_a, 0x00020000);
   const auto rsb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, bytes_b, 0x00020000);
-  // bit 31 set for an element outside the operand: offsets of in-range elements are < 2^31
-  auto oob = [](bool ok) { return (uint32_t)(!ok) << 31; };
-  auto load = [&](float (&a)[S], float (&b)[S], int kc) {
-    const int k0 = kc + h * S;
-    if (!TA && (vec & 1)) {
+  // byte offset of the lane's element at k = 8h, and 8h itself: past any range for a row
+  // outside the matrix
+  const uint32_t oa = ((TA ? m : m * (uint32_t)p.lda) + h * S * sta) * 4u;
+  const uint32_t ob = ((TB ? n * (uint32_t)p.ldb : n) + h * S * stb) * 4u;
+  const int ha = m < M ? h * S : INT32_MAX, hb = n < N ? h * S : INT32_MAX;
+  // offsets of in-range elements are < 2^31; 2^31 is past every descriptor's end
+  auto load1 = [&](auto width, float (&x)[S], const auto& rs, uint32_t o, uint32_t st, int hs, int kc) {
+    constexpr int W = decltype(width)::value;
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        float4 v = {0.f, 0.f, 0.f, 0.f};
-        if (mok && k0 + 4 * q < ke) v = *(const float4*)(A + (int64_t)m * lda + k0 + 4 * q);
-        a[4 * q] = v.x, a[4 * q + 1] = v.y, a[4 * q + 2] = v.z, a[4 * q + 3] = v.w;
-      }
-    } else {
+    for (int s = 0; s < S; s += W) {
+      const uint32_t off = hs < ke - kc - s ? o + (uint32_t)(kc + s) * st * 4u : 1u << 31;
+      if constexpr (W == 1) {
+        x[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+      } else {
+        uint32_t u[W];  // a bit cast of a vector's element itself reads element 0
+        if constexpr (W == 2) {
+          const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
+          u[0] = v[0], u[1] = v[1];
+        } else {
+          const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+          u[0] = v[0], u[1] = v[1], u[2] = v[2], u[3] = v[3];
+        }
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const uint32_t k = (uint32_t)(k0 + s), e = TA ? k * la + m : m * la + k;
-        a[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, (e * 4u) | oob(mok & (k0 + s < ke)),
-                                                                              0, 0));
-      }
-    }
-    if (TB && (vec & 2)) {
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        float4 v = {0.f, 0.f, 0.f, 0.f};
-        if (nok && k0 + 4 * q < ke) v = *(const float4*)(B + (int64_t)n * ldb + k0 + 4 * q);
-        b[4 * q] = v.x, b[4 * q + 1] = v.y, b[4 * q + 2] = v.z, b[4 * q + 3] = v.w;
-      }
-    } else {
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const uint32_t k = (uint32_t)(k0 + s), e = TB ? n * lb + k : k * lb + n;
-        b[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsb, (e * 4u) | oob(nok & (k0 + s < ke)),
-                                                                              0, 0));
+        for (int e = 0; e < W; ++e) x[s + e] = __builtin_bit_cast(float, u[e]);
       }
     }
+  };
+  auto load = [&](auto wa, auto wb, float (&a)[S], float (&b)[S], int kc) {
+    load1(wa, a, rsa, oa, sta, ha, kc);
+    load1(wb, b, rsb, ob, stb, hb, kc);
   };
   f32x16 acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  auto mma = [&](const float (&a)[S], const float (&b)[S]) {
+  auto contract = [&](auto wa, auto wb) {
+    float a[D][S], b[D][S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+    for (int d = 0; d < D; ++d) load(wa, wb, a[d], b[d], kb + d * FK);
+    for (int kc = kb; kc < ke; kc += D * FK) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        if (kc + d * FK >= ke) return;
+#pragma unroll
+        for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][s], b[d][s], acc, 0, 0, 0);
+        load(wa, wb, a[d], b[d], kc + (d + D) * FK);
+      }
+    }
   };
-  float a0[S], b0[S], a1[S], b1[S];
-  if (kb < ke) load(a0, b0, kb);
-  for (int kc = kb; kc < ke; kc += 2 * FK) {
-    if (kc + FK < ke) load(a1, b1, kc + FK);
-    mma(a0, b0);
-    if (kc + FK >= ke) break;
-    if (kc + 2 * FK < ke) load(a0, b0, kc + 2 * FK);
-    mma(a1, b1);
-  }
+  typedef std::integral_constant<int, 1> W1;
+  typedef std::integral_constant<int, 2> W2;
+  typedef std::integral_constant<int, 4> W4;
+  auto with_b = [&](auto wa) {
+    if constexpr (TB) {
+      if ((vec >> 4) == 4) return contract(wa, W4{});
+      if ((vec >> 4) == 2) return contract(wa, W2{});
+    }
+    contract(wa, W1{});
+  };
+  const int va = vec & 15;
+  if (TA || va == 1) with_b(W1{});
+  else if (va == 4) with_b(W4{});
+  else with_b(W2{});
+  auto put = [&](int64_t gr, int64_t gc, float sum) {
+    const int64_t i = gr * ldc + gc;
+    float v = alpha * sum + (beta != 0.f ? beta * Cin[i] : 0.f);
+    if (p.post == 1) v = fmaxf(v, 0.f);
+    else if (p.post == 2) v = Cin[i] > 0.f ? v : 0.f;
+    C[i] = v;
+  };
   // lane holds column lane & 31, rows 8 (v / 4) + 4 (lane / 32) + v % 4 of its tile
   if constexpr (SPLIT) {
 #pragma unroll
@@ -432,44 +453,105 @@ __global__ __launch_bounds__(KW > 1 ? 64 * KW : 256) void k_gemm_f32_direct(
 #pragma unroll
       for (int x = 1; x < KW; ++x) sum += red[x][i];
       const int64_t gr = m0 + r, gc = n0 + c;
-      if (gr < M && gc < N) C[gr * ldc + gc] = alpha * sum + (beta != 0.f ? beta * C[gr * ldc + gc] : 0.f);
+      if (gr < M && gc < N) put(gr, gc, sum);
     }
   } else {
     const int64_t gc = n0 + (lane & 31);
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int64_t gr = m0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-      if (gr < M && gc < N) C[gr * ldc + gc] = alpha * acc[v] + (beta != 0.f ? beta * C[gr * ldc + gc] : 0.f);
+      if (gr < M && gc < N) put(gr, gc, acc[v]);
     }
   }
+}
+
+template <int KW, bool TA, bool TB>
+__global__ __launch_bounds__(KW > 1 ? 64 * KW : 256, KW > 1 ? 4 : 3) void k_gemm_f32_direct(F32Prod p, float alpha, float beta,
+                                                                           int64_t sA, int64_t sB, int64_t sC,
+                                                                           int32_t bytes_a, int32_t bytes_b, int vec) {
+  __shared__ float red[KW > 1 ? KW : 1][KW > 1 ? FT * FT : 1];
+  p.A += (int64_t)blockIdx.z * sA;
+  p.B += (int64_t)blockIdx.z * sB;
+  p.C += (int64_t)blockIdx.z * sC;
+  p.Cin += (int64_t)blockIdx.z * sC;
+  f32_direct_tile<KW, TA, TB>(p, (int)blockIdx.y, (int)blockIdx.x, 0, (int)p.K, bytes_a, bytes_b, vec, alpha, beta,
+                              (float(*)[FT * FT])red);
+}
+
+struct F32Group {
+  F32Prod p[F32_GROUP];
+  int32_t bytes_a[F32_GROUP], bytes_b[F32_GROUP], vec[F32_GROUP], tiles_n[F32_GROUP], first[F32_GROUP + 1];
+  int32_t n, splits;
+};
+
+// Several small products in one launch: a block of KW waves takes one 32x32 tile of one
+// product, or one contraction slice of it.
+template <int KW, bool TA>
+__global__ __launch_bounds__(64 * KW) void k_gemm_f32_group(F32Group g) {
+  __shared__ float red[KW][FT * FT];
+  int i = 0;
+  while (i + 1 < g.n && (int)blockIdx.x >= g.first[i + 1]) ++i;
+  F32Prod p = g.p[i];
+  const int u = (int)blockIdx.x - g.first[i], t = u / g.splits, sl = u % g.splits;
+  const int K = (int)p.K, kq = (K + g.splits * FK - 1) / (g.splits * FK) * FK;
+  const int kb = sl * kq, ke = kb + kq < K ? kb + kq : K;  // kb >= ke: a slab of zeros
+  p.C += (int64_t)sl * p.M * p.N;
+  const int bm = t / g.tiles_n[i], bn = t % g.tiles_n[i];
+  const float beta = p.Cin && p.post < 2 ? 1.f : 0.f;
+  if (p.tb) f32_direct_tile<KW, TA, true>(p, bm, bn, kb, ke, g.bytes_a[i], g.bytes_b[i], g.vec[i], 1.f, beta, red);
+  else f32_direct_tile<KW, TA, false>(p, bm, bn, kb, ke, g.bytes_a[i], g.bytes_b[i], g.vec[i], 1.f, beta, red);
+}
+
+// Bytes the operands span, and the floats per load of each (`vec` of f32_direct_tile).
+struct F32Span {
+  int64_t a, b;
+  int vec;
+  bool fits;
+};
+static F32Span f32_span(const F32Prod& p, int64_t sA = 0, int64_t sB = 0) {
+  const int64_t ea = 4 * (p.ta ? (p.K - 1) * p.lda + p.M : (p.M - 1) * p.lda + p.K);
+  const int64_t eb = 4 * (p.tb ? (p.N - 1) * p.ldb + p.K : (p.K - 1) * p.ldb + p.N);
+  auto width = [&](const float* x, int64_t ld, int64_t stride) {
+    auto by = [&](int w) { return p.K % w == 0 && ld % w == 0 && stride % w == 0 && (uintptr_t)x % (4 * w) == 0; };
+    return by(4) ? 4 : by(2) ? 2 : 1;
+  };
+  const int vec = (p.ta ? 1 : width(p.A, p.lda, sA)) | (p.tb ? width(p.B, p.ldb, sB) : 1) << 4;
+  return {ea, eb, vec, ea < (int64_t(1) << 31) && eb < (int64_t(1) << 31)};
 }
 
 // The fp32 block form. Whole-contraction 64x64 tiles once they alone give >= 512 blocks
 // (direct form up to K = 256, the LDS-staged one beyond), else 32x32 tiles with the
 // contraction split over waves: the direct form with 16 waves from K = 512 on, else 8.
 // The LDS-staged form also serves operands of 2^31 bytes or more.
+static bool f32_big(int64_t M, int64_t N, int64_t batch) { return cdiv(M, 2 * FT) * cdiv(N, 2 * FT) * batch >= 512; }
+
+template <bool TA, bool TB>
+static bool launch_f32_direct(const F32Prod& p, int64_t batch, float alpha, float beta, int64_t sA, int64_t sB,
+                              int64_t sC, hipStream_t s) {
+  const F32Span sp = f32_span(p, sA, sB);
+  const bool big = f32_big(p.M, p.N, batch);
+  if (!sp.fits || (big && p.K > 256)) return false;
+  const int64_t t = big ? 2 * FT : FT;
+  const dim3 grid((unsigned)cdiv(p.N, t), (unsigned)cdiv(p.M, t), (unsigned)batch);
+#define PD_FD(KW_)                                                                                                   \
+  hipLaunchKernelGGL((k_gemm_f32_direct<KW_, TA, TB>), grid, dim3(KW_ > 1 ? 64 * KW_ : 256), 0, s, p, alpha, beta, sA, \
+                     sB, sC, (int32_t)sp.a, (int32_t)sp.b, sp.vec)
+  if (big) PD_FD(1);
+  else if (p.K >= 512) PD_FD(16);
+  else PD_FD(8);
+#undef PD_FD
+  return true;
+}
+
 template <bool TA, bool TB>
 static void launch_gemm_f32_l(int64_t batch, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
                               const float* B, int64_t ldb, float* C, int64_t ldc, float alpha, float beta, int64_t sA,
                               int64_t sB, int64_t sC, hipStream_t s) {
+  const F32Prod p{M, N, K, A, lda, TA, B, ldb, TB, C, ldc, C, 0};
+  if (launch_f32_direct<TA, TB>(p, batch, alpha, beta, sA, sB, sC, s)) return;
   const dim3 g32((unsigned)cdiv(N, FT), (unsigned)cdiv(M, FT), (unsigned)batch);
   const dim3 g64((unsigned)cdiv(N, 2 * FT), (unsigned)cdiv(M, 2 * FT), (unsigned)batch);
-  const int64_t ea = 4 * (TA ? (K - 1) * lda + M : (M - 1) * lda + K);  // bytes one operand spans
-  const int64_t eb = 4 * (TB ? (N - 1) * ldb + K : (K - 1) * ldb + N);
-  const bool direct = ea < (int64_t(1) << 31) && eb < (int64_t(1) << 31);
-  const bool big = cdiv(M, 2 * FT) * cdiv(N, 2 * FT) * batch >= 512;
-  if (direct && (!big || K <= 256)) {
-    const bool v4 = K % 4 == 0;
-    const int vec = (!TA && v4 && lda % 4 == 0 && sA % 4 == 0 && aligned16(A) ? 1 : 0) |
-                    (TB && v4 && ldb % 4 == 0 && sB % 4 == 0 && aligned16(B) ? 2 : 0);
-#define PD_FD(KW_, G_)                                                                                               \
-  hipLaunchKernelGGL((k_gemm_f32_direct<KW_, TA, TB>), G_, dim3(KW_ > 1 ? 64 * KW_ : 256), 0, s, M, N, K, A, lda, B, \
-                     ldb, C, ldc, alpha, beta, sA, sB, sC, (int32_t)ea, (int32_t)eb, vec)
-    if (big) PD_FD(1, g64);
-    else if (K >= 512) PD_FD(16, g32);
-    else PD_FD(8, g32);
-#undef PD_FD
-  } else if (big)
+  if (f32_big(M, N, batch))
     hipLaunchKernelGGL((k_gemm_f32<1, TA, TB>), g64, dim3(256), 0, s, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, sA,
                        sB, sC);
   else if (K >= 1024)
@@ -487,6 +569,42 @@ static void launch_gemm_f32(int64_t batch, int64_t M, int64_t N, int64_t K, cons
   else if (ta) launch_gemm_f32_l<true, false>(batch, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, sA, sB, sC, s);
   else if (tb) launch_gemm_f32_l<false, true>(batch, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, sA, sB, sC, s);
   else launch_gemm_f32_l<false, false>(batch, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, sA, sB, sC, s);
+}
+
+bool gemm_f32_direct(const F32Prod& p, hipStream_t s) {
+  const float beta = p.Cin && p.post < 2 ? 1.f : 0.f;
+  if (p.ta) return p.tb ? launch_f32_direct<true, true>(p, 1, 1.f, beta, 0, 0, 0, s)
+                        : launch_f32_direct<true, false>(p, 1, 1.f, beta, 0, 0, 0, s);
+  return p.tb ? launch_f32_direct<false, true>(p, 1, 1.f, beta, 0, 0, 0, s)
+              : launch_f32_direct<false, false>(p, 1, 1.f, beta, 0, 0, 0, s);
+}
+
+bool gemm_f32_group(const F32Prod* p, int n, int splits, hipStream_t s) {
+  F32Group g{};
+  g.n = n;
+  g.splits = splits;
+  int64_t blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    const F32Span sp = f32_span(p[i]);
+    if (!sp.fits || p[i].ta != p[0].ta) return false;
+    g.p[i] = p[i];
+    g.bytes_a[i] = (int32_t)sp.a;
+    g.bytes_b[i] = (int32_t)sp.b;
+    g.vec[i] = sp.vec;
+    g.tiles_n[i] = (int32_t)cdiv(p[i].N, FT);
+    g.first[i] = (int32_t)blocks;
+    blocks += cdiv(p[i].M, FT) * g.tiles_n[i] * splits;
+    if (blocks >= (int64_t(1) << 31)) return false;
+  }
+  g.first[n] = (int32_t)blocks;
+  // partial sums at most as long as the single products': 16 waves over a long contraction,
+  // 8 over the slices of a transposed A's
+#define PD_FG(KW_, TA_) hipLaunchKernelGGL((k_gemm_f32_group<KW_, TA_>), dim3((unsigned)blocks), dim3(64 * KW_), 0, s, g)
+  if (p[0].ta) PD_FG(8, true);
+  else if (p[0].K >= 512) PD_FG(16, false);
+  else PD_FG(8, false);
+#undef PD_FG
+  return true;
 }
 
 __global__ void k_zero_tail_rows(const int32_t* __restrict__ offsets, int E, int64_t J, int64_t width, int out_bytes,

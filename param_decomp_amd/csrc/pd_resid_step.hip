@@ -15,8 +15,11 @@
 // draw, masked activations and imp-min term form one column-mapped pass (one lane per
 // component over RM_ROWS rows), and its backward (mask pullback into both a V operands,
 // squashing and gate pullbacks, gate-parameter partials) another; the partials are added
-// over row chunks in a fixed order. At the 1-layer benchmark shape that is 31 launches
-// per step, against about 90 for the same step composed from the library's primitives.
+// over row chunks in a fixed order. Relus and residual sums are the products' epilogues,
+// independent small products share a launch. At the 1-layer benchmark shape (2048 x 1000, C =
+// 100) that is 22 launches and 223 us per step (31 and 296 with one launch per product, relu,
+// copy and weight gradient), against about 90 launches for the same step composed from the
+// library's primitives.
 #include <algorithm>
 #include <vector>
 
@@ -280,9 +283,45 @@ struct RmArena {
 
 struct RmWork {
   std::vector<float*> r, rm, hidc, hid, hg, ha, graw, acts;  // per layer (r, rm: L + 1) / per site
-  float *clean, *out, *d_out, *d_r, *d_r2, *d_acts, *d_ha, *d_hg, *d_hid, *rec_part, *imp_part, *gpart;
+  float *clean, *out, *d_out, *d_r, *d_r2, *d_acts, *d_hid, *rec_part, *imp_part, *gpart, *wpart;
+  float *d_ha[2], *d_hg[2];  // mlp_in's, mlp_out's: a layer's weight gradients are taken together
+  int splits;                // contraction slices of the weight gradients, 0: one product at a time
   size_t bytes;
 };
+
+// A layer's weight gradients (up to 6 products over the batch) run in one launch, each
+// contraction cut into slices of at least 256 rows, as many as give the chip four blocks
+// per CU; their slabs are added in order afterwards. One at a time each took 16 us however
+// small its output: 16 waves of one CU walking the whole batch. Outputs that fill the chip by
+// themselves stay single products. At 2048 rows, D = 1000, C = 100, M = 50 (280 tiles, 4 slices):
+// 81 us in five launches, 31 in two.
+// What bounds them now is L2: a 32x32 tile of one wave reads 512 bytes per MFMA.
+static int rm_splits(const RmDims& D) {
+  const int64_t tm = cdiv(D.M, 32), tc = cdiv(D.C, 32), td = cdiv(D.D, 32);
+  const int64_t tiles = (D.L > 1 ? 3 : 2) * td * tc + 3 * tm * tc;
+  if (tiles > 1024) return 0;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({D.B / 256, cdiv(1024, tiles), 16}));
+}
+
+// Sums of consecutive [n] slabs, in order: the weight gradients' contraction slices.
+struct RmSums {
+  const float* src[4];
+  float* dst[4];
+  int64_t n[4], first[5];
+  int32_t slabs[4];
+};
+__global__ __launch_bounds__(256) void k_rm_sum_slabs(RmSums a) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int q = 0;
+  while (q < 3 && i >= a.first[q + 1]) ++q;
+  i -= a.first[q];
+  const int64_t n = a.n[q];
+  if (i >= n) return;
+  const float* src = a.src[q] + i;
+  float sum = src[0];
+  for (int x = 1; x < a.slabs[q]; ++x) sum += src[x * n];
+  a.dst[q][i] = sum;
+}
 
 static RmWork rm_layout(const RmDims& D, char* base) {
   RmArena A{base};
@@ -308,12 +347,16 @@ static RmWork rm_layout(const RmDims& D, char* base) {
   W.d_r = A.take(B * D.D);
   W.d_r2 = A.take(B * D.D);
   W.d_acts = A.take(B * D.C);
-  W.d_ha = A.take(B * D.C);
-  W.d_hg = A.take(B * D.C);
+  for (int q = 0; q < 2; ++q) {
+    W.d_ha[q] = A.take(B * D.C);
+    W.d_hg[q] = A.take(B * D.C);
+  }
   W.d_hid = A.take(B * D.M);
   W.rec_part = A.take(RM_REC_BLOCKS);
   W.imp_part = A.take((int64_t)D.nsites() * D.chunks() * D.cblocks());
   W.gpart = A.take((int64_t)D.nsites() * D.chunks() * RM_GATE * D.C);
+  W.splits = rm_splits(D);
+  W.wpart = A.take(W.splits * (int64_t)D.C * (3 * (int64_t)D.D + 3 * (int64_t)D.M));
   W.bytes = A.off;
   return W;
 }
@@ -379,20 +422,43 @@ int pd_resid_mlp_step(int64_t B, int F, int D, int M, int C, int L, const float*
                   int tb, float* c, int64_t ldc, float beta) {
     return pd_gemm(PD_DTYPE_F32, m, nn, k, a, lda, ta, b, ldb, tb, c, ldc, PD_DTYPE_F32, 1.f, beta, s);
   };
+  auto prod = [&](int64_t m, int64_t nn, int64_t k, const float* a, int ta, const float* b, int tb, float* c,
+                  const float* cin = nullptr, int post = 0) {
+    return F32Prod{m, nn, k, a, ta ? m : k, ta, b, tb ? k : nn, tb, c, nn, cin, post};
+  };
+  // One product with its Cin / post in the epilogue; where the direct form does not take it,
+  // as separate passes.
+  auto fused = [&](const F32Prod& q) {
+    if (gemm_f32_direct(q, s)) return (int)PD_OK;
+    const bool add = q.Cin && q.post < 2;
+    if (add && q.Cin != q.C)
+      hipMemcpyAsync(q.C, q.Cin, (size_t)q.M * q.N * sizeof(float), hipMemcpyDeviceToDevice, s);
+    if (int e = gemm(q.M, q.N, q.K, q.A, q.lda, q.ta, q.B, q.ldb, q.tb, q.C, q.ldc, add ? 1.f : 0.f)) return e;
+    const int64_t n = q.M * q.N;
+    if (q.post == 1) hipLaunchKernelGGL(k_rm_relu, dim3(rm_ew_blocks(n)), dim3(256), 0, s, q.C, n);
+    if (q.post == 2) hipLaunchKernelGGL(k_rm_relu_bwd, dim3(rm_ew_blocks(n)), dim3(256), 0, s, q.C, q.Cin, n);
+    return (int)PD_OK;
+  };
+  // Two independent products over the same rows: in one launch while both outputs are small
+  // (fewer than 1024 32x32 tiles together, four blocks of 8 waves per CU), else one by one.
+  auto two = [&](const F32Prod& x, const F32Prod& y) {
+    const F32Prod q[2] = {x, y};
+    if (cdiv(x.M, 32) * (cdiv(x.N, 32) + cdiv(y.N, 32)) < 1024 && gemm_f32_group(q, 2, 1, s)) return (int)PD_OK;
+    const int e = fused(x);
+    return e ? e : fused(y);
+  };
   const dim3 sgrid((unsigned)Dm.cblocks(), (unsigned)Dm.chunks());
   const int64_t nsite_blocks = Dm.chunks() * Dm.cblocks();
 
   // ---- clean pass: r_{l+1} = r_l + relu(r_l W_in^T) W_out^T; the gate inputs a V
-  if ((rc = gemm(B, D, F, x, F, 0, W_E, D, 0, W.r[0], D, 0.f))) return rc;
+  if ((rc = fused(prod(B, D, F, x, 0, W_E, 0, W.r[0])))) return rc;
   for (int l = 0; l < L; ++l) {
-    if ((rc = gemm(B, M, D, W.r[l], D, 0, W_in[l], D, 1, W.hidc[l], M, 0.f))) return rc;
-    hipLaunchKernelGGL(k_rm_relu, dim3(rm_ew_blocks(B * M)), dim3(256), 0, s, W.hidc[l], B * M);
-    hipMemcpyAsync(W.r[l + 1], W.r[l], (size_t)B * D * sizeof(float), hipMemcpyDeviceToDevice, s);
-    if ((rc = gemm(B, D, M, W.hidc[l], M, 0, W_out[l], M, 1, W.r[l + 1], D, 1.f))) return rc;
-    if ((rc = gemm(B, C, D, W.r[l], D, 0, V[2 * l], C, 0, W.hg[2 * l], C, 0.f))) return rc;
-    if ((rc = gemm(B, C, M, W.hidc[l], M, 0, V[2 * l + 1], C, 0, W.hg[2 * l + 1], C, 0.f))) return rc;
+    if ((rc = two(prod(B, M, D, W.r[l], 0, W_in[l], 1, W.hidc[l], nullptr, 1),
+                  prod(B, C, D, W.r[l], 0, V[2 * l], 0, W.hg[2 * l]))))
+      return rc;
+    if ((rc = fused(prod(B, D, M, W.hidc[l], 0, W_out[l], 1, W.r[l + 1], W.r[l])))) return rc;
+    if ((rc = fused(prod(B, C, M, W.hidc[l], 0, V[2 * l + 1], 0, W.hg[2 * l + 1])))) return rc;
   }
-  if ((rc = gemm(B, F, D, W.r[L], D, 0, W_U, F, 0, W.clean, F, 0.f))) return rc;
 
   // ---- masked pass
   auto site_fwd = [&](int si) {
@@ -401,48 +467,79 @@ int pd_resid_mlp_step(int64_t B, int F, int D, int M, int C, int L, const float*
   };
   for (int l = 0; l < L; ++l) {
     const int si = 2 * l, so = 2 * l + 1;
-    if (l > 0 && (rc = gemm(B, C, D, W.rm[l], D, 0, V[si], C, 0, W.ha[si], C, 0.f))) return rc;
+    if (l > 0 && (rc = fused(prod(B, C, D, W.rm[l], 0, V[si], 0, W.ha[si])))) return rc;
     site_fwd(si);
-    if ((rc = gemm(B, M, C, W.acts[si], C, 0, U[si], M, 0, W.hid[l], M, 0.f))) return rc;
-    hipLaunchKernelGGL(k_rm_relu, dim3(rm_ew_blocks(B * M)), dim3(256), 0, s, W.hid[l], B * M);
-    if ((rc = gemm(B, C, M, W.hid[l], M, 0, V[so], C, 0, W.ha[so], C, 0.f))) return rc;
+    if ((rc = fused(prod(B, M, C, W.acts[si], 0, U[si], 0, W.hid[l], nullptr, 1)))) return rc;
+    if ((rc = fused(prod(B, C, M, W.hid[l], 0, V[so], 0, W.ha[so])))) return rc;
     site_fwd(so);
-    hipMemcpyAsync(W.rm[l + 1], W.rm[l], (size_t)B * D * sizeof(float), hipMemcpyDeviceToDevice, s);
-    if ((rc = gemm(B, D, C, W.acts[so], C, 0, U[so], D, 0, W.rm[l + 1], D, 1.f))) return rc;
+    if ((rc = fused(prod(B, D, C, W.acts[so], 0, U[so], 0, W.rm[l + 1], W.rm[l])))) return rc;
   }
-  if ((rc = gemm(B, F, D, W.rm[L], D, 0, W_U, F, 0, W.out, F, 0.f))) return rc;
+  // the target's output is first needed here, beside the masked one
+  if ((rc = two(prod(B, F, D, W.r[L], 0, W_U, 0, W.clean), prod(B, F, D, W.rm[L], 0, W_U, 0, W.out)))) return rc;
   const int64_t nout = B * F;
   hipLaunchKernelGGL(k_rm_recon, dim3(RM_REC_BLOCKS), dim3(256), 0, s, W.out, W.clean, nout,
                      recon_coeff * 2.f / (float)nout, W.d_out, W.rec_part);
   if ((rc = check_launch(what))) return rc;
 
   // ---- backward: d_r is the masked residual's cotangent
-  if ((rc = gemm(B, D, F, W.d_out, F, 0, W_U, F, 1, W.d_r, D, 0.f))) return rc;
+  if ((rc = fused(prod(B, D, F, W.d_out, 0, W_U, 1, W.d_r)))) return rc;
   const float imp_scale = imp_coeff / (float)B;
-  auto site_bwd = [&](int si, float* d_hg) {
+  auto site_bwd = [&](int si, float* d_ha, float* d_hg) {
     hipLaunchKernelGGL(k_rm_site_bwd, sgrid, dim3(RM_COLS * RM_WAVES), 0, s, W.d_acts, W.hg[si], W.ha[si], W.graw[si], B, C,
-                       gt[si], layout, p, imp_scale, W.d_ha, d_hg, W.gpart + (int64_t)si * Dm.chunks() * RM_GATE * C);
+                       gt[si], layout, p, imp_scale, d_ha, d_hg, W.gpart + (int64_t)si * Dm.chunks() * RM_GATE * C);
+  };
+  // A layer's weight gradients; q[i + 1] adds into q[i]'s output where both have the same C.
+  auto weight_grads = [&](const F32Prod* q, int n) {
+    F32Prod parts[F32_GROUP];
+    RmSums sums{};
+    int outs = 0;
+    int64_t total = 0;
+    float* part = W.wpart;
+    for (int i = 0; i < n; ++i) {
+      const int64_t mn = q[i].M * q[i].N;
+      parts[i] = q[i];
+      parts[i].C = part;
+      if (i == 0 || q[i].C != q[i - 1].C) {
+        sums.src[outs] = part;
+        sums.dst[outs] = q[i].C;
+        sums.n[outs] = mn;
+        sums.first[outs++] = total;
+        total += mn;
+      }
+      sums.slabs[outs - 1] += W.splits;
+      part += W.splits * mn;
+    }
+    sums.first[4] = total;
+    if (W.splits && gemm_f32_group(parts, n, W.splits, s)) {
+      hipLaunchKernelGGL(k_rm_sum_slabs, dim3((unsigned)cdiv(total, 256)), dim3(256), 0, s, sums);
+      return (int)PD_OK;
+    }
+    for (int i = 0; i < n; ++i)
+      if (int e = gemm(q[i].M, q[i].N, q[i].K, q[i].A, q[i].lda, 1, q[i].B, q[i].ldb, 0, q[i].C, q[i].ldc,
+                       i && q[i].C == q[i - 1].C ? 1.f : 0.f))
+        return e;
+    return (int)PD_OK;
   };
   for (int l = L - 1; l >= 0; --l) {
     const int si = 2 * l, so = 2 * l + 1;
     // mlp_out: its output adds into the residual
-    if ((rc = gemm(C, D, B, W.acts[so], C, 1, W.d_r, D, 0, grads + G.dU[so], D, 0.f))) return rc;
-    if ((rc = gemm(B, C, D, W.d_r, D, 0, U[so], D, 1, W.d_acts, C, 0.f))) return rc;
-    site_bwd(so, W.d_hg);
-    if ((rc = gemm(M, C, B, W.hid[l], M, 1, W.d_ha, C, 0, grads + G.dV[so], C, 0.f))) return rc;
-    if ((rc = gemm(M, C, B, W.hidc[l], M, 1, W.d_hg, C, 0, grads + G.dV[so], C, 1.f))) return rc;
-    if ((rc = gemm(B, M, C, W.d_ha, C, 0, V[so], C, 1, W.d_hid, M, 0.f))) return rc;
-    hipLaunchKernelGGL(k_rm_relu_bwd, dim3(rm_ew_blocks(B * M)), dim3(256), 0, s, W.d_hid, W.hid[l], B * M);
+    if ((rc = fused(prod(B, C, D, W.d_r, 0, U[so], 1, W.d_acts)))) return rc;
+    site_bwd(so, W.d_ha[1], W.d_hg[1]);
+    if ((rc = fused(prod(B, M, C, W.d_ha[1], 0, V[so], 1, W.d_hid, W.hid[l], 2)))) return rc;
     // mlp_in
-    if ((rc = gemm(C, M, B, W.acts[si], C, 1, W.d_hid, M, 0, grads + G.dU[si], M, 0.f))) return rc;
-    if ((rc = gemm(B, C, M, W.d_hid, M, 0, U[si], M, 1, W.d_acts, C, 0.f))) return rc;
+    if ((rc = fused(prod(B, C, M, W.d_hid, 0, U[si], 1, W.d_acts)))) return rc;
     const bool shared = W.ha[si] == W.hg[si];
-    site_bwd(si, shared ? W.d_ha : W.d_hg);
-    if ((rc = gemm(D, C, B, W.rm[l], D, 1, W.d_ha, C, 0, grads + G.dV[si], C, 0.f))) return rc;
-    if (!shared && (rc = gemm(D, C, B, W.r[l], D, 1, W.d_hg, C, 0, grads + G.dV[si], C, 1.f))) return rc;
+    site_bwd(si, W.d_ha[0], shared ? W.d_ha[0] : W.d_hg[0]);
+    const F32Prod dw[F32_GROUP] = {
+        prod(C, D, B, W.acts[so], 1, W.d_r, 0, grads + G.dU[so]),
+        prod(M, C, B, W.hid[l], 1, W.d_ha[1], 0, grads + G.dV[so]),
+        prod(M, C, B, W.hidc[l], 1, W.d_hg[1], 0, grads + G.dV[so]),
+        prod(C, M, B, W.acts[si], 1, W.d_hid, 0, grads + G.dU[si]),
+        prod(D, C, B, W.rm[l], 1, W.d_ha[0], 0, grads + G.dV[si]),
+        prod(D, C, B, W.r[l], 1, W.d_hg[0], 0, grads + G.dV[si])};
+    if ((rc = weight_grads(dw, shared ? 5 : 6))) return rc;
     if (l > 0) {  // the residual cotangent below this layer
-      hipMemcpyAsync(W.d_r2, W.d_r, (size_t)B * D * sizeof(float), hipMemcpyDeviceToDevice, s);
-      if ((rc = gemm(B, D, C, W.d_ha, C, 0, V[si], C, 1, W.d_r2, D, 1.f))) return rc;
+      if ((rc = fused(prod(B, D, C, W.d_ha[0], 0, V[si], 1, W.d_r2, W.d_r)))) return rc;
       std::swap(W.d_r, W.d_r2);
     }
   }
