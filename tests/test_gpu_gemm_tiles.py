@@ -57,3 +57,25 @@ def test_big_tile_two_segments(device, d_in, C):
     want = torch.where(route[:, None], acts @ U.float() + d.float()[:, None] * target, target)
     # the stored xV may round to the neighbouring bf16 value in another order of its sum
     assert _rel(out, want) < 4e-3
+
+
+@pytest.mark.parametrize("K", [768, 776, 1000, 1032])
+@pytest.mark.parametrize("M,N", [(1, 8), (300, 264), (2048, 2048)])
+def test_four_stage_ring(device, M, N, K):
+    a, b = _rand(device, 7, M, K), _rand(device, 8, N, K)
+    got = ops.gemm(a, b, trans_b=True, out_dtype=torch.float32)
+    # two fp32 sums of K terms in different orders, each within sqrt(K) 2^-24 = 1.9e-6
+    assert _rel(got, a.float() @ b.float().t()) < 4e-6
+
+
+@pytest.mark.parametrize("N", [1023, 1025, 1537, 3001])  # one slice, then a ragged last one
+def test_ci_mlp_sliced_weight_gradient(device, N):
+    dims = (72, 136, 64)
+    x, g = _rand(device, 9, N, dims[0]), _rand(device, 10, N, dims[2])
+    w = [_rand(device, 11 + i, dims[i], dims[i + 1]) for i in range(2)]
+    b = [torch.zeros(d, dtype=torch.bfloat16, device=device) for d in dims[1:]]
+    _, ws = ops.ci_mlp_fwd(x, w, b)
+    dW, _, _ = ops.ci_mlp_bwd(x, w, g, ws, True)
+    # the head's: the hidden activations round to bf16 from either order of their sum
+    a = torch.nn.functional.gelu((x.float() @ w[0].float()).to(torch.bfloat16).float()).to(torch.bfloat16).float()
+    assert _rel(dW[1], a.t() @ g.float()) < 4e-3
