@@ -388,10 +388,14 @@ __global__ __launch_bounds__(256) void k_kl_transpose(const bf16_t* __restrict__
   }
 }
 
-// Tiles of the fused passes: 128 positions x 256 vocab columns, 8 waves of 64x64. With one
-// head for both sides (a tied head, as in the LM step) a stage holds A | B | A2 and both
-// products share the head's fragments; two heads take one k loop after the other.
-typedef DtlCfg<128, 256, 2, 4, false> CfgKL;
+// Tiles of the fused passes: 128 positions x 256 vocab columns, 8 waves. With one head for
+// both sides (a tied head, as in the LM step) a stage holds A | B | A2 and both products
+// share the head's fragments; its waves are 32x128, so a position's statistics are two
+// sums of 128 columns. 64x64 waves read as many fragments per MFMA, but four sums of 64
+// columns move the last fp32 bits of logZ, which the LM step's bf16 backward amplifies to
+// 8e-3 of its q/k gradients. Two heads take one k loop after the other in waves of 64x64,
+// which read 4 fragments for 4 MFMAs where 32x128 reads 5.
+typedef DtlCfg<128, 256, 4, 2, false> CfgKL;
 typedef DtlCfg<128, 256, 2, 4, false, 3> CfgKLTwo;
 static int64_t kl_tiles(const KLChunks& K, int64_t V, int bn) {
   int64_t n = 0;
