@@ -502,15 +502,18 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_f32_group(F32Group g) {
   else f32_direct_tile<KW, TA, false>(p, bm, bn, kb, ke, g.bytes_a[i], g.bytes_b[i], g.vec[i], 1.f, beta, red);
 }
 
-// Bytes the operands span, and the floats per load of each (`vec` of f32_direct_tile).
+// Bytes the operands span (>= 0), and the floats per load of each (`vec` of f32_direct_tile).
 struct F32Span {
   int64_t a, b;
   int vec;
   bool fits;
 };
 static F32Span f32_span(const F32Prod& p, int64_t sA = 0, int64_t sB = 0) {
-  const int64_t ea = 4 * (p.ta ? (p.K - 1) * p.lda + p.M : (p.M - 1) * p.lda + p.K);
-  const int64_t eb = 4 * (p.tb ? (p.N - 1) * p.ldb + p.K : (p.K - 1) * p.ldb + p.N);
+  // no contraction reads nothing: the last-row formulas would be negative at K = 0 where a
+  // k-row is padded, and a negative record count is one past 2^31, inside which the loads'
+  // out-of-range offset lies
+  const int64_t ea = p.K == 0 ? 0 : 4 * (p.ta ? (p.K - 1) * p.lda + p.M : (p.M - 1) * p.lda + p.K);
+  const int64_t eb = p.K == 0 ? 0 : 4 * (p.tb ? (p.N - 1) * p.ldb + p.K : (p.K - 1) * p.ldb + p.N);
   auto width = [&](const float* x, int64_t ld, int64_t stride) {
     auto by = [&](int w) { return p.K % w == 0 && ld % w == 0 && stride % w == 0 && (uintptr_t)x % (4 * w) == 0; };
     return by(4) ? 4 : by(2) ? 2 : 1;

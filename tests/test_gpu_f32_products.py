@@ -39,6 +39,24 @@ def test_direct_form_load_widths(device, M, N, K, pad, shift):
             assert _rel(got, (a.t() if ta else a).double() @ (b.t() if tb else b).double()) < 3e-6, (ta, tb)
 
 
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_no_contraction(device, ta, tb, beta):
+    """K = 0 with padded rows leaves beta C, plain and batched, and reads neither operand."""
+    M, N, ld = 40, 33, 64
+    a, b = torch.ones(8, ld, device=device), torch.ones(8, ld, device=device)
+    for call, z in ((lambda c: L.call("pd_gemm", L.dtype_code(a.dtype), M, N, 0, L.ptr(a), ld, ta, L.ptr(b), ld, tb,
+                                      L.ptr(c), N, L.dtype_code(c.dtype), 1.0, beta, L.stream()), 1),
+                    (lambda c: L.call("pd_gemm_strided_batched", L.dtype_code(a.dtype), 2, M, N, 0, L.ptr(a), ld, ld,
+                                      ta, L.ptr(b), ld, ld, tb, L.ptr(c), N, M * N, L.dtype_code(c.dtype), 1.0, beta,
+                                      L.stream()), 2)):
+        c = torch.randn(z, M, N, device=device)
+        want = beta * c
+        call(c)
+        assert torch.equal(c, want)
+
+
 @pytest.mark.parametrize("B,F,D,M,C,n_layers", [(3, 20, 100, 10, 20, 2), (511, 33, 101, 13, 37, 2), (1030, 33, 102, 14, 36, 3),
                                          (64, 24, 1000, 20, 520, 1), (33000, 20, 300, 30, 20, 1)])
 def test_resid_mlp_step_product_forms(device, B, F, D, M, C, n_layers):
