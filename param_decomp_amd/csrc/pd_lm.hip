@@ -244,60 +244,66 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
     if (tid < TILE) srow[tid] = n0 + tid < a.N ? (int)((n0 + tid) / a.rps) : 0;
     __syncthreads();
   }
-  // the four passes' loads go out together
-  uint2 pws[4], hws[4];
-  float dts[4];
-  bool rts[4];
-  uint4 tws[LAYOUT == MASK_SRC ? 4 : 1];
-#pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
-    const int r = PD_LM_ROW(pass);
-    const int64_t n = n0 + r;
-    if (n < a.N && qok) {
-      const int64_t idx = n * a.C + q0 + q4;
-      pws[pass] = *(const uint2*)(a.ci_pre + idx);
-      hws[pass] = *(const uint2*)(xV + idx);
-      dts[pass] = a.delta ? a.delta[n] : 0.f;
-      rts[pass] = !a.route || a.route[n];
-      if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)srow[r] * a.C + q0 + q4);
-    }
-  }
+  // With a source table the four passes' loads go out together: they are the time. A draw is
+  // (draw_bits bounds the pass), and loads ahead of it only widen the wave: 32 registers
+  // against 57, 8192 x 4096 75 against 84 us, 1536 x 1024 9.6 against 10.4.
+  constexpr int AHEAD = LAYOUT == MASK_SRC ? 4 : 1;
   float imp = 0.f;
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
-    const int r = PD_LM_ROW(pass);
-    const int64_t n = n0 + r;
-    bf16_t o[4] = {0, 0, 0, 0};
-    if (n < a.N && qok) {
-      const int64_t idx = n * a.C + q0 + q4;
-      const float dt = dts[pass];
-      const bool routed = rts[pass];
-      const uint2 pw = pws[pass], hw = hws[pass];
-      const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
-      const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
-      float uv[4];
-      if constexpr (LAYOUT == MASK_SRC) src_quad_values(tws[pass], a.src_dtype, uv);
-      uint32_t ub = 0;
+  for (int first = 0; first < 4; first += AHEAD) {
+    uint2 pws[4], hws[4];
+    float dts[4];
+    bool rts[4];
+    uint4 tws[LAYOUT == MASK_SRC ? 4 : 1];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = lower_fwd(pre[e]);
-        if constexpr (PM == PM_SL0) SLv.ps[r][q4 + e] = sl0_psi(upper_fwd(pre[e]), a.g2, a.psis);
-        else imp += powp<PM>(upper_fwd(pre[e]), a.p);
-        float u;
-        if constexpr (LAYOUT == MASK_SRC) {
-          u = uv[e];
-        } else {
-          const uint32_t kb = (draw_bits(a.k0, a.k1, idx + e, total, 8, LAYOUT) & 0xFFu) >> 1;
-          ub |= kb << (8 * e);
-          u = (float)kb * (1.f / 128.f);
-        }
-        o[e] = routed ? f32_to_bf16(hv[e] * (lo + (1.f - lo) * u - dt)) : (bf16_t)0;
+    for (int pass = first; pass < first + AHEAD; ++pass) {
+      const int r = PD_LM_ROW(pass);
+      const int64_t n = n0 + r;
+      if (n < a.N && qok) {
+        const int64_t idx = n * a.C + q0 + q4;
+        pws[pass] = *(const uint2*)(a.ci_pre + idx);
+        hws[pass] = *(const uint2*)(xV + idx);
+        dts[pass] = a.delta ? a.delta[n] : 0.f;
+        rts[pass] = !a.route || a.route[n];
+        if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)srow[r] * a.C + q0 + q4);
       }
-      if constexpr (LAYOUT != MASK_SRC) *(uint32_t*)(ubits + idx) = ub;
-      *(uint2*)(acts + n * a.ld + q0 + q4) = make_uint2(bf_pack(o[0], o[1]), bf_pack(o[2], o[3]));
-    } else if constexpr (PM == PM_SL0) {
+    }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) SLv.ps[r][q4 + e] = 0.f;
+    for (int pass = first; pass < first + AHEAD; ++pass) {
+      const int r = PD_LM_ROW(pass);
+      const int64_t n = n0 + r;
+      bf16_t o[4] = {0, 0, 0, 0};
+      if (n < a.N && qok) {
+        const int64_t idx = n * a.C + q0 + q4;
+        const float dt = dts[pass];
+        const bool routed = rts[pass];
+        const uint2 pw = pws[pass], hw = hws[pass];
+        const float pre[4] = {bf_lo(pw.x), bf_hi(pw.x), bf_lo(pw.y), bf_hi(pw.y)};
+        const float hv[4] = {bf_lo(hw.x), bf_hi(hw.x), bf_lo(hw.y), bf_hi(hw.y)};
+        float uv[4];
+        if constexpr (LAYOUT == MASK_SRC) src_quad_values(tws[pass], a.src_dtype, uv);
+        uint32_t ub = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = lower_fwd(pre[e]);
+          if constexpr (PM == PM_SL0) SLv.ps[r][q4 + e] = sl0_psi(upper_fwd(pre[e]), a.g2, a.psis);
+          else imp += powp<PM>(upper_fwd(pre[e]), a.p);
+          float u;
+          if constexpr (LAYOUT == MASK_SRC) {
+            u = uv[e];
+          } else {
+            const uint32_t kb = (draw_bits(a.k0, a.k1, idx + e, total, 8, LAYOUT) & 0xFFu) >> 1;
+            ub |= kb << (8 * e);
+            u = (float)kb * (1.f / 128.f);
+          }
+          o[e] = routed ? f32_to_bf16(hv[e] * (lo + (1.f - lo) * u - dt)) : (bf16_t)0;
+        }
+        if constexpr (LAYOUT != MASK_SRC) *(uint32_t*)(ubits + idx) = ub;
+        *(uint2*)(acts + n * a.ld + q0 + q4) = make_uint2(bf_pack(o[0], o[1]), bf_pack(o[2], o[3]));
+      } else if constexpr (PM == PM_SL0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) SLv.ps[r][q4 + e] = 0.f;
+      }
     }
   }
   if constexpr (PM == PM_SL0) {
@@ -331,15 +337,18 @@ __global__ __launch_bounds__(256) void k_lm_mask_bwd(LMMaskArgs a, const bf16_t*
     if (tid < 64) SG.grp[tid] = n0 + tid < a.N ? (int)((n0 + tid) / a.rps) : -1;  // each row's source row
     __syncthreads();
   }
-  // the loads of two passes go out together (of all four: half the waves, and slower)
+  // With a source table the loads of two passes go out together (of all four: half the waves,
+  // and slower); without one a pass's loads are few, and two passes' held 51 registers
+  // against 35: 8192 x 1024 23.7 against 26.9 us, 8192 x 4096 69.8 against 68.4.
+  constexpr int AHEAD = SRC ? 2 : 1;
 #pragma unroll
-  for (int half = 0; half < 4; half += 2) {
+  for (int first = 0; first < 4; first += AHEAD) {
     uint2 pws[4], hws[4], dws[4];
     uint32_t ubs[4];
     float dts[4];
     uint4 tws[SRC ? 4 : 1];
 #pragma unroll
-    for (int pass = half; pass < half + 2; ++pass) {
+    for (int pass = first; pass < first + AHEAD; ++pass) {
       const int r = PD_LM_ROW(pass);
       const int64_t n = n0 + r;
       if (n < a.N && qok) {
@@ -353,7 +362,7 @@ __global__ __launch_bounds__(256) void k_lm_mask_bwd(LMMaskArgs a, const bf16_t*
       }
     }
 #pragma unroll
-    for (int pass = half; pass < half + 2; ++pass) {
+    for (int pass = first; pass < first + AHEAD; ++pass) {
       const int r = PD_LM_ROW(pass);
       const int64_t n = n0 + r;
       bf16_t o[4] = {0, 0, 0, 0};
