@@ -340,13 +340,16 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // the hardware returns as 0. Behind a branch the compiler has to assume that the loads were
 // not issued and waits for every load in flight before each batch's MFMAs. F32_AHEAD batches
 // are in flight: these launches hold one or two blocks per CU, so the load latency is what
-// bounds them, and a fourth batch spills at 16 waves per block (128 registers).
+// bounds them; a third batch was slower (104 registers against 75, so two blocks of 8 waves
+// per CU against three): ResidualMLP step 222 against 210 us, 895x961x1521 with both
+// transposed 81 against 76. A contraction of one or two batches per wave issues just those:
+// loads past its range cost the address unit as much as data.
 // Block forms as in k_gemm_f32 (KW waves splitting the contraction of a 32x32 tile, or 4
 // waves of a 64x64 tile); the summation order is fixed. Each operand must span fewer than
 // 2^31 bytes (checked on the host). 2048x1000 over 50, both K-contiguous at row stride 50,
-// 17.6 us in dword loads (and a 3.6 us copy before it), 14.5 in 8-byte
-// loads; the whole residual-MLP step 296 -> 223 us with the grouped launches below.
-constexpr int F32_AHEAD = 3;
+// 17.6 us in dword loads (and a 3.6 us copy before it), 14.5 in 8-byte loads; the whole
+// residual-MLP step 296 -> 210 us with the grouped launches below.
+constexpr int F32_AHEAD = 2;
 
 template <int KW, bool TA, bool TB>
 __device__ inline void f32_direct_tile(const F32Prod& p, int bm, int bn, int kbeg, int kend, int32_t bytes_a,
@@ -408,16 +411,32 @@ __device__ inline void f32_direct_tile(const F32Prod& p, int bm, int bn, int kbe
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
   auto contract = [&](auto wa, auto wb) {
     float a[D][S], b[D][S];
+    auto mfma = [&](int d) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][s], b[d][s], acc, 0, 0, 0);
+    };
+    if (ke - kb <= 2 * FK) {  // at most two batches: both in flight, none past the range
+      if (kb >= ke) return;
+      load(wa, wb, a[0], b[0], kb);
+      if (ke - kb > FK) load(wa, wb, a[1], b[1], kb + FK);
+      mfma(0);
+      if (ke - kb > FK) mfma(1);
+      return;
+    }
 #pragma unroll
     for (int d = 0; d < D; ++d) load(wa, wb, a[d], b[d], kb + d * FK);
-    for (int kc = kb; kc < ke; kc += D * FK) {
+    int kc = kb;
+    for (; kc + D * FK < ke; kc += D * FK) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        if (kc + d * FK >= ke) return;
-#pragma unroll
-        for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][s], b[d][s], acc, 0, 0, 0);
+        mfma(d);
         load(wa, wb, a[d], b[d], kc + (d + D) * FK);
       }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (kc + d * FK >= ke) return;
+      mfma(d);
     }
   };
   typedef std::integral_constant<int, 1> W1;

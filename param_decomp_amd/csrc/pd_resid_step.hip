@@ -17,7 +17,7 @@
 // squashing and gate pullbacks, gate-parameter partials) another; the partials are added
 // over row chunks in a fixed order. Relus and residual sums are the products' epilogues,
 // independent small products share a launch. At the 1-layer benchmark shape (2048 x 1000, C =
-// 100) that is 22 launches and 223 us per step (31 and 296 with one launch per product, relu,
+// 100) that is 22 launches and 210 us per step (31 and 296 with one launch per product, relu,
 // copy and weight gradient), against about 90 launches for the same step composed from the
 // library's primitives.
 #include <algorithm>

@@ -11,7 +11,7 @@ of each gradient's norm (the bound of the oracle comparison)."""
 import pytest
 import torch
 
-from param_decomp_amd import _lib as L, toys
+from param_decomp_amd import _lib as L, ops, toys
 
 pytestmark = pytest.mark.gpu
 
@@ -36,6 +36,20 @@ def test_direct_form_load_widths(device, M, N, K, pad, shift):
             got = torch.empty(M, N, device=device)
             L.call("pd_gemm", L.dtype_code(a.dtype), M, N, K, a.data_ptr(), a.stride(0), int(ta), b.data_ptr(),
                    b.stride(0), int(tb), L.ptr(got), N, L.dtype_code(got.dtype), 1.0, 0.0, L.stream())
+            assert _rel(got, (a.t() if ta else a).double() @ (b.t() if tb else b).double()) < 3e-6, (ta, tb)
+
+
+# one to five 16-deep batches per wave and none, whole and ragged, in blocks of 8 and 16 waves
+# (70 x 40) and of one wave per tile (2048 x 1024)
+@pytest.mark.parametrize("M,N,K", [(70, 40, k) for k in (16, 31, 130, 256, 257, 300, 384, 511, 512, 700, 1100, 1300)] +
+                         [(2048, 1024, k) for k in (5, 16, 33, 48, 64, 250)])
+def test_direct_form_batches(device, M, N, K):
+    g = torch.Generator(device=device).manual_seed(K)
+    for ta in (False, True):
+        for tb in (False, True):
+            a = torch.randn(*((K, M) if ta else (M, K)), device=device, generator=g)
+            b = torch.randn(*((N, K) if tb else (K, N)), device=device, generator=g)
+            got = ops.gemm(a, b, trans_a=ta, trans_b=tb, out_dtype=torch.float32)
             assert _rel(got, (a.t() if ta else a).double() @ (b.t() if tb else b).double()) < 3e-6, (ta, tb)
 
 
