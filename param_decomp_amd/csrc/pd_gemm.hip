@@ -698,7 +698,7 @@ static int launch_dtl_any(const GemmArgs& a, bool a_kmaj, bool b_kmaj, int c_dty
       if (big) return launch_dtl<CfgDtlBig, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);            \
     if constexpr (MODE == MODE_DENSE && !(AMN) && !(BMN))                                           \
       if (deep_ring(a.M, a.N, a.K)) return launch_dtl<CfgDtlDeep, MODE>(a, c_dtype, kedge, grid, s); \
-    return launch_dtl<CfgDtlSmall<AMN, BMN>, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);           \
+    return launch_dtl<CfgDtlSmall<MODE, AMN, BMN>, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);     \
   }
   if (a_kmaj && b_kmaj) PD_L(false, false)
   if (a_kmaj) PD_L(false, true)
@@ -808,7 +808,7 @@ int grouped_gemm(const void* lhs, const void* rhs, const int32_t* offsets, int64
     if (big_tiles_grouped(J, E, N))
       return launch_dtl<CfgDtlBig, MODE_GROUPED>(a, out_dtype, kedge,
                                                  dim3((unsigned)cdiv(N, 256), (unsigned)(cdiv(J, 256) + E)), s);
-    return launch_dtl<CfgDtlRA, MODE_GROUPED>(a, out_dtype, kedge, grid, s);
+    return launch_dtl<CfgDtl, MODE_GROUPED>(a, out_dtype, kedge, grid, s);
   }
   if (!b_kmaj && dtl_fits(J, K, 0, 0) && dtl_fits_mn(K, N))  // each expert's rhs stored [K][N]
     return launch_dtl<CfgDtl, MODE_GROUPED, false, true>(a, out_dtype, kedge, grid, s);

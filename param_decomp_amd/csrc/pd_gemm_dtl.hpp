@@ -348,26 +348,41 @@ inline bool deep_ring(int64_t M, int64_t N, int64_t K) {
 }
 // 256x256x64 tiles, 8 waves (128 KB of LDS, one block per CU): fewer LDS bytes per MFMA.
 typedef DtlCfg<256, 256, 2, 4, true> CfgDtlBig;
-template <bool AMN, bool BMN>
-using CfgDtlSmall = std::conditional_t<AMN || BMN, CfgDtl, CfgDtlRA>;
+// The small tile of a launch: 4 waves where both operands are K-major and one product fills
+// the grid, 8 elsewhere (batches and ragged groups of few rows: 53 x 712x64x208 9.0 against
+// 9.9 us, 8 groups of 53 rows over 248 6.6 against 7.2).
+template <int MODE, bool AMN, bool BMN>
+using CfgDtlSmall = std::conditional_t<AMN || BMN || MODE == MODE_BATCHED, CfgDtl, CfgDtlRA>;
 
-// Whether `rows` x N outputs take 256x256 tiles (one block per CU) rather than 128x128 (two
-// per CU): by the rounds of 256 big or 512 small tiles, a partial round costing 0.8 + 0.2 of
-// its fill and a round of small tiles 0.64 of a round of big ones (half the products at 0.8
-// of the rate). Big against small, us: 192 big tiles (4096x3072x4096) 101 / 117, 384
-// (8192x3072x4864) 238 / 248, 512 (65536x512x512) 46 / 60, 256 (65536x256x512) 28 / 31; 128
-// (8192x1024x768) 21.7 / 17.6, 48 (768x4096x4096) 91 / 51. Grouped rows: J plus half a tile
-// per group for the groups' ragged ends.
-inline bool big_tiles(int64_t rows, int64_t N, int64_t problems = 1) {
+// Whether an output takes `big` 256x256 tiles (one block per CU) rather than `small` 128x128
+// ones (two per CU): by the rounds of 256 big or 512 small tiles, a partial round costing
+// 0.8 + 0.2 of its fill and a round of small tiles 0.64 of a round of big ones (half the
+// products at 0.8 of the rate). Big against small, us: 192 big tiles (4096x3072x4096) 101 /
+// 117, 384 (8192x3072x4864) 238 / 248, 512 (65536x512x512) 46 / 60, 256 (65536x256x512) 28 /
+// 31; 128 (8192x1024x768) 21.7 / 17.6, 48 (768x4096x4096) 91 / 51.
+inline bool big_rounds(int64_t big, int64_t small) {
   auto rounds = [](int64_t tiles, int64_t cap) {  // in fifths
     const int64_t full = tiles / cap, rem = tiles % cap;
     return 5.0 * full + (rem ? 4.0 + (double)rem / cap : 0.0);
   };
-  auto up = [](int64_t x, int64_t n) { return (x + n - 1) / n; };
-  return rounds(problems * up(rows, 256) * up(N, 256), 256) <= 0.64 * rounds(problems * up(rows, 128) * up(N, 128), 512);
+  return rounds(big, 256) <= 0.64 * rounds(small, 512);
 }
-inline bool big_tiles_grouped(int64_t J, int E, int64_t N, int64_t problems = 1) {
-  return big_tiles(J + (int64_t)E * 128, N, problems);
+inline int64_t tiles_up(int64_t x, int64_t n) { return (x + n - 1) / n; }
+inline bool big_tiles(int64_t rows, int64_t N) {
+  return big_rounds(tiles_up(rows, 256) * tiles_up(N, 256), tiles_up(rows, 128) * tiles_up(N, 128));
+}
+// The same for J rows in E groups whose sizes only the device knows: the rows' tiles plus
+// half a tile per group for the ragged ends, and at least one per group (of any size: small
+// groups are what a big tile wastes most on). Big against small, us: 1352 rows in 128 groups
+// over 440 (N = 528) 34 / 23, 560 in 128 over 96 (N = 1528) 29 / 21, 50664 in 32 over 144 (N =
+// 1968) 81 / 92.
+inline bool big_tiles_grouped(int64_t J, int64_t E, int64_t N, int64_t problems = 1) {
+  const int64_t groups = E < J ? E : J;
+  auto tiles = [&](int64_t t) {
+    const int64_t rows = tiles_up(J + groups * (t / 2), t);
+    return problems * (rows > groups ? rows : groups) * tiles_up(N, t);
+  };
+  return big_rounds(tiles(256), tiles(128));
 }
 
 // The kernel addresses each operand through a 31-bit buffer record count (rows = M or N

@@ -44,6 +44,18 @@ def test_big_tile_groups(device, sizes, K):
     assert _rel(got, want) < 2e-3
 
 
+@pytest.mark.parametrize("trans_rhs", [True, False])
+@pytest.mark.parametrize("K", [72, 512])
+def test_groups_of_few_rows(device, K, trans_rhs):
+    sizes, N = [3, 0, 1, 130, 17, 0, 128, 64], 264
+    offs = torch.tensor([0] + sizes, device=device).cumsum(0).to(torch.int32)
+    lhs, rhs = _rand(device, 3, sum(sizes), K), _rand(device, 4, len(sizes), *((N, K) if trans_rhs else (K, N)))
+    got = ops.grouped_gemm(lhs, rhs, offs, trans_rhs=trans_rhs)
+    want = torch.cat([x.float() @ (rhs[e].float().t() if trans_rhs else rhs[e].float())
+                      for e, x in enumerate(lhs.split(sizes))])
+    assert _rel(got, want) < 2e-3
+
+
 @pytest.mark.parametrize("d_in,C", [(200, 136), (64, 72), (8, 128)])
 def test_big_tile_two_segments(device, d_in, C):
     T, d_out = 4000, 3072
