@@ -90,7 +90,7 @@ struct F32Prod {
   int32_t post;
 };
 // The product through the direct form, or false (nothing launched) where pd_gemm would take
-// another form.
+// another form or refuse it.
 bool gemm_f32_direct(const F32Prod& p, hipStream_t s);
 // Up to F32_GROUP products with one `ta` in one launch, for outputs too small to fill the
 // GPU alone. splits > 1 cuts every contraction into that many slices, each written to its

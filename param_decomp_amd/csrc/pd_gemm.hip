@@ -594,6 +594,7 @@ static void launch_gemm_f32(int64_t batch, int64_t M, int64_t N, int64_t K, cons
 }
 
 bool gemm_f32_direct(const F32Prod& p, hipStream_t s) {
+  if (cdiv(p.M, FT) > 65535 || cdiv(p.N, FT) > 65535) return false;  // pd_gemm refuses it
   const float beta = p.Cin && p.post < 2 ? 1.f : 0.f;
   if (p.ta) return p.tb ? launch_f32_direct<true, true>(p, 1, 1.f, beta, 0, 0, 0, s)
                         : launch_f32_direct<true, false>(p, 1, 1.f, beta, 0, 0, 0, s);

@@ -89,3 +89,20 @@ def test_host_prng_matches_oracle():
         assert prng.split(k, 4, partitionable=False) == tf.split(tf.prng_key(seed), 4, partitionable=False)
         assert prng.fold_in(k, 12) == tf.fold_in(tf.prng_key(seed), 12)
         assert prng.threefry2x32((0, 0), 0, 0) == (0x6B200159, 0x99BA4EFE)
+
+
+def test_resid_mlp_step_refuses_more_rows_than_a_product_takes():
+    """2.1M rows are more 32-row tiles than a product's grid holds: refused by the first
+    product, before anything is launched (the operands are never read)."""
+    import numpy as np
+
+    from param_decomp_amd import _lib as L
+
+    if not os.path.exists(L.LIB_PATH):
+        pytest.skip("HIP library not built")
+    B, w = 32 * 65535 + 1, 8
+    buf = np.zeros(64, np.float32).ctypes.data
+    ptrs = (ctypes.c_void_p * 8)(*[buf] * 8)
+    with pytest.raises(L.PDError, match="too large"):
+        L.call("pd_resid_mlp_step", B, w, w, w, w, 1, buf, buf, buf, ptrs, ptrs, ptrs, ptrs, ptrs, 0, 0, 1, 1.0, 1.0,
+               1.0, buf, buf, None, buf, 2**62, None)
