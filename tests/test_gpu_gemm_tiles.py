@@ -91,3 +91,29 @@ def test_ci_mlp_sliced_weight_gradient(device, N):
     # the head's: the hidden activations round to bf16 from either order of their sum
     a = torch.nn.functional.gelu((x.float() @ w[0].float()).to(torch.bfloat16).float()).to(torch.bfloat16).float()
     assert _rel(dW[1], a.t() @ g.float()) < 4e-3
+
+
+def _gelu_grad(z):
+    return 0.5 * (1 + torch.erf(z * 0.5**0.5)) + z * torch.exp(-0.5 * z * z) * (2 * torch.pi)**-0.5
+
+
+# 256x256 tiles with ragged edges in both directions (hidden layer, head and the pullback into
+# the hidden layer); the four-stage ring with a k tail in the backward, with and without GELU'
+@pytest.mark.parametrize("N,dims", [(3000, (72, 4104, 4104)), (300, (72, 776, 840))])
+def test_ci_mlp_tiles(device, N, dims):
+    x, g = _rand(device, 20, N, dims[0]), _rand(device, 21, N, dims[2])
+    w = [(_rand(device, 22 + i, dims[i], dims[i + 1]).float() / dims[i]**0.5).to(torch.bfloat16) for i in range(2)]
+    b = [_rand(device, 24 + i, dims[i + 1]) for i in range(2)]
+    pre, ws = ops.ci_mlp_fwd(x, w, b)
+    dW, db, dx = ops.ci_mlp_bwd(x, w, g, ws, True)
+    r = lambda t: t.to(torch.bfloat16).float()  # noqa: E731
+    wf, gf = [t.float() for t in w], g.float()
+    z = r(r(x.float() @ wf[0]) + b[0].float())
+    a = r(torch.nn.functional.gelu(z))
+    dz = r(r(gf @ wf[1].t()) * _gelu_grad(z))
+    want = dict(pre=r(r(a @ wf[1]) + b[1].float()), dx=r(dz @ wf[0].t()), dW0=x.float().t() @ dz, dW1=a.t() @ gf,
+                db0=dz.sum(0), db1=gf.sum(0))
+    got = dict(pre=pre, dx=dx, dW0=dW[0], dW1=dW[1], db0=db[0], db1=db[1])
+    # values rounded to bf16 on the way may take the neighbour in another order of their sum
+    for k in want:
+        assert _rel(got[k], want[k]) < 4e-3, k

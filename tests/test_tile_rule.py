@@ -40,13 +40,18 @@ def rule(tmp_path_factory):
     (65536, 42, 512, 2, "big"), (50664, 32, 1968, 1, "big"),
     # few rows per group: a tile per group whatever its size
     (1352, 128, 528, 1, "small"), (560, 128, 1528, 1, "small"), (248, 64, 1312, 1, "small"), (40, 128, 4096, 1, "small"),
-    (20578, 5, 520, 1, "big"), (20196, 5, 520, 1, "big")])  # the group sizes of the GPU test
+    # the group sizes of the GPU tests
+    (20578, 5, 520, 1, "big"), (20196, 5, 520, 1, "big"), (8192, 42, 512, 2, "big"), (343, 8, 264, 1, "small")])
 def test_grouped_tiles(rule, J, E, N, problems, tile):
     assert rule("grouped", J, E, N, problems) == tile
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
     (4096, 3072, 4096, "big"), (8192, 1024, 768, "small"), (768, 4096, 4096, "deep"), (3001, 768, 4096, "deep"),
-    (3000, 4104, 320, "big"), (4000, 3072, 200, "big"), (2048, 2048, 768, "deep"), (2048, 2048, 760, "small")])
+    (3000, 4104, 320, "big"), (4000, 3072, 200, "big"), (2048, 2048, 768, "deep"), (2048, 2048, 760, "small"),
+    (4096, 3072, 768, "big"), (4096, 4096, 776, "big"), (4000, 4104, 200, "small"),
+    # the CI MLP's: hidden layer, head and pullback; the pullback and the input gradient
+    (3000, 4104, 72, "big"), (3000, 4104, 4104, "big"), (3000, 72, 4104, "deep"), (300, 776, 840, "deep"),
+    (300, 72, 776, "deep")])
 def test_dense_tiles(rule, M, N, K, tile):
     assert rule("dense", M, N, K) == tile
