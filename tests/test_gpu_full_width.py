@@ -5,8 +5,9 @@ those workloads select is compared against the oracle, not only checked for fini
   256x256 grouped tiles of the N=512 component products (`grouped_gemm_pair`) and of
   every paired weight gradient (`grouped_gemm_dw_kmajor_pair`), K=512 main loops over
   several k stages, and ragged per-expert contraction lengths;
-- the dense products' 256x256 buffer-fed tile (`CfgDtlBig`, taken once the grid has >= 256
-  such tiles) in every operand layout, and the 128x128 one just below that size;
+- the dense products' 256x256 buffer-fed tile (`CfgDtlBig`, taken by the rounds of big and
+  small tiles an output needs) in every operand layout, and the 128x128 one at a size
+  whose last big tiles would take a round of their own;
 - the public grouped products at K = N = 512 with ragged and empty groups;
 - the LM stack at the Llama-4L widths (the streamed KL's dual products at V = 50277) and
   the dense step at 768 -> 3072, C = 4096.
@@ -97,13 +98,13 @@ def test_moe_stack_step_full_width_matches_oracle(device):
 @pytest.mark.parametrize("M,N,K", [(4096, 3072, 768), (4096, 4096, 776), (4000, 4104, 200)])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_gemm_big_tile_layouts(device, ta, tb, M, N, K):
-    """The dense site's shapes in every operand layout: 192 256x256 tiles stay on the
-    128x128 buffer-fed kernel; >= 256 (one per CU) select the 256x256 one, here with a
-    k-tail stage and ragged M and N edges. fp32 output within fp32 accumulation-order
-    error of a float64 product; bf16 output within bf16 rounding."""
+    """The dense site's shapes in every operand layout. 192 and 256 256x256 tiles (one
+    round, the second with a k-tail stage) take the 256x256 buffer-fed kernel; 272 would
+    start a second round and take the 128x128 one, here with ragged M and N edges and a
+    k tail (test_tile_rule.py asks the rule itself). fp32 output within fp32
+    accumulation-order error of a float64 product; bf16 output within bf16 rounding."""
     from param_decomp_amd import ops
 
-    assert -(-M // 256) * -(-N // 256) >= 192
     rng = np.random.default_rng(M + N + K + 2 * ta + tb)
     A = _bf(rng.normal(size=(K, M) if ta else (M, K)), device)
     B = _bf(rng.normal(size=(N, K) if tb else (K, N)), device)
