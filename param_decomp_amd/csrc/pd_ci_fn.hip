@@ -5,11 +5,12 @@
 // preactivations of a site are L_n(GELU(... GELU(L_1(x)))), L_i(a) = a @ W_i + b_i with
 // W_i stored [d_i, d_i+1] and exact-erf GELU, in bf16 compute with fp32 accumulation:
 // every product is rounded to bf16, the bias is added to that bf16 value and rounded,
-// and GELU's output is rounded. The forward GEMMs run on W_i^T copies (both operands
-// K-contiguous) with the bias and GELU in the epilogue, saving z_i (pre-GELU) and
-// a_i = GELU(z_i) in the workspace. The backward runs d_a = d_z @ W_i^T with
-// d_z_prev = bf16(d_a * GELU'(z_prev)) in the epilogue, dW_i = a_i-1^T @ d_z_i on
-// K-contiguous copies, and db_i as a two-phase fixed-order column sum.
+// and GELU's output is rounded. Every product reads its operands as stored. The forward
+// GEMMs have the bias and GELU in the epilogue and save z_i (pre-GELU) and a_i = GELU(z_i)
+// in the workspace; a weight past the kernel's 31-bit range goes through a transposed copy.
+// The backward runs d_a = d_z @ W_i^T with d_z_prev = bf16(d_a * GELU'(z_prev)) in the
+// epilogue, dW_i = a_i-1^T @ d_z_i in contraction slices where its tiles leave CUs idle,
+// and db_i as a two-phase fixed-order column sum.
 //
 // Component-activation readout (pd/core/ci_fn/implementations/transformer/
 // component_conditioning.py:215-245): per component, s+ sig(a+ h + b+) + s- sig(a- (-h) +

@@ -335,7 +335,7 @@ __device__ inline void gate_weights_load(int64_t c, const float* __restrict__ w_
 }
 
 // The exact gate of a flagged component (device erff/expf GELU) from its weights at stride
-// st, shared by both binned passes: returns g, sets gp = dg/dh and go[j] = (GELU,
+// st, in the binned forward and the flagged components' backward: returns g, sets gp = dg/dh and go[j] = (GELU,
 // GELU')(z_j).
 __device__ inline float gate_exact(const float* w, int st, float hv, GeluOut* go, float& gp) {
   float g = w[48 * st];
@@ -349,11 +349,6 @@ __device__ inline float gate_exact(const float* w, int st, float hv, GeluOut* go
   }
   return g;
 }
-
-// Moment slot q = 8 mb + m of lane l in a wave's region: float4 (2 mb + m / 4) of lane l,
-// component m % 4 (lane-contiguous 16-byte slots, so a wave's accesses are conflict-free
-// whatever the lanes' bins).
-__device__ inline int mom_index(int q, int lane) { return (((q >> 3) * 2 + ((q >> 2) & 1)) * 64 + lane) * 4 + (q & 3); }
 
 // The bf16 forward with the binned gate: block = 64 components x (FWD_WAVES * 64) tokens;
 // the 64 components' tables sit in LDS as lt[2b + half][lane] (16-byte slots, so a wave's
@@ -531,8 +526,10 @@ __global__ __launch_bounds__(SITE_COLS) void k_step_bwd(const T* __restrict__ da
 // 2w + l / 32 (BWD_ROWS consecutive tokens). Per element: g and dg/dh from the table,
 // the squashing pullback dg, dh = da (m - d) + dg g'
 // written token-major, and dg T_m(tau_m), m < 8, added into the lane's own LDS slots of its
-// moment bin mb (two 16-byte read-add-writes; one writer per slot and LDS operations of a
-// wave run in order, so the sums are deterministic). A flagged component's lanes do
+// moment bin mb (slot q = 8 mb + m of lane l is component m % 4 of float4 2 mb + m / 4 of
+// lane l: 16-byte slots side by side over the lanes, so a wave's accesses are conflict-free
+// whatever its bins; two read-add-writes; one writer per slot and LDS operations of a wave
+// run in order, so the sums are deterministic). A flagged component's lanes do
 // nothing (k_step_bwd_exact). The block then adds its 8 streams per slot in a fixed
 // order: partial[row block][q][c], q < GATE_MOM. LDS: the 32 components' tables (32 KB) and the 4 waves'
 // slots (128 KB).

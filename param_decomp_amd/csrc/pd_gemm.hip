@@ -1,9 +1,9 @@
 // GEMM kernels for the masked-component path (gfx950), v_mfma_f32_32x32x16_bf16.
 //
 // bf16 products run on the buffer-fed kernel of pd_gemm_dtl.hpp in every operand layout
-// (an MN-contiguous operand is transposed on its way out of LDS): 128x128x64 tiles, 8
-// waves of 32x64, two stages, two blocks per CU; 256x256 tiles (one block per CU) once the
-// grid has at least 256 of them.
+// (an MN-contiguous operand is transposed on its way out of LDS): 128x128x64 tiles in 4 or
+// 8 waves, two blocks per CU, or 256x256 tiles, one block per CU, by the rounds of each an
+// output takes (`big_tiles`).
 //
 // Operands beyond the buffer kernel's 31-bit addressing: the register-staged kernel
 // below. LDS holds both operands

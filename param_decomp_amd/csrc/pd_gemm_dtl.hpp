@@ -13,13 +13,14 @@
 // record count ends at the operand's last row, so rows past the operand extent, and
 // chunks past the end of its last row, load as zeros; their outputs are never stored.
 //
-// Two (or four) LDS stages, software-pipelined inside a wave (pipe_stage). A stage is four k16 steps;
-// the fragments of step n+1 are read from LDS between the MFMAs of step n (two register
-// sets), and the last step of a stage reads the first fragments of the next one, after the
-// one barrier of the stage: this wave's loads of the next stage have landed (vmcnt) and
-// its reads of this stage are done (lgkmcnt), so behind the barrier the next stage is
-// visible and this one's space is free. The loads of stage kt+2 go out in two halves,
-// between the MFMAs of stage kt's last step and of stage kt+1's first step. The order is
+// A ring of NS LDS stages (two, three or four), software-pipelined inside a wave
+// (pipe_stage). A stage is four k16 steps; the fragments of step n+1 are read from LDS
+// between the MFMAs of step n (two register sets), and the last step of a stage reads the
+// first fragments of the next one, after the one barrier of the stage: this wave's loads of
+// the next stage have landed (vmcnt) and its reads of this stage are done (lgkmcnt), so
+// behind the barrier the next stage is visible and this one's space is free. The loads of
+// stage kt+NS go out between the MFMAs of stage kt's last step; with SPLIT (256x256 tiles,
+// two stages) half of them between those of stage kt+1's first step. The order is
 // pinned by scheduling barriers: left to itself the compiler reads a step's fragments into
 // the registers of the step before, after its MFMAs, so a wave alternates between waiting
 // for LDS and computing. Same products, same k order, so the same bits as the unpipelined
