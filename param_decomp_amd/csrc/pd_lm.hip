@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
   }
   // With a source table the four passes' loads go out together: they are the time. A draw is
   // (draw_bits bounds the pass), and loads ahead of it only widen the wave: 32 registers
-  // against 57, 8192 x 4096 75 against 84 us, 1536 x 1024 9.6 against 10.4.
+  // against 57, alone 8192 x 4096 74 against 81 us, 2048 x 1024 10.3 against 11.5.
   constexpr int AHEAD = LAYOUT == MASK_SRC ? 4 : 1;
   float imp = 0.f;
 #pragma unroll
@@ -255,18 +255,20 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
     float dts[4];
     bool rts[4];
     uint4 tws[LAYOUT == MASK_SRC ? 4 : 1];
-#pragma unroll
-    for (int pass = first; pass < first + AHEAD; ++pass) {
+    auto load = [&](int pass) {
       const int r = PD_LM_ROW(pass);
       const int64_t n = n0 + r;
-      if (n < a.N && qok) {
-        const int64_t idx = n * a.C + q0 + q4;
-        pws[pass] = *(const uint2*)(a.ci_pre + idx);
-        hws[pass] = *(const uint2*)(xV + idx);
-        dts[pass] = a.delta ? a.delta[n] : 0.f;
-        rts[pass] = !a.route || a.route[n];
-        if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)srow[r] * a.C + q0 + q4);
-      }
+      const int64_t idx = n * a.C + q0 + q4;
+      dts[pass] = a.delta ? a.delta[n] : 0.f;
+      rts[pass] = !a.route || a.route[n];
+      pws[pass] = *(const uint2*)(a.ci_pre + idx);
+      hws[pass] = *(const uint2*)(xV + idx);
+      if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)srow[r] * a.C + q0 + q4);
+    };
+    if constexpr (AHEAD > 1) {
+#pragma unroll
+      for (int pass = first; pass < first + AHEAD; ++pass)
+        if (n0 + PD_LM_ROW(pass) < a.N && qok) load(pass);
     }
 #pragma unroll
     for (int pass = first; pass < first + AHEAD; ++pass) {
@@ -274,6 +276,7 @@ __global__ __launch_bounds__(256) void k_lm_mask_fwd(LMMaskArgs a, const bf16_t*
       const int64_t n = n0 + r;
       bf16_t o[4] = {0, 0, 0, 0};
       if (n < a.N && qok) {
+        if constexpr (AHEAD == 1) load(pass);
         const int64_t idx = n * a.C + q0 + q4;
         const float dt = dts[pass];
         const bool routed = rts[pass];
@@ -338,8 +341,8 @@ __global__ __launch_bounds__(256) void k_lm_mask_bwd(LMMaskArgs a, const bf16_t*
     __syncthreads();
   }
   // With a source table the loads of two passes go out together (of all four: half the waves,
-  // and slower); without one a pass's loads are few, and two passes' held 51 registers
-  // against 35: 8192 x 1024 23.7 against 26.9 us, 8192 x 4096 69.8 against 68.4.
+  // and slower). Without one a pass's loads are few and two passes' held 51 registers
+  // against 35: alone 4096 x 1024 10.8 against 12.5 us, 8192 x 4096 69.5 against 69.7.
   constexpr int AHEAD = SRC ? 2 : 1;
 #pragma unroll
   for (int first = 0; first < 4; first += AHEAD) {
@@ -347,19 +350,21 @@ __global__ __launch_bounds__(256) void k_lm_mask_bwd(LMMaskArgs a, const bf16_t*
     uint32_t ubs[4];
     float dts[4];
     uint4 tws[SRC ? 4 : 1];
-#pragma unroll
-    for (int pass = first; pass < first + AHEAD; ++pass) {
+    auto load = [&](int pass) {
       const int r = PD_LM_ROW(pass);
       const int64_t n = n0 + r;
-      if (n < a.N && qok) {
-        const int64_t idx = n * a.C + q0 + q4;
-        pws[pass] = *(const uint2*)(a.ci_pre + idx);
-        hws[pass] = *(const uint2*)(xV + idx);
-        dws[pass] = (!a.route || a.route[n]) ? *(const uint2*)(d_acts + idx) : make_uint2(0u, 0u);
-        dts[pass] = a.delta ? a.delta[n] : 0.f;
-        ubs[pass] = SRC ? 0u : *(const uint32_t*)(ubits + idx);
-        if constexpr (SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)SG.grp[r] * a.C + q0 + q4);
-      }
+      const int64_t idx = n * a.C + q0 + q4;
+      dts[pass] = a.delta ? a.delta[n] : 0.f;
+      pws[pass] = *(const uint2*)(a.ci_pre + idx);
+      hws[pass] = *(const uint2*)(xV + idx);
+      dws[pass] = (!a.route || a.route[n]) ? *(const uint2*)(d_acts + idx) : make_uint2(0u, 0u);
+      ubs[pass] = SRC ? 0u : *(const uint32_t*)(ubits + idx);
+      if constexpr (SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, (int64_t)SG.grp[r] * a.C + q0 + q4);
+    };
+    if constexpr (AHEAD > 1) {
+#pragma unroll
+      for (int pass = first; pass < first + AHEAD; ++pass)
+        if (n0 + PD_LM_ROW(pass) < a.N && qok) load(pass);
     }
 #pragma unroll
     for (int pass = first; pass < first + AHEAD; ++pass) {
@@ -368,6 +373,7 @@ __global__ __launch_bounds__(256) void k_lm_mask_bwd(LMMaskArgs a, const bf16_t*
       bf16_t o[4] = {0, 0, 0, 0};
       float dmsum = 0.f;
       if (n < a.N && qok) {
+        if constexpr (AHEAD == 1) load(pass);
         const int64_t idx = n * a.C + q0 + q4;
         const float dt = dts[pass];
         const uint2 pw = pws[pass], hw = hws[pass], dw = dws[pass];

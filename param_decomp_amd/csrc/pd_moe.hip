@@ -343,21 +343,23 @@ __global__ __launch_bounds__(256) void k_mask_fwd_tile(SiteMaskArgs a, const bf1
   __syncthreads();
   // With a source table the four passes' loads go out together: they are the time. A draw is
   // (draw_bits bounds the pass), and loads ahead of it only widen the wave: 27 registers
-  // against 49, 65536 x 512 77 against 83 us, 8192 x 512 14.8 against 15.6.
+  // against 49, alone 65536 x 512 78 against 83 us, 8192 x 512 15.8 against 16.6.
   constexpr int AHEAD = LAYOUT == MASK_SRC ? 4 : 1;
   float imp = 0.f;
 #pragma unroll
   for (int first = 0; first < 4; first += AHEAD) {
     uint2 pws[4], hws[4];
     uint4 tws[LAYOUT == MASK_SRC ? 4 : 1];
-#pragma unroll
-    for (int pass = first; pass < first + AHEAD; ++pass) {
+    auto load = [&](int pass) {
       const int r = PD_TILE4_ROW(pass);
-      if (j0 + r < a.J && qok) {
-        pws[pass] = *(const uint2*)(a.ci_pre + (int64_t)rows[r].slot * a.c + q0 + q4);
-        hws[pass] = *(const uint2*)(h + (j0 + r) * a.c + q0 + q4);
-        if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, rows[r].srow * a.c + q0 + q4);
-      }
+      pws[pass] = *(const uint2*)(a.ci_pre + (int64_t)rows[r].slot * a.c + q0 + q4);
+      hws[pass] = *(const uint2*)(h + (j0 + r) * a.c + q0 + q4);
+      if constexpr (LAYOUT == MASK_SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, rows[r].srow * a.c + q0 + q4);
+    };
+    if constexpr (AHEAD > 1) {
+#pragma unroll
+      for (int pass = first; pass < first + AHEAD; ++pass)
+        if (j0 + PD_TILE4_ROW(pass) < a.J && qok) load(pass);
     }
 #pragma unroll
     for (int pass = first; pass < first + AHEAD; ++pass) {
@@ -365,6 +367,7 @@ __global__ __launch_bounds__(256) void k_mask_fwd_tile(SiteMaskArgs a, const bf1
       const int64_t j = j0 + r;
       bf16_t o[4] = {0, 0, 0, 0};
       if (j < a.J && qok) {
+        if constexpr (AHEAD == 1) load(pass);
         const int64_t idx = j * a.c + q0 + q4;
         const MaskRow row = rows[r];
         const int64_t src = (int64_t)row.slot * a.c + q0 + q4;
@@ -438,16 +441,18 @@ __global__ __launch_bounds__(256) void k_mask_bwd_tile(SiteMaskArgs a, const bf1
   for (int first = 0; first < 4; first += AHEAD) {
     uint2 pws[4], hws[4], dws[4];
     uint4 tws[SRC ? 4 : 1];
-#pragma unroll
-    for (int pass = first; pass < first + AHEAD; ++pass) {
+    auto load = [&](int pass) {
       const int r = PD_TILE4_ROW(pass);
-      if (j0 + r < a.J && qok) {
-        const int64_t idx = (j0 + r) * a.c + q0 + q4;
-        pws[pass] = *(const uint2*)(a.ci_pre + (int64_t)rows[r].slot * a.c + q0 + q4);
-        hws[pass] = *(const uint2*)(h + idx);
-        dws[pass] = *(const uint2*)(d_acts + idx);
-        if constexpr (SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, rows[r].srow * a.c + q0 + q4);
-      }
+      const int64_t idx = (j0 + r) * a.c + q0 + q4;
+      pws[pass] = *(const uint2*)(a.ci_pre + (int64_t)rows[r].slot * a.c + q0 + q4);
+      hws[pass] = *(const uint2*)(h + idx);
+      dws[pass] = *(const uint2*)(d_acts + idx);
+      if constexpr (SRC) tws[pass] = src_quad_load(a.src, a.src_dtype, rows[r].srow * a.c + q0 + q4);
+    };
+    if constexpr (AHEAD > 1) {
+#pragma unroll
+      for (int pass = first; pass < first + AHEAD; ++pass)
+        if (j0 + PD_TILE4_ROW(pass) < a.J && qok) load(pass);
     }
 #pragma unroll
     for (int pass = first; pass < first + AHEAD; ++pass) {
@@ -456,6 +461,7 @@ __global__ __launch_bounds__(256) void k_mask_bwd_tile(SiteMaskArgs a, const bf1
       bf16_t o[4] = {0, 0, 0, 0};
       float dmsum = 0.f;
       if (j < a.J && qok) {
+        if constexpr (AHEAD == 1) load(pass);
         const int64_t idx = j * a.c + q0 + q4;
         const MaskRow row = rows[r];
         const int64_t src = (int64_t)row.slot * a.c + q0 + q4;
