@@ -25,9 +25,11 @@
 // the registers of the step before, after its MFMAs, so a wave alternates between waiting
 // for LDS and computing. Same products, same k order, so the same bits as the unpipelined
 // loop; 256x256 tiles 4096x3072x4096 with B MN-major 131 -> 104 us (785 -> 994 TFLOP/s),
-// both MN-major 137 -> 104 us, K-major 8192x4096x3072 210 -> 169 us. What bounds the loop
-// now is the LDS port: at 64x128 per wave a k16 step is 48 KB of fragment reads and 16 KB of
-// load writes per CU, 512 clocks at 128 B, as many as its MFMAs take.
+// both MN-major 137 -> 104 us, K-major 8192x4096x3072 210 -> 169 us. By the
+// counters (8192x4096x3072 in 256x256 tiles) the matrix cores are busy 0.78 of the clocks
+// in which a CU holds a block and the LDS reads 0.31, so the LDS port does not bound it;
+// the rest is the stage barrier and its waits, 0.14 of the launch without a block (first
+// loads, epilogue, last round), and a clock that falls to 1.8 GHz under this load.
 // The barrier is a bare s_barrier with compiler-only memory clobbers: a fenced
 // __syncthreads would wait for every load in flight.
 //
