@@ -598,24 +598,30 @@ __device__ inline void spread_step() {
 // issue(ahead, half): that half of the loads of the stage `ahead` stages
 // on (NS stages, AHEAD loads of the later ones left in flight); mfma(kk, f):
 // step kk's products. MFMAS, READS: a step's MFMAs and LDS reads; LOADS0, LOADS3: the loads issued in steps 0 and 3.
-template <int MFMAS, int READS, int LOADS0, int LOADS3, int NS, int AHEAD, class F, class Read, class ReadNext, class Issue, class Mfma>
+// LAST: the tile's last stage, after which nothing is loaded, read or waited for.
+template <int MFMAS, int READS, int LOADS0, int LOADS3, int NS, int AHEAD, bool LAST, class F, class Read, class ReadNext,
+          class Issue, class Mfma>
 __device__ inline void pipe_stage(F (&f)[2], Read&& read, ReadNext&& read_next, Issue&& issue, Mfma&& mfma) {
   read(1, f[1]);
-  issue(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+  if constexpr (!LAST) issue(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
   mfma(0, f[0]);
-  spread_step<MFMAS, READS, LOADS0>();
+  spread_step<MFMAS, READS, LAST ? 0 : LOADS0>();
   read(2, f[0]);
   mfma(1, f[1]);
   spread_step<MFMAS, READS, 0>();
   read(3, f[1]);
   mfma(2, f[0]);
   spread_step<MFMAS, READS, 0>();
-  wait_loads_and_lds<AHEAD>();
-  lds_barrier();
-  read_next(f[0]);
-  issue(std::integral_constant<int, NS>{}, std::integral_constant<int, 0>{});
-  mfma(3, f[1]);
-  spread_step<MFMAS, READS, LOADS3>();
+  if constexpr (LAST) {
+    mfma(3, f[1]);
+  } else {
+    wait_loads_and_lds<AHEAD>();
+    lds_barrier();
+    read_next(f[0]);
+    issue(std::integral_constant<int, NS>{}, std::integral_constant<int, 0>{});
+    mfma(3, f[1]);
+    spread_step<MFMAS, READS, LOADS3>();
+  }
 }
 
 template <class CFG, typename TC>
@@ -822,10 +828,10 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
   lds_barrier();
   read_frags<CFG>(smem, fo, lane, 0, f[0]);
   constexpr int READS = TM * (AMN ? 2 : 1) + TN * (BMN ? 2 : 1);
-  auto stage = [&](int64_t kt, auto edge) {
+  auto stage = [&](int64_t kt, auto edge, auto last) {
     const char* st = smem + CFG::ring(kt) * CFG::STAGE_BYTES;
     const char* nx = smem + CFG::ring(kt + 1) * CFG::STAGE_BYTES;
-    pipe_stage<TM * TN, READS, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD>(
+    pipe_stage<TM * TN, READS, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD, decltype(last)::value>(
         f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
         [&](Frags<CFG>& g) { read_frags<CFG>(nx, fo, lane, 0, g); },
         [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
@@ -834,13 +840,9 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl(GemmArgs p, typename EPI::
           dtl_mfma<CFG>(g.a, g.b, acc);
         });
   };
-  if constexpr (KEDGE) {
-    if (nk > 0) stage(0, std::true_type{});
-    for (int64_t kt = 1; kt < nk - 1; ++kt) stage(kt, std::false_type{});
-    if (nk > 1) stage(nk - 1, std::true_type{});
-  } else {
-    for (int64_t kt = 0; kt < nk; ++kt) stage(kt, std::false_type{});
-  }
+  if (KEDGE && nk > 1) stage(0, std::true_type{}, std::false_type{});
+  for (int64_t kt = KEDGE; kt < nk - 1; ++kt) stage(kt, std::false_type{}, std::false_type{});
+  if (nk > 0) stage(nk - 1, std::integral_constant<bool, KEDGE>{}, std::true_type{});
   wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG, TC>(p, ea, t, wm, wn, tid, acc, smem);
 }
@@ -912,10 +914,10 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
     wait_vmcnt<LOADS>();
     lds_barrier();
     read(smem, 0, f[0]);
-    auto stage = [&](int64_t kt, auto edge) {
+    auto stage = [&](int64_t kt, auto edge, auto last) {
       const char* st = smem + (int)(kt & 1) * SB;
       const char* nx = smem + (int)(~kt & 1) * SB;
-      pipe_stage<2 * TM * TN, 2 * TM + TN, 0, LOADS, 2, 0>(
+      pipe_stage<2 * TM * TN, 2 * TM + TN, 0, LOADS, 2, 0, decltype(last)::value>(
           f, [&](int kk, F2& g) { read(st, kk, g); }, [&](F2& g) { read(nx, 0, g); },
           [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
           [&](int kk, F2& g) {
@@ -929,8 +931,8 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
             dtl_mfma<CFG>(g.a2, g.x.b, acc2);
           });
     };
-    for (int64_t kt = 0; kt < nk - KEDGE; ++kt) stage(kt, std::false_type{});
-    if constexpr (KEDGE) stage(nk - 1, std::true_type{});
+    for (int64_t kt = 0; kt < nk - 1; ++kt) stage(kt, std::false_type{}, std::false_type{});
+    stage(nk - 1, std::integral_constant<bool, KEDGE>{}, std::true_type{});
   } else {
     auto issue = [&](int64_t kt, auto h) {  // stages nk .. 2 nk - 1 are the second product's
       if (decltype(h)::value) return;
@@ -947,10 +949,10 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
     wait_vmcnt<CFG::AHEAD + CFG::INSTS>();
     lds_barrier();
     read_frags<CFG>(smem, fo, lane, 0, f[0]);
-    auto stage = [&](int64_t kt, int64_t k0, auto edge, f32x16 (&ac)[TM][TN]) {
+    auto stage = [&](int64_t kt, int64_t k0, auto edge, auto last, f32x16 (&ac)[TM][TN]) {
       const char* st = smem + CFG::ring(kt) * SB;
       const char* nx = smem + CFG::ring(kt + 1) * SB;
-      pipe_stage<TM * TN, TM + TN, 0, CFG::INSTS, NS, CFG::AHEAD>(
+      pipe_stage<TM * TN, TM + TN, 0, CFG::INSTS, NS, CFG::AHEAD, decltype(last)::value>(
           f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
           [&](Frags<CFG>& g) { read_frags<CFG>(nx, fo, lane, 0, g); },
           [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
@@ -959,10 +961,11 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_dual(GemmArgs p, typename 
             dtl_mfma<CFG>(g.a, g.b, ac);
           });
     };
-    for (int64_t kt = 0; kt < nk - KEDGE; ++kt) stage(kt, 0, std::false_type{}, acc);
-    if constexpr (KEDGE) stage(nk - 1, (nk - 1) * BK, std::true_type{}, acc);
-    for (int64_t kt = nk; kt < 2 * nk - KEDGE; ++kt) stage(kt, 0, std::false_type{}, acc2);
-    if constexpr (KEDGE) stage(2 * nk - 1, (nk - 1) * BK, std::true_type{}, acc2);
+    const std::false_type no{};
+    for (int64_t kt = 0; kt < nk - KEDGE; ++kt) stage(kt, 0, no, no, acc);
+    if constexpr (KEDGE) stage(nk - 1, (nk - 1) * BK, std::true_type{}, no, acc);
+    for (int64_t kt = nk; kt < 2 * nk - 1; ++kt) stage(kt, 0, no, no, acc2);
+    stage(2 * nk - 1, (nk - 1) * BK, std::integral_constant<bool, KEDGE>{}, std::true_type{}, acc2);
   }
   wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG>(p, ea, t, wm, wn, tid, acc, acc2, smem);
@@ -1074,10 +1077,12 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
   read_frags<CFG>(smem, fo1, lane, 0, f[0]);
   // stage kt of a segment whose fragments sit at fo, the next stage's at fon; its k range
   // starts at k0 and ends at kend
-  auto stage = [&](int64_t kt, const auto& fo, const auto& fon, int64_t k0, int64_t kend, auto edge, auto reads) {
+  auto stage = [&](int64_t kt, const auto& fo, const auto& fon, int64_t k0, int64_t kend, auto edge, auto reads,
+                   auto last) {
     const char* st = smem + CFG::ring(kt) * CFG::STAGE_BYTES;
     const char* nx = smem + CFG::ring(kt + 1) * CFG::STAGE_BYTES;
-    pipe_stage<TM * TN, decltype(reads)::value, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD>(
+    pipe_stage<TM * TN, decltype(reads)::value, CFG::INSTS - CFG::HALF, CFG::HALF, CFG::NS, CFG::AHEAD,
+               decltype(last)::value>(
         f, [&](int kk, Frags<CFG>& g) { read_frags<CFG>(st, fo, lane, kk, g); },
         [&](Frags<CFG>& g) { read_frags<CFG>(nx, fon, lane, 0, g); },
         [&](auto ahead, auto h) { issue(kt + decltype(ahead)::value, h); },
@@ -1090,8 +1095,9 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
   constexpr std::integral_constant<int, TM + TN * (B2MN ? 2 : 1)> r2{};
   // segment 1; its last stage reads segment 2's first fragments (KEDGE: and masks its k tail)
   constexpr bool LAST1 = KEDGE || B1MN != B2MN;
-  for (int64_t kt = 0; kt < nk1 - LAST1; ++kt) stage(kt, fo1, fo1, kt * BK, K1, std::false_type{}, r1);
-  if constexpr (LAST1) stage(nk1 - 1, fo1, fo2, (nk1 - 1) * BK, K1, std::integral_constant<bool, KEDGE>{}, r1);
+  const std::false_type no{};
+  for (int64_t kt = 0; kt < nk1 - LAST1; ++kt) stage(kt, fo1, fo1, kt * BK, K1, no, r1, no);
+  if constexpr (LAST1) stage(nk1 - 1, fo1, fo2, (nk1 - 1) * BK, K1, std::integral_constant<bool, KEDGE>{}, r1, no);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int64_t row = m0 + wm * CFG::WTM + i * 32 + (lane & 31);
@@ -1105,8 +1111,8 @@ __global__ __launch_bounds__(CFG::NT) void k_gemm_dtl_kcat(GemmArgs p, KcatArgs 
       for (int v = 0; v < 16; ++v) acc[i][j][v] *= rs;
   }
   // segment 2
-  for (int64_t kt = nk1; kt < nk - KEDGE; ++kt) stage(kt, fo2, fo2, (kt - nk1) * BK, K2, std::false_type{}, r2);
-  if constexpr (KEDGE) stage(nk - 1, fo2, fo2, (nk - 1 - nk1) * BK, K2, std::true_type{}, r2);
+  for (int64_t kt = nk1; kt < nk - 1; ++kt) stage(kt, fo2, fo2, (kt - nk1) * BK, K2, no, r2, no);
+  stage(nk - 1, fo2, fo2, (nk - 1 - nk1) * BK, K2, std::integral_constant<bool, KEDGE>{}, r2, std::true_type{});
   wait_vmcnt<0>();  // the empty loads past the last stage still write their zeros
   EPI::template run<CFG, TC>(p, ea, t, wm, wn, tid, acc, smem);
 }
