@@ -320,33 +320,33 @@ def pmc_l2_summary(csv_path: str, command: str, n_xcd: int = 8, n_ch: int = 16) 
 # launch is the dispatch-weighted mean over its kernels in the committed PMC summary.
 PHASE_KERNEL = {
     # (the GEMM kernels of a phase also run in other phases: the clean pass, the backward)
-    MOE: {"gemm_dw": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 4, 2, 2, false>, float, 2,",
-                      "pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, float, 2,"),
-          "gemm_fwd": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 4, 2, 2, false>, unsigned short, 1, false, pd::EpiStore",
-                       "pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, unsigned short, 1, false, pd::EpiStore",
+    MOE: {"gemm_dw": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, float, 2,",
+                      "pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, false, 2>, float, 2,"),
+          "gemm_fwd": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, unsigned short, 1, false, pd::EpiStore",
+                       "pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, false, 2>, unsigned short, 1, false, pd::EpiStore",
                        "pd::k_gemm_dtl_kcat<"),
           "gemm_dx": ("pd::k_gemm_dtl_kcat<",),
-          "gemm_dx_mask": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 4, 2, 2, false>, unsigned short, 1, false, "
+          "gemm_dx_mask": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, unsigned short, 1, false, "
                            "pd::EpiMaskBwd",
-                           "pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, unsigned short, 1, false, "
+                           "pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, false, 2>, unsigned short, 1, false, "
                            "pd::EpiMaskBwd"),
           "mask_fwd": ("pd::k_mask_fwd_tile",), "mask_bwd": ("pd::k_mask_bwd_tile", "pd::k_mask_bwd_vec")},
     # dense GEMM phases by template and grid (work-items: tiles x 512 threads at T 4096,
-    # 768 -> 3072, C 4096; the 4096 x 4096 products run on 256x256 tiles)
+    # 768 -> 3072, C 4096; all but dV on 256x256 tiles)
     DENSE: {"gate_mask_fwd": ("pd::k_step_fwd_tab", "pd::k_gate_range", "pd::k_gate_table"),
             "gate_mask_bwd": ("pd::k_step_bwd",), "gate_grad_reduce": ("pd::k_gate_finalize",),
             "recon": ("pd::k_step_recon",),
-            "gemm_target": ("pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, unsigned short, 0, false, "
-                            "pd::EpiStore, false, false> @393216",),
-            "gemm_xV": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 4, 2, 2, false>, unsigned short, 0, false, "
+            "gemm_target": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, unsigned short, 0, false, "
+                            "pd::EpiStore, false, false> @98304",),
+            "gemm_xV": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, unsigned short, 0, false, "
                         "pd::EpiStore, false, true> @131072",),
-            "gemm_actsU": ("pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, unsigned short, 0, false, "
-                           "pd::EpiStore, false, true> @393216",),
-            "gemm_dU": ("pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, float, 0, false, "
-                        "pd::EpiStore, true, true> @393216",),
-            "gemm_da": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 4, 2, 2, false>, unsigned short, 0, false, "
+            "gemm_actsU": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, unsigned short, 0, false, "
+                           "pd::EpiStore, false, true> @98304",),
+            "gemm_dU": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, float, 0, false, "
+                        "pd::EpiStore, true, true> @98304",),
+            "gemm_da": ("pd::k_gemm_dtl<pd::DtlCfg<256, 256, 2, 4, true, 2>, unsigned short, 0, false, "
                         "pd::EpiStore, false, false> @131072",),
-            "gemm_dV": ("pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, 2, true>, float, 0, false, "
+            "gemm_dV": ("pd::k_gemm_dtl<pd::DtlCfg<128, 128, 4, 2, false, 2>, float, 0, false, "
                         "pd::EpiStore, true, true> @98304",)},
 }
 

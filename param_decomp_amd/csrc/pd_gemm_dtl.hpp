@@ -20,7 +20,9 @@
 // the next stage have landed (vmcnt) and its reads of this stage are done (lgkmcnt), so
 // behind the barrier the next stage is visible and this one's space is free. The loads of
 // stage kt+NS go out between the MFMAs of stage kt's last step; with SPLIT (256x256 tiles,
-// two stages) half of them between those of stage kt+1's first step. The order is
+// two stages) half of them between those of stage kt+1's first step. A tile's last stage
+// loads, reads and waits for nothing (run like the others, on empty descriptors, it cost
+// contractions of one to six stages 5-8%). The order is
 // pinned by scheduling barriers: left to itself the compiler reads a step's fragments into
 // the registers of the step before, after its MFMAs, so a wave alternates between waiting
 // for LDS and computing. Same products, same k order, so the same bits as the unpipelined
