@@ -697,8 +697,10 @@ static int launch_dtl_any(const GemmArgs& a, bool a_kmaj, bool b_kmaj, int c_dty
   {                                                                                                 \
     if constexpr (BIG_OK)                                                                           \
       if (big) return launch_dtl<CfgDtlBig, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);            \
-    if constexpr (MODE == MODE_DENSE && !(AMN) && !(BMN))                                           \
+    if constexpr (MODE == MODE_DENSE && !(AMN) && !(BMN)) {                                         \
       if (deep_ring(a.M, a.N, a.K)) return launch_dtl<CfgDtlDeep, MODE>(a, c_dtype, kedge, grid, s); \
+      if (!dense_fills(a.M, a.N)) return launch_dtl<CfgDtl, MODE>(a, c_dtype, kedge, grid, s);      \
+    }                                                                                               \
     return launch_dtl<CfgDtlSmall<MODE, AMN, BMN>, MODE, AMN, BMN>(a, c_dtype, kedge, grid, s);     \
   }
   if (a_kmaj && b_kmaj) PD_L(false, false)

@@ -355,9 +355,13 @@ inline bool deep_ring(int64_t M, int64_t N, int64_t K) {
 typedef DtlCfg<256, 256, 2, 4, true> CfgDtlBig;
 // The small tile of a launch: 4 waves where both operands are K-major and one product fills
 // the grid, 8 elsewhere (batches and ragged groups of few rows: 53 x 712x64x208 9.0 against
-// 9.9 us, 8 groups of 53 rows over 248 6.6 against 7.2).
+// 9.9 us, 8 groups of 53 rows over 248 6.6 against 7.2). A dense product fills it from 7/8
+// of a round of two blocks per CU on: below, CUs hold one block, 4 or 8 waves of it. 4 against
+// 8 waves, us: 259 tiles (4688x808x2032) 32.1 / 30.0, 384 (8192x768x7168) 101.9 / 99.7, 496
+// (7912x968x1464) 32.9 / 34.0, 512 (8192x1024x3072) 52.7 / 53.4.
 template <int MODE, bool AMN, bool BMN>
 using CfgDtlSmall = std::conditional_t<AMN || BMN || MODE == MODE_BATCHED, CfgDtl, CfgDtlRA>;
+inline bool dense_fills(int64_t M, int64_t N) { return ((M + 127) / 128) * ((N + 127) / 128) >= 448; }
 
 // Whether an output takes `big` 256x256 tiles (one block per CU) rather than `small` 128x128
 // ones (two per CU): by the rounds of 256 big or 512 small tiles, a partial round costing
