@@ -740,7 +740,7 @@ int pd_gemm(int dtype, int64_t M, int64_t N, int64_t K, const void* A, int64_t l
     return fail(PD_EUNSUPPORTED, "pd_gemm: bf16 operands need 16B alignment and contiguous dims / ld % 8 == 0");
   GemmArgs a{M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, C, ldc, alpha, beta, nullptr, 0, 0, 0};
   if (dtl_fits_any(M, N, K, lda, a_kmaj, ldb, b_kmaj))
-    return launch_dtl_any<MODE_DENSE, true>(a, a_kmaj, b_kmaj, c_dtype, K % 64 != 0, big_tiles(M, N), 1, s);
+    return launch_dtl_any<MODE_DENSE, true>(a, a_kmaj, b_kmaj, c_dtype, K % 64 != 0, big_tiles(M, N, K), 1, s);
   if (use_big_tile(M, N))
     return launch_bf16<CfgBig, MODE_DENSE>(a, a_kmaj, b_kmaj, c_dtype,
                                            dim3((unsigned)cdiv(N, 256), (unsigned)cdiv(M, 256)), s);

@@ -365,22 +365,30 @@ inline bool dense_fills(int64_t M, int64_t N) { return ((M + 127) / 128) * ((N +
 
 // Whether an output takes `big` 256x256 tiles (one block per CU) rather than `small` 128x128
 // ones (two per CU): by the rounds of 256 big or 512 small tiles, a partial round costing
-// 0.8 + 0.2 of its fill and a round of small tiles 0.64 of a round of big ones (half the
-// products at 0.8 of the rate). Big against small, us: 192 big tiles (4096x3072x4096) 101 /
-// 117, 384 (8192x3072x4864) 238 / 248, 512 (65536x512x512) 46 / 60, 256 (65536x256x512) 28 /
-// 31; 128 (8192x1024x768) 21.7 / 17.6, 48 (768x4096x4096) 91 / 51.
-inline bool big_rounds(int64_t big, int64_t small) {
+// 0.8 + 0.2 of its fill. A round of small tiles is half the products of a round of big ones
+// and costs `small_round` of it. Big against small, us: 192 big tiles
+// (4096x3072x4096) 101 / 117, 384 (8192x3072x4864) 238 / 248, 512 (65536x512x512) 46 / 60,
+// 256 (65536x256x512) 28 / 31; 128 (8192x1024x768) 21.7 / 17.6, 48 (768x4096x4096) 91 / 51.
+inline bool big_rounds(int64_t big, int64_t small, double small_round) {
   auto rounds = [](int64_t tiles, int64_t cap) {  // in fifths
     const int64_t full = tiles / cap, rem = tiles % cap;
     return 5.0 * full + (rem ? 4.0 + (double)rem / cap : 0.0);
   };
-  return rounds(big, 256) <= 0.64 * rounds(small, 512);
+  return rounds(big, 256) <= small_round * rounds(small, 512);
 }
 inline int64_t tiles_up(int64_t x, int64_t n) { return (x + n - 1) / n; }
-inline bool big_tiles(int64_t rows, int64_t N) {
-  return big_rounds(tiles_up(rows, 256) * tiles_up(N, 256), tiles_up(rows, 128) * tiles_up(N, 128));
+// One product: 0.66 over a long contraction, 0.58 up to K = 1024, where a lone block's ramp
+// (first loads, epilogue) has nothing beside it. Over 370 drawn products 1.5% slower than the
+// better tile each time with 0.64 throughout, 0.6% with these.
+inline bool big_tiles(int64_t rows, int64_t N, int64_t K) {
+  return big_rounds(tiles_up(rows, 256) * tiles_up(N, 256), tiles_up(rows, 128) * tiles_up(N, 128),
+                    K <= 1024 ? 0.58 : 0.66);
 }
-// The same for J rows in E groups whose sizes only the device knows: the rows' tiles plus
+// Two-segment and grouped products run beside another stream's in the steps, where the small
+// tile's waves cost more than alone: 65536x512x256 in 42 groups takes 39.6 against 41.5 us
+// alone, yet the MoE step's forward products 1.65 against 1.59 ms.
+constexpr double SHARED_ROUND = 0.64;
+// J rows in E groups whose sizes only the device knows: the rows' tiles plus
 // half a tile per group for the ragged ends, and at least one per group (of any size: small
 // groups are what a big tile wastes most on). Big against small, us: 1352 rows in 128 groups
 // over 440 (N = 528) 34 / 23, 560 in 128 over 96 (N = 1528) 29 / 21, 50664 in 32 over 144 (N =
@@ -391,7 +399,7 @@ inline bool big_tiles_grouped(int64_t J, int64_t E, int64_t N, int64_t problems 
     const int64_t rows = tiles_up(J + groups * (t / 2), t);
     return problems * (rows > groups ? rows : groups) * tiles_up(N, t);
   };
-  return big_rounds(tiles(256), tiles(128));
+  return big_rounds(tiles(256), tiles(128), SHARED_ROUND);
 }
 
 // The kernel addresses each operand through a 31-bit buffer record count (rows = M or N
@@ -1141,7 +1149,7 @@ inline int launch_dense_epi(const GemmArgs& a, const typename EPI::Args& ea, hip
     return fail(PD_EUNSUPPORTED, std::string(what) + ": operands of 2 GiB or more");
   if ((a.M + CfgDtl::BM - 1) / CfgDtl::BM > 65535 || (a.N + CfgDtl::BN - 1) / CfgDtl::BN > 65535)
     return fail(PD_EUNSUPPORTED, std::string(what) + ": too large");
-  if (EPI::BIG_OK && big_tiles(a.M, a.N)) launch_epi_cfg<CfgDtlBig, EPI, TC, BMN>(a, ea, s);
+  if (EPI::BIG_OK && big_tiles(a.M, a.N, a.K)) launch_epi_cfg<CfgDtlBig, EPI, TC, BMN>(a, ea, s);
   else if (!BMN && deep_ring(a.M, a.N, a.K)) launch_epi_cfg<CfgDtlDeep, EPI, TC, BMN>(a, ea, s);
   else launch_epi_cfg<CfgDtl, EPI, TC, BMN>(a, ea, s);
   return check_launch(what);
@@ -1166,7 +1174,8 @@ inline int launch_kcat_epi(const GemmArgs& a, const KcatArgs& q, const typename 
     return fail(PD_EUNSUPPORTED, std::string(what) + ": operands of 2 GiB or more");
   if ((a.M + CfgDtlRA::BM - 1) / CfgDtlRA::BM > 65535 || (a.N + CfgDtlRA::BN - 1) / CfgDtlRA::BN > 65535)
     return fail(PD_EUNSUPPORTED, std::string(what) + ": too large");
-  if (big_tiles(a.M, a.N) && EPI::LDS_BYTES <= 2 * CfgDtlBig::STAGE_BYTES)
+  if (big_rounds(tiles_up(a.M, 256) * tiles_up(a.N, 256), tiles_up(a.M, 128) * tiles_up(a.N, 128), SHARED_ROUND) &&
+      EPI::LDS_BYTES <= 2 * CfgDtlBig::STAGE_BYTES)
     launch_kcat_cfg<CfgDtlBig, EPI, TC, B1MN, B2MN>(a, q, ea, s);
   else if (!B1MN && !B2MN && deep_ring(a.M, a.N, a.K + q.K1))
     launch_kcat_cfg<CfgDtlDeep, EPI, TC, B1MN, B2MN>(a, q, ea, s);

@@ -17,7 +17,7 @@ int main(int n, char** v) {
   long a[4] = {0, 0, 0, 1};
   for (int i = 2; i < n; ++i) a[i - 2] = atol(v[i]);
   const char* r = "small";
-  if (v[1][0] == 'd') r = pd::big_tiles(a[0], a[1]) ? "big" : pd::deep_ring(a[0], a[1], a[2]) ? "deep"
+  if (v[1][0] == 'd') r = pd::big_tiles(a[0], a[1], a[2]) ? "big" : pd::deep_ring(a[0], a[1], a[2]) ? "deep"
                                                      : pd::dense_fills(a[0], a[1]) ? "small" : "small, 8 waves";
   else if (pd::big_tiles_grouped(a[0], a[1], a[2], a[3])) r = "big";
   puts(r);
@@ -48,8 +48,8 @@ def test_grouped_tiles(rule, J, E, N, problems, tile):
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
-    (4096, 3072, 4096, "big"), (8192, 1024, 768, "small"), (768, 4096, 4096, "deep"), (3001, 768, 4096, "deep"),
-    (3000, 4104, 320, "big"), (4000, 3072, 200, "big"), (2048, 2048, 768, "deep"), (2048, 2048, 760, "small, 8 waves"),
+    (4096, 3072, 4096, "big"), (8192, 1024, 768, "small"), (768, 4096, 4096, "deep"), (8192, 3072, 4864, "big"), (3001, 768, 4096, "deep"),
+    (3000, 4104, 8, "big"), (3000, 4104, 320, "big"), (4000, 3072, 200, "big"), (2048, 2048, 768, "deep"), (2048, 2048, 760, "small, 8 waves"),
     (8192, 768, 7168, "small, 8 waves"), (8192, 1024, 3072, "small"), (7912, 968, 1464, "small"),
     (4096, 3072, 768, "big"), (4096, 4096, 776, "big"), (4000, 4104, 200, "small"),
     # the CI MLP's: hidden layer, head and pullback; the pullback and the input gradient
