@@ -4,6 +4,7 @@ These passes are bound by the random draw and run beside another stream's produc
 registers or fewer, eight of their waves leave a quarter of a SIMD's 512 to those products
 (loads issued ahead of the draw cost 49 to 67 and made every pass slower)."""
 
+import os
 import re
 import struct
 
@@ -41,6 +42,8 @@ def _kernels():
 @pytest.mark.parametrize("pattern", [r"k_mask_fwd_tileILi[01]ELi\dE", r"k_lm_mask_fwdILi[01]ELi\dE",
                                      r"k_lm_mask_bwdILi\dELb0E"])
 def test_drawn_mask_passes(pattern):
+    if not os.path.exists(builder.LIB):
+        pytest.skip("HIP library not built")
     found = {n: v for n, v in _kernels().items() if re.search(pattern, n)}
     assert len(found) in (4, 8)
     assert all(v <= 48 for v in found.values()), found
